@@ -28,7 +28,7 @@ constexpr size_t NA_OFF_CFL = 0;                 // 1 value, padded to 256 bytes
 constexpr size_t NA_OFF_PART_CFL = 32;
 constexpr size_t NA_OFF_HIST = NA_OFF_PART_CFL + NA_CFL_BLOCKS;
 constexpr size_t NA_OFF_TILES = NA_OFF_HIST + NA_HIST * NGLB;
-constexpr size_t NA_DOUBLES = NA_OFF_TILES + NA_TILES * NGLB;   // 831,520 doubles = 6.65 MB
+constexpr size_t NA_DOUBLES = NA_OFF_TILES + NA_TILES * NPART;  // 1,552,416 doubles = 12.4 MB
 static __device__ __align__(256) double scratch[NA_DOUBLES];
 
 namespace {
@@ -672,7 +672,7 @@ void drop_graphs(cmf_hip_ctx* h) {
 
 template <class R>
 int grow_partials(cmf_hip_ctx* h, DevState<R>& S, int nrun) {
-    const size_t need = (size_t)nrun * tiles_cells(h->M, upd_bs(h)) * NGLB;
+    const size_t need = (size_t)nrun * tiles_cells(h->M, upd_bs(h)) * NPART;
     if (need > h->partial_cap) {
         // k_update of a cached graph writes into S.partials: the old buffer is freed here
         drop_graphs(h);

@@ -50,48 +50,16 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double* lds /* [NV][B
     __syncthreads();
 }
 
-// Compensated block sum (TwoSum, Knuth): every partial sum is carried as hi + lo
-// with lo the exact rounding error of each addition, so the result is the
-// correctly rounded sum of the NV inputs up to O(2^-106) relative terms, whatever
-// the number of cells. Needs IEEE additions without contraction (the files are
-// compiled with -ffp-contract=off). Result in lds[k * NW] as hi + lo, rounded.
-__device__ __forceinline__ void two_sum(double a, double b, double& s, double& e) {
-    s = a + b;
-    const double bb = s - a;
-    e = (a - (s - bb)) + (b - bb);
-}
-template <int BS, int NV>
-__device__ __forceinline__ void block_sum_comp(double (&v)[NV], double* lds /* [2][NV][BS/64] */) {
+// Compensated block sum of the budget terms (low parts vl, or NULL): term k in h, l
+// of thread k < NGLB
+template <int BS>
+__device__ __forceinline__ void block_sum_comp(const double* v, const double* vl, double* lds /* [2][NGLB][BS/64] */,
+                                               double& h, double& l) {
     constexpr int NW = BS / 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    double lo[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) lo[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const double oh = __shfl_down(v[k], off, 64), ol = __shfl_down(lo[k], off, 64);
-            double sh, e;
-            two_sum(v[k], oh, sh, e);
-            v[k] = sh;
-            lo[k] = (lo[k] + ol) + e;
-        }
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) { lds[k * NW + wave] = v[k]; lds[(NV + k) * NW + wave] = lo[k]; }
+    wave_sum_comp<NGLB>(v, lds, lds + NGLB * NW, NW, threadIdx.x >> 6, 0, vl);
     __syncthreads();
-    if (threadIdx.x < NV) {
-        double hi = 0.0, l = 0.0;
-        for (int w = 0; w < NW; ++w) {
-            double sh, e;
-            two_sum(hi, lds[threadIdx.x * NW + w], sh, e);
-            hi = sh;
-            l = (l + lds[(NV + threadIdx.x) * NW + w]) + e;
-        }
-        lds[threadIdx.x * NW] = hi + l;
-    }
-    __syncthreads();
+    h = 0.0; l = 0.0;
+    if (threadIdx.x < NGLB) comp_total(lds, lds + NGLB * NW, NW, threadIdx.x, h, l);
 }
 
 // Tile t of a launch of G blocks: with xcd set and G a multiple of 8, the blocks
@@ -230,30 +198,6 @@ __device__ __forceinline__ void kinemix_outflow(const DevMap& M, const DevState<
 // scheme and the launch picks the one StepArgs::lkine asks for, so the default
 // (local inertial) kernel is compiled as if the option did not exist; the
 // persistent k_substep carries both and branches once per tile.
-// Hanazaki-2022 reservoir operation (LDAMH22), src/cmf_ctrl_damout_mod.F90:354-378,
-// before the storage limiter. Zones: normal (<= NorVol), water supply (<= ConVol),
-// flood control (< EmeVol), emergency. r_volupa is the dam's own flood-control
-// volume over its upstream area (damout:204 stores every dam's ratio at index NDAM;
-// here each dam reads its own). Default-real constants 1. and 0.2 widened.
-__device__ __forceinline__ double dam_rule_h22(double vol, double inflow, double norvol, double convol,
-                                               double emevol, double qn, double qf, double r_volupa) {
-    if (vol <= norvol) return qn * (vol / convol);
-    const double quad = (vol - norvol) / (emevol - norvol);        // ((V-NorVol)/(EmeVol-NorVol))**2
-    const double pre = qn * 0.5 + (quad * quad) * (qf - qn);
-    if (vol <= convol) {
-        if (qf <= inflow) return qn * 0.5 + ((vol - norvol) / (convol - norvol)) * (qf - qn);
-        return pre;
-    }
-    if (vol < emevol) {
-        if (qf <= inflow) {
-            const double cut = vmax(1.0 - r_volupa / K_0P2F, 0.0);
-            return qf + ((cut * (vol - convol)) / (emevol - convol)) * (inflow - qf);
-        }
-        return pre;
-    }
-    return vmax(inflow, qf);
-}
-
 template <class R, bool MB, bool KINE>
 __device__ __forceinline__ void outflow_cell(const DevMap& M, const DevState<R>& S, const StepArgs& A, int s) {
     const Slot x = cell_slot<MB>(M, s);
@@ -281,10 +225,7 @@ __device__ __forceinline__ void outflow_cell(const DevMap& M, const DevState<R>&
         fldout_pre = S.fldout[s];                                   // D2FLDOUT_PRE
     }
     if (!I.active) return;
-    const R gdt = R(I.gdt);
-    const R zero = R(0), one = R(1);
-    const R flddph_pre = vmax(rivdph_pre - R(f_rivhgt), zero);
-    const R rivwth = R(f_rivwth), rivman = R(f_rivman);
+    const R zero = R(0);
     const bool river = nxt >= 0;                                     // mouths carry a negative code
     R q_r, q_f = zero, vel;
     if constexpr (KINE) {
@@ -294,129 +235,29 @@ __device__ __forceinline__ void outflow_cell(const DevMap& M, const DevState<R>&
         if (A.lslpmix && M.i2mask[i] == 0) kinemix_outflow<R, MB>(M, S, A, i, nxt, s, m, I.dt, q_r, q_f, vel);
         else kine_outflow<R>(M, S, A, i, nxt, s, I.dt, q_r, q_f, vel);
     } else {
-        // Water-surface terms of outflw:45-58. With R = double they are evaluated as
-        // the reference writes them (SFCELV = RIVELV + RIVDPH, slopes and depths from
-        // SFCELV). With R = float the same quantities are formed from depths and the
-        // exact FP64 elevation difference, rounded once: a ~250 m surface elevation
-        // keeps only ~1.5e-5 m in FP32, which the slope (a difference of a few cm)
-        // would otherwise inherit.
-        //   hs  = SFCELV - DWNELV          (slope numerator)
-        //   hr  = max(SFCELV, DWNELV) - RIVELV,  hrp the same with the _PRE values
-        //   (mouths: hr = RIVDPH, hrp = RIVDPH_PRE)
-        //   fa  = surface above ELEVTN for the floodplain (outflw:88, :147), fap the _PRE one
-        R hs, hr, hrp, fa, fap, rdst;
-        if (sizeof(R) == sizeof(double)) {
-            const R rivelv = R((double)f_elevtn - (double)f_rivhgt);    // maps:722
-            const R elevtn = R(f_elevtn);
-            const R sfcelv = rivelv + rivdph;                           // outflw:45-47
-            const R sfcelv_pre = rivelv + rivdph_pre;
-            if (river) {                                                 // outflw:52-57
-                const int j = nxt, sj = sidx<MB>(M, j, m);
-                const R rivelv_j = R(rivelv_of(M, j));
-                const R dwn = rivelv_j + S.rivdph[sj];
-                const R dwn_pre = rivelv_j + S.rivdph_pre[sj];
-                const R dsfc = vmax(sfcelv, dwn), dsfc_pr = vmax(sfcelv_pre, dwn_pre);
-                hs = sfcelv - dwn;
-                hr = dsfc - rivelv;
-                hrp = dsfc_pr - rivelv;
-                fa = dsfc - elevtn;
-                fap = dsfc_pr - elevtn;
-                rdst = one / R(f_nxtdst);
-            } else {
-                const R dwn = R(M.dwnelv[i]);
-                hs = sfcelv - dwn;
-                hr = rivdph;
-                hrp = rivdph_pre;
-                fa = sfcelv - elevtn;
-                fap = sfcelv_pre - elevtn;
-                rdst = one / R(A.pdstmth);
-            }
-        } else {
-            const double e_i = (double)f_elevtn - (double)f_rivhgt;
-            if (river) {
-                const int j = nxt, sj = sidx<MB>(M, j, m);
-                const R dz = R(rivelv_of(M, j) - e_i);                   // RIVELV(j) - RIVELV(i)
-                const R dj = S.rivdph[sj], dj_pre = S.rivdph_pre[sj];
-                hs = (rivdph - dj) - dz;
-                hr = vmax(rivdph, dz + dj);
-                hrp = vmax(rivdph_pre, dz + dj_pre);
-                rdst = one / R(f_nxtdst);
-            } else {
-                hs = rivdph - R(M.dwnelv[i] - e_i);
-                hr = rivdph;
-                hrp = rivdph_pre;
-                rdst = one / R(A.pdstmth);
-            }
-            const R hgt = R(f_rivhgt);                                   // ELEVTN = RIVELV + RIVHGT
-            fa = hr - hgt;
-            fap = hrp - hgt;
-        }
-        // ---- river channel: outflw:60-80 (river), :119-139 (mouth)
-        {
-            const R dslp = hs * rdst;
-            const R dflw = hr, dflw_pr = hrp;
-            R dare = rivwth * dflw;
-            dare = vmax(dare, R(1.e-10));
-            R dflw_im = vsqrt(dflw * dflw_pr);
-            dflw_im = vmax(dflw_im, R(1.e-6));
-            const R dout_pr = qr_pre * (one / rivwth);
-            const R dout = (rivwth * (dout_pr + (gdt * dflw_im) * dslp)) *
-                           (one / (one + ((gdt * (rivman * rivman)) * vabs(dout_pr)) * vpow(dflw_im, R(K_P7O3))));
-            const R dvel = qr_old * (one / dare);
-            const bool mask = (dflw_im > R(K_1EM5F)) && (dare > R(K_1EM5F));
-            q_r = mask ? dout : zero;
-            vel = mask ? dvel : zero;
-        }
-        // ---- floodplain: outflw:84-116 (river), :143-171 (mouth). Surface heights
-        // above ELEVTN = RIVELV + RIVHGT: max(SFCELV, DWNELV) - ELEVTN = hr - RIVHGT.
-        if (A.lfldout) {
-            const R gdtn2 = gdt * (R(A.pmanfld) * R(A.pmanfld));
-            const R dfsto = R(fldsto_d);
-            const R rrl = one / R(f_rivlen);
-            R dslp = hs * rdst;
-            dslp = vmax(R(-0.005), vmin(R(0.005), dslp));
-            R dflw, dflw_pr, dare, dare_pr;
-            if (river) {
-                dflw = vmax(fa, zero);
-                dare = dfsto * rrl;
-                dare = vmax(dare - flddph * rivwth, zero);
-                dflw_pr = fap;
-                dare_pr = fldsto_pre * rrl;
-                dare_pr = vmax(dare_pr - flddph_pre * rivwth, R(1.e-6));
-            } else {
-                dflw = fa;
-                dare = vmax(dfsto * rrl - flddph * rivwth, zero);
-                dflw_pr = fap;
-                dare_pr = vmax(fldsto_pre * rrl - flddph_pre * rivwth, R(1.e-6));
-            }
-            const R t = dflw * dflw_pr;
-            R dflw_im = vsqrt(vmax(t, zero));
-            dflw_im = vmax(dflw_im, R(1.e-6));
-            R dare_im = vsqrt(dare * dare_pr);
-            dare_im = vmax(dare_im, R(1.e-6));
-            const R dout_pr = fldout_pre;
-            const R dout = (dout_pr + (gdt * dare_im) * dslp) *
-                           (one / (one + ((gdtn2 * vabs(dout_pr)) * vpow(dflw_im, R(K_P4O3))) * (one / dare_im)));
-            const R thr = river ? R(1.e-5) : R(K_1EM5F);
-            const bool mask = (dflw_im > thr) && (dare > thr);
-            const R f = mask ? dout : zero;
-            q_f = (f * q_r > zero) ? f : zero;
-        }
-        // ---- reverse-flow storage limiter, river cells: outflw:175-182
+        FlowIn<R> c;
+        c.rivdph = rivdph; c.rivdph_pre = rivdph_pre; c.qr_pre = qr_pre; c.qr_old = qr_old;
+        c.fldsto = R(fldsto_d); c.flddph = flddph; c.fldsto_pre = fldsto_pre; c.fldout_pre = fldout_pre;
+        c.storge = storge;
+        c.elevtn = f_elevtn; c.rivhgt = f_rivhgt; c.rivwth = f_rivwth; c.rivman = f_rivman;
+        c.nxtdst = f_nxtdst; c.rivlen = f_rivlen;
+        c.river = river;
+        c.dj = zero; c.dj_pre = zero;
         if (river) {
-            R dout = ((-q_r) - q_f) * R(I.dt);
-            dout = vmax(dout, R(K_1EM10F));
-            R rate = (R(0.05) * storge) / dout;
-            rate = vmin(rate, one);
-            q_r = q_r * rate;
-            q_f = q_f * rate;
+            const int sj = sidx<MB>(M, nxt, m);
+            c.zdn = rivelv_of(M, nxt);
+            c.dj = S.rivdph[sj]; c.dj_pre = S.rivdph_pre[sj];
+        } else {
+            c.zdn = M.dwnelv[i];
         }
+        const Surface<R> sf = surface_of<R>(c);
+        vel = river_vel<R>(c, sf);
+        local_inertial<R>(c, sf, A.lfldout, A.pmanfld, A.pdstmth, I.dt, I.gdt, q_r, q_f);
     }
     // ---- reservoir operation: damout:316-498 (Yamazaki & Funato or Hanazaki-2022 rule)
     if (A.ldamout) {
         const int code = M.i1dam[i];
         if (code > 0) {
-            q_r = zero; q_f = zero;
             double inf = (double)S.runoff[s];                       // :447
             for (int k = M.up_ptr[i]; k < M.up_ptr[i + 1]; ++k) {   // :456-464, ascending
                 const int u = M.up_idx[k];
@@ -427,54 +268,12 @@ __device__ __forceinline__ void outflow_cell(const DevMap& M, const DevState<R>&
                 }
             }
             S.daminf[s] = inf;
-            const double dt = I.dt;
-            if (code == 10 && river) {                               // :471-493
-                const int j = nxt;
-                double dslope = ((double)M.elevtn[i] - (double)M.elevtn[j]) * (1.0 / (double)M.nxtdst[i]);
-                dslope = vmax(dslope, A.pminslp);
-                const double rd = (double)rivdph;
-                const double dvel = ((1.0 / (double)M.rivman[i]) * sqrt(dslope)) * pow(rd, K_2O3F);
-                const double darea = (double)M.rivwth[i] * rd;
-                vel = R(dvel);
-                double q = darea * dvel;
-                q_r = R(vmin(q, S.rivsto[s] / dt));
-                const double dslope_f = vmin(0.005, dslope);
-                const double fd = (double)S.flddph[s];
-                const double dvel_f = ((1.0 / A.pmanfld) * sqrt(dslope_f)) * pow(fd, K_2O3F);
-                double dare_f = S.fldsto[s] * (1.0 / (double)M.rivlen[i]);
-                dare_f = vmax(dare_f - fd * (double)M.rivwth[i], 0.0);
-                const double qf = dare_f * dvel_f;
-                q_f = R(vmin(qf, S.fldsto[s] / dt));
-            }
             const int d = M.dam_of_cell[i];
-            if (d >= 0 && M.damstat[d] > 0) {                        // :344-419
-                const double vol = S.damsto[s];
-                const double cv = M.dam_convol[d], av = M.dam_adjvol[d], ev = M.dam_emevol[d];
-                const double qn = M.dam_qn[d], qf = M.dam_qf[d], qa = M.dam_qa[d];
-                double out = 0.0;
-                if (M.ldamh22) {
-                    out = dam_rule_h22(vol, inf, M.dam_norvol[d], cv, ev, qn, qf, M.dam_r_volupa[d]);
-                } else if (vol <= cv) {
-                    out = qn * sqrt(vol / cv);
-                } else if (vol > cv && vol <= av) {
-                    const double xx = (vol - cv) / (av - cv);
-                    out = qn + (xx * (xx * xx)) * (qa - qn);
-                } else if (vol > av && vol <= ev) {
-                    if (inf >= qf) {
-                        out = qn + ((vol - cv) / (ev - cv)) * (inf - qn);
-                        const double tmp = qa + pow((vol - av) / (ev - av), K_0P1F) * (qf - qa);
-                        out = vmax(out, tmp);
-                    } else {
-                        out = qa + pow((vol - av) / (ev - av), K_0P1F) * (qf - qa);
-                    }
-                } else if (vol > ev) {
-                    out = (inf >= qf) ? inf : qf;
-                }
-                out = vmin(vmin(out, vol / dt), (S.rivsto[s] + S.fldsto[s]) / dt);
-                out = vmax(out, 0.0);
-                q_r = R(out);
-                q_f = zero;
-            }
+            const bool kine = code == 10 && river;
+            double vk = 0.0, vf = 0.0;
+            if (kine) dam_kine_factors(M, A.pminslp, A.pmanfld, i, nxt, vk, vf);
+            dam_outflow<R>(M, kine, vk, vf, f_rivwth, f_rivlen, d >= 0 && M.damstat[d] > 0, d, inf, I.dt, rivdph,
+                           S.flddph[s], S.rivsto[s], S.fldsto[s], d >= 0 ? S.damsto[s] : 0.0, q_r, q_f, vel);
         }
     }
     S.qr_u[s] = q_r;
@@ -735,28 +534,15 @@ __device__ __forceinline__ void update_cell(const DevMap& M, const DevState<R>& 
     S.rivout[s] = qrl;
     S.fldout[s] = qfl;
     S.fldsto_pre[s] = R(fs);
-    // CMF_CALC_STONXT, stonxt:54-98
-    g[G_STOPRE] = rs + fs;
-    g[G_RIVINF] = rinf * dt + finf * dt;
-    g[G_RIVOUT] = ((double)qrl * dt + (double)qfl * dt) + pout * dt;
-    rs = (rs + rinf * dt) - (double)qrl * dt;
-    if (rs < 0.0) { fs = fs + rs; rs = 0.0; }
-    fs = ((fs + finf * dt) - (double)qfl * dt) - pout * dt;
-    if (fs < 0.0) { rs = vmax(rs + fs, 0.0); fs = 0.0; }
-    g[G_STONXT] = rs + fs;
     const R outflw = qrl + qfl;
-    R drivrof = (runoff * (R(1) - fldfrc_old)) * R(dt);
-    const R dfldrof = (runoff * fldfrc_old) * R(dt);
-    if (A.lupsinf) drivrof = drivrof + upsinf * R(dt);             // stonxt:81
-    rs = rs + (double)drivrof;
-    fs = fs + (double)dfldrof;
+    storage_next<R>(rs, fs, rinf, finf, pout, qrl, qfl, dt, runoff, fldfrc_old, A.lupsinf, upsinf, g);
     double st = rs + fs;
     if (A.llevee) st = st + levsto;
     g[G_STONEW] = (double)R(st);
     // CMF_PHYSICS_FLDSTG
     Stage o;
-    if (A.llevee) stage_levee(M, i, geo, lev, rs, fs, levsto, o);
-    else stage_def(M, i, geo, rs, fs, o);
+    if (A.llevee) stage_levee(M, MapHgt(M, i), geo, lev, rs, fs, levsto, o);
+    else stage_def(M, MapHgt(M, i), geo, rs, fs, o);
     S.rivsto[s] = o.rivsto;
     S.fldsto[s] = o.fldsto;
     const R rivdph = R(o.rivdph);
@@ -887,10 +673,14 @@ __device__ __forceinline__ void update_tile(const DevMap& M, const DevState<R>& 
         // budget sums are kept for single-instance handles only (MB = false), so
         // the ensemble kernels carry no budget registers
         if (!MB && A.budget) {
-            block_sum_comp<BS, NGLB>(g, lds);
+            double h, l;
+            block_sum_comp<BS>(g, nullptr, lds, h, l);
             // per-substep slot: reduced once for all substeps at the end of the outer step
-            if (threadIdx.x < NGLB)
-                S.partials[((size_t)A.prow * ntc + t) * NGLB + threadIdx.x] = lds[threadIdx.x * (BS / 64)];
+            if (threadIdx.x < NGLB) {
+                double* part = S.partials + ((size_t)A.prow * ntc + t) * NPART;
+                part[threadIdx.x] = h;
+                part[NGLB + threadIdx.x] = l;
+            }
             __syncthreads();
         }
     } else {
@@ -991,22 +781,17 @@ __global__ __launch_bounds__(BS) void k_substep(DevMap M, DevState<R> S, StepArg
 constexpr int RBS = 256;
 __global__ __launch_bounds__(RBS) void k_reduce_budget(const double* partials, int nb, double* out) {
     __shared__ double lds[2 * NGLB * (RBS / 64)];
-    const double* src = partials + (size_t)blockIdx.x * nb * NGLB;
+    const double* src = partials + (size_t)blockIdx.x * nb * NPART;
     double v[NGLB], lo[NGLB];
 #pragma unroll
     for (int k = 0; k < NGLB; ++k) { v[k] = 0.0; lo[k] = 0.0; }
     for (int b = threadIdx.x; b < nb; b += RBS)
 #pragma unroll
-        for (int k = 0; k < NGLB; ++k) {
-            double sh, e;
-            two_sum(v[k], src[(size_t)b * NGLB + k], sh, e);
-            v[k] = sh;
-            lo[k] = lo[k] + e;
-        }
-#pragma unroll
-    for (int k = 0; k < NGLB; ++k) v[k] = v[k] + lo[k];
-    block_sum_comp<RBS, NGLB>(v, lds);
-    if (threadIdx.x < NGLB) out[(size_t)blockIdx.x * NGLB + threadIdx.x] = lds[threadIdx.x * (RBS / 64)];
+        for (int k = 0; k < NGLB; ++k)
+            comp_add(v[k], lo[k], src[(size_t)b * NPART + k], src[(size_t)b * NPART + NGLB + k]);
+    double h, l;
+    block_sum_comp<RBS>(v, lo, lds, h, l);
+    if (threadIdx.x < NGLB) out[(size_t)blockIdx.x * NGLB + threadIdx.x] = h + l;
 }
 
 // ---------------------------------------------------------------------------
@@ -1033,8 +818,8 @@ __device__ __forceinline__ double stage_slot(const DevMap& M, const DevState<R>&
     Stage o;
     const double levsto = A.llevee ? S.levsto[s] : 0.0;
     const Geom geo = load_geom(M, i);
-    if (A.llevee) stage_levee(M, i, geo, load_lev(M, i), S.rivsto[s], S.fldsto[s], levsto, o);
-    else stage_def(M, i, geo, S.rivsto[s], S.fldsto[s], o);
+    if (A.llevee) stage_levee(M, MapHgt(M, i), geo, load_lev(M, i), S.rivsto[s], S.fldsto[s], levsto, o);
+    else stage_def(M, MapHgt(M, i), geo, S.rivsto[s], S.fldsto[s], o);
     S.rivsto[s] = o.rivsto;
     S.fldsto[s] = o.fldsto;
     const R rivdph = R(o.rivdph);

@@ -298,7 +298,7 @@ int cmf_hip_physics_advance(cmf_handle h, double* dt, int32_t* nt_out,
  * step the model (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc). It calls no hipMalloc/hipFree and no allocating
  * library routine: the budget partial sums, the budget rows and the CFL partial
- * minima live in a fixed 6.65 MB device array of the library (one copy per GPU,
+ * minima live in a fixed 12.4 MB device array of the library (one copy per GPU,
  * held until the process ends; its address is looked up when a handle is
  * created). Same semantics and results as cmf_hip_physics_advance (the
  * substeps always run as three phase kernels; no graph replay, no event
