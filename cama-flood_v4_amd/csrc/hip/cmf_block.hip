@@ -1,0 +1,674 @@
+// cmf_block.hip -- many substeps of a single model per launch.
+//
+// The three-phase kernels (cmf_kernels.hip) stream the whole state through HBM on
+// every substep and meet the grid between phases. River networks do not need
+// that: a cell depends on its neighbours along the river only, two cells
+// downstream and two upstream per substep (the limiter rate of a cell needs the
+// outflows of its upstream cells, and those their downstream depths). So the
+// network is cut into blocks of T cells, one workgroup each, one cell per thread:
+// whole basins where they fit, connected parts of larger ones. A block also loads
+// the cells within reach of its own over the kmax substeps of a launch and steps
+// those redundantly, a shrinking ring of them as the substeps pass, so no block
+// waits for another. State lives in registers and LDS between the substeps; HBM
+// sees it once per launch. Every value is computed by the statements of the
+// three-phase kernels on the same inputs, so results are the same bits.
+#include "cmf_block.hpp"
+
+#include <algorithm>
+
+namespace cmf {
+
+// ---------------------------------------------------------------------------
+// Partition. Cells come in depth-first order (every cell after its upstream
+// subtree). Basins of at most T cells stay whole; larger ones are cut bottom-up
+// into connected pieces of at most `cap` cells, so a piece has one downstream cut
+// and about one upstream cut. The dependency sets of a piece, r counting the
+// substeps that follow in the launch:
+//   U_0     = the owned cells
+//   R_r     = U_r + upstream(U_r) + downstream(U_r)      limiter rates needed
+//   Q_r     = R_r + upstream(R_r)                        outflows needed
+//   U_(r+1) = Q_r + downstream(Q_r) + upstream(dam cells of Q_r)
+// (a dam's inflow is the previous flow of its upstream cells). code = position of
+// the first set a cell is in: U_r <= 3r, R_r <= 3r+1, Q_r <= 3r+2.
+bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
+                      const uint8_t* special, int T, int kmax, BlockPlan& out) {
+    out = BlockPlan();
+    if (n <= 0 || T > 1024 || kmax < 1 || 3 * kmax > 200) return false;
+    const int cap = std::max(T / 4, T - 48 * kmax);
+    std::vector<int32_t> total((size_t)n, 1), resid((size_t)n), piece((size_t)n);
+    std::vector<uint8_t> root((size_t)n, 0);
+    for (int p = 0; p < n; ++p) {
+        if (up_ptr[p + 1] - up_ptr[p] > 250) return false;
+        if (next[p] >= 0) {
+            if (next[p] <= p) return false;                        // needs the depth-first order
+            total[(size_t)next[p]] += total[(size_t)p];
+        }
+    }
+    // basin sizes, then the cuts
+    for (int p = n - 1; p >= 0; --p) piece[(size_t)p] = next[p] >= 0 ? piece[(size_t)next[p]] : total[(size_t)p];
+    bool closed = true;
+    for (int p = 0; p < n; ++p) {
+        const int lim = piece[(size_t)p] <= T ? T : cap;
+        closed = closed && lim == T;
+        int r = 1;
+        for (int k = up_ptr[p]; k < up_ptr[p + 1]; ++k)
+            if (!root[(size_t)up_idx[k]]) r += resid[(size_t)up_idx[k]];
+        while (r > lim) {
+            int b = -1;
+            for (int k = up_ptr[p]; k < up_ptr[p + 1]; ++k) {
+                const int u = up_idx[k];
+                if (!root[(size_t)u] && (b < 0 || resid[(size_t)u] > resid[(size_t)b])) b = u;
+            }
+            root[(size_t)b] = 1;
+            r -= resid[(size_t)b];
+        }
+        resid[(size_t)p] = r;
+        if (next[p] < 0) root[(size_t)p] = 1;
+    }
+    int npc = 0;
+    for (int p = n - 1; p >= 0; --p) piece[(size_t)p] = root[(size_t)p] ? npc++ : piece[(size_t)next[p]];
+    // owned cells of every piece, ascending
+    std::vector<int32_t> off((size_t)npc + 1, 0), own((size_t)n);
+    for (int p = 0; p < n; ++p) off[(size_t)piece[(size_t)p] + 1] += 1;
+    for (int i = 0; i < npc; ++i) off[(size_t)i + 1] += off[(size_t)i];
+    {
+        std::vector<int32_t> fill(off.begin(), off.end() - 1);
+        for (int p = 0; p < n; ++p) own[(size_t)fill[(size_t)piece[(size_t)p]]++] = p;
+    }
+    // local cells (owned first) and codes of every piece; a piece whose
+    // surroundings overfill a block is halved
+    struct Piece { int32_t beg, size, spec, dams, kines; };        // into loc / codes; special cells
+    std::vector<Piece> done;
+    std::vector<int32_t> loc, mark((size_t)n, -1), cur;
+    std::vector<uint8_t> codes, curc;
+    loc.reserve((size_t)n + (size_t)n / 4);
+    codes.reserve((size_t)n + (size_t)n / 4);
+    const int max_spec = blk_special(T);
+    const int max_dams = blk_dams(T), max_kines = blk_kines(T);
+    auto piece_of = [&](const std::vector<int32_t>& c, size_t from, int count) {
+        Piece p{(int32_t)loc.size(), count, 0, 0, 0};
+        for (int j = 0; special && j < count; ++j) {
+            const uint8_t f = special[(size_t)c[from + j]];
+            p.spec += (f & (BLK_DAM | BLK_LEV)) != 0;
+            p.kines += (f & BLK_KINE) != 0;
+            p.dams += (f & BLK_DAM) && !(f & BLK_KINE);
+        }
+        return p;
+    };
+    auto fits = [&](const Piece& p) { return p.size <= T && p.spec <= max_spec && p.dams <= max_dams && p.kines <= max_kines; };
+    std::vector<std::vector<int32_t>> work;
+    int stamp = 0;
+    for (int i = 0; i < npc; ++i) {
+        const int a = off[(size_t)i], b = off[(size_t)i + 1], rt = own[(size_t)b - 1];
+        const Piece whole = piece_of(own, (size_t)a, b - a);
+        if (next[rt] < 0 && total[(size_t)rt] == b - a && fits(whole)) {   // a whole basin
+            done.push_back(whole);
+            loc.insert(loc.end(), own.begin() + a, own.begin() + b);
+            codes.insert(codes.end(), (size_t)(b - a), (uint8_t)0);
+            continue;
+        }
+        work.assign(1, std::vector<int32_t>(own.begin() + a, own.begin() + b));
+        while (!work.empty()) {
+            cur.swap(work.back());
+            work.pop_back();
+            const int nown = (int)cur.size(), id = stamp++;
+            curc.assign((size_t)nown, 0);
+            for (int x : cur) mark[(size_t)x] = id;
+            uint8_t c = 0;
+            auto add = [&](int x) {
+                if (x >= 0 && mark[(size_t)x] != id) { mark[(size_t)x] = id; cur.push_back(x); curc.push_back(c); }
+            };
+            auto add_up = [&](int x) { for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) add(up_idx[k]); };
+            size_t r0 = 0, q0 = 0;                                  // members whose neighbours are already in
+            for (int r = 0; r < kmax && (int)cur.size() <= T; ++r) {
+                const size_t eu = cur.size();
+                c = (uint8_t)(3 * r + 1);
+                for (size_t j = r0; j < eu; ++j) { add_up(cur[j]); add(next[cur[j]]); }
+                const size_t er = cur.size();
+                c = (uint8_t)(3 * r + 2);
+                for (size_t j = r0; j < er; ++j) add_up(cur[j]);
+                const size_t eq = cur.size();
+                c = (uint8_t)(3 * r + 3);
+                for (size_t j = q0; j < eq; ++j) {
+                    add(next[cur[j]]);
+                    if (special && (special[(size_t)cur[j]] & BLK_DAMUP)) add_up(cur[j]);
+                }
+                r0 = er;
+                q0 = eq;
+            }
+            const Piece pc = piece_of(cur, 0, (int)cur.size());
+            if (fits(pc)) {
+                done.push_back(pc);
+                closed = closed && (int)cur.size() == nown;
+                loc.insert(loc.end(), cur.begin(), cur.end());
+                codes.insert(codes.end(), curc.begin(), curc.end());
+                continue;
+            }
+            if (nown < 2) return false;
+            // halve: cut above the cell whose subtree inside the piece is nearest to half
+            cur.resize((size_t)nown);
+            const int idp = stamp++;
+            for (int x : cur) { mark[(size_t)x] = idp; resid[(size_t)x] = 1; }
+            int best = -1, bd = n;
+            for (int x : cur) {
+                const int d = std::abs(2 * resid[(size_t)x] - nown);
+                if (x != cur.back() && d < bd) { bd = d; best = x; }
+                if (next[x] >= 0 && mark[(size_t)next[x]] == idp) resid[(size_t)next[x]] += resid[(size_t)x];
+            }
+            std::vector<int32_t> lo, hi;
+            const int idh = stamp++;
+            for (int j = nown - 1; j >= 0; --j) {
+                const int x = cur[(size_t)j];
+                if (x == best || (next[x] >= 0 && mark[(size_t)next[x]] == idh)) mark[(size_t)x] = idh;
+            }
+            for (int x : cur) (mark[(size_t)x] == idh ? hi : lo).push_back(x);
+            work.push_back(std::move(lo));
+            work.push_back(std::move(hi));
+        }
+    }
+    // pieces into blocks: the large ones best-fit by descending size, the small
+    // ones fill the room that is left, in order
+    std::vector<std::vector<int32_t>> bins;
+    std::vector<Piece> room;                                       // what is left in each
+    {
+        auto holds = [](const Piece& r, const Piece& p) {
+            return r.size >= p.size && r.spec >= p.spec && r.dams >= p.dams && r.kines >= p.kines;
+        };
+        auto put = [&](int b, size_t k) {
+            if (b < 0) {
+                b = (int)bins.size();
+                bins.emplace_back();
+                room.push_back({0, T, max_spec, max_dams, max_kines});
+            }
+            const Piece& p = done[k];
+            Piece& r = room[(size_t)b];
+            bins[(size_t)b].push_back((int32_t)k);
+            r.size -= p.size; r.spec -= p.spec; r.dams -= p.dams; r.kines -= p.kines;
+            return b;
+        };
+        std::vector<std::vector<int32_t>> by_size((size_t)T + 1), by_room((size_t)T + 1);
+        const int small = T / 16;
+        for (size_t k = 0; k < done.size(); ++k)
+            if (done[k].size > small) by_size[(size_t)done[k].size].push_back((int32_t)k);
+        for (int s = T; s > small; --s)
+            for (int32_t k : by_size[(size_t)s]) {
+                int b = -1;
+                for (int r = s; r <= T && b < 0; ++r)
+                    if (!by_room[(size_t)r].empty() && holds(room[(size_t)by_room[(size_t)r].back()], done[(size_t)k])) {
+                        b = by_room[(size_t)r].back();
+                        by_room[(size_t)r].pop_back();
+                    }
+                b = put(b, (size_t)k);
+                by_room[(size_t)room[(size_t)b].size].push_back(b);
+            }
+        size_t b = 0;
+        for (size_t k = 0; k < done.size(); ++k) {
+            if (done[k].size > small) continue;
+            while (b < bins.size() && !holds(room[b], done[k])) ++b;
+            put(b < bins.size() ? (int)b : -1, k);
+        }
+    }
+    const int nb = (int)bins.size();
+    const size_t np = (size_t)nb * (size_t)T;
+    out.T = T; out.kmax = kmax; out.nblk = nb; out.closed = closed;
+    out.cell.assign(np, -1);
+    out.topo.assign(2 * np, 0);
+    out.upx_ptr.assign(np, 0);
+    out.ndam.assign((size_t)nb, 0);
+    // order inside a block: dam, kinematic and levee cells in places of their own
+    // (their wavefronts take the rare paths, the others never do), then the owned
+    // cells, then the ring by code
+    std::vector<int32_t>& pos = resid;                               // local index in the block
+    std::vector<int32_t> place((size_t)T), count((size_t)3 * kmax + 6), spot((size_t)T);
+    std::fill(mark.begin(), mark.end(), -1);
+    for (int b = 0; b < nb; ++b) {
+        const std::vector<int32_t>& bin = bins[(size_t)b];
+        auto code_of = [&](size_t e) { return closed ? 0 : (int)codes[e]; };
+        auto key_of = [&](size_t e) {
+            const uint8_t f = special ? special[(size_t)loc[e]] : 0;
+            return f & BLK_KINE ? 1 : (f & BLK_DAM ? 0 : (f & BLK_LEV ? 2 : 3 + code_of(e)));
+        };
+        std::fill(count.begin(), count.end(), 0);
+        for (int32_t k : bin)
+            for (int j = 0; j < done[(size_t)k].size; ++j) count[(size_t)key_of((size_t)done[(size_t)k].beg + j) + 1] += 1;
+        const int na = count[1], nk = count[2];
+        out.ndam[(size_t)b] = na | (nk << 16);
+        for (size_t i = 0; i + 1 < count.size(); ++i) count[i + 1] += count[i];
+        // spot[rank in that order] = place
+        for (int i = 0; i < na; ++i) spot[(size_t)i] = i;
+        for (int i = 0; i < nk; ++i) spot[(size_t)(na + i)] = BLK_KINE_AT + i;
+        for (int i = na + nk, l = na; i < T; ++i, ++l) {
+            if (nk > 0 && l == BLK_KINE_AT) l += nk;
+            spot[(size_t)i] = l;
+        }
+        int q = 0;
+        for (int32_t k : bin)
+            for (int j = 0; j < done[(size_t)k].size; ++j, ++q)
+                place[(size_t)q] = spot[(size_t)count[(size_t)key_of((size_t)done[(size_t)k].beg + j)]++];
+        q = 0;
+        for (int32_t k : bin) {
+            const Piece& pc = done[(size_t)k];
+            // a piece's neighbours are looked up inside the piece: two pieces of one
+            // block may both hold a cell
+            for (int j = 0; j < pc.size; ++j) {
+                const int x = loc[(size_t)pc.beg + j];
+                mark[(size_t)x] = k;
+                pos[(size_t)x] = place[(size_t)(q + j)];
+            }
+            for (int j = 0; j < pc.size; ++j, ++q) {
+                const int x = loc[(size_t)pc.beg + j];
+                const int code = code_of((size_t)pc.beg + j);
+                const size_t e0 = (size_t)b * T + place[(size_t)q];
+                uint32_t nx = TOPO_MOUTH;
+                if (next[x] >= 0) {
+                    const bool in = mark[(size_t)next[x]] == k;
+                    if (!in && code <= 3 * (kmax - 1) + 2) return false;   // cannot be
+                    nx = in ? (uint32_t)pos[(size_t)next[x]] : (uint32_t)place[(size_t)q];
+                }
+                int nup = up_ptr[x + 1] - up_ptr[x];
+                for (int e = up_ptr[x]; e < up_ptr[x + 1]; ++e)
+                    if (mark[(size_t)up_idx[e]] != k) {
+                        if (code <= 3 * (kmax - 1) + 1) return false;      // cannot be
+                        nup = 0;                                      // never asked for
+                        break;
+                    }
+                const uint32_t u0 = nup > 0 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x]]] : 0u;
+                const uint32_t u1 = nup > 1 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x] + 1]] : u0;
+                const uint32_t fl = special ? special[(size_t)x] & (BLK_DAM | BLK_LEV) : 0u;
+                out.cell[e0] = x;
+                out.topo[e0] = nx | (u0 << TOPO_UP0) | (fl << TOPO_FLAGS);
+                out.topo[np + e0] = u1 | ((uint32_t)nup << TOPO_NUP) | ((uint32_t)code << TOPO_CODE);
+                if (nup > 2) {
+                    out.upx_ptr[e0] = (int32_t)out.upx.size();
+                    for (int e = up_ptr[x] + 2; e < up_ptr[x + 1]; ++e)
+                        out.upx.push_back((uint16_t)pos[(size_t)up_idx[e]]);
+                }
+            }
+        }
+        for (int l = 0; l < T; ++l)
+            if (out.cell[(size_t)b * T + l] < 0) out.topo[np + (size_t)b * T + l] = 255u << TOPO_CODE;   // idle
+    }
+    if (out.upx.empty()) out.upx.push_back(0);
+    return true;
+}
+
+// ---------------------------------------------------------------------------
+// Values of the cells of a block between the phases and substeps. With FP64 state
+// the arrays of T cells take 120 bytes a cell and the first NL floodplain heights 20
+// more, which fills the 160 KB of a CU with 1024 cells; the mixed form has room for
+// all heights.
+template <class R, int T, bool LEV, bool DAM>
+struct BlockLds {
+    static constexpr bool kOutSum = sizeof(R) == sizeof(float);
+    static constexpr int NL = kOutSum ? 8 : 5, NS = blk_special(T), ND = blk_dams(T) + blk_kines(T);
+    R dph[T], dphp[T], q[T], f[T], rate[T];    // read by neighbours
+    R fpre[T], fdph[T], ffrc[T];               // own floodplain state
+    R a_riv[T], a_fld[T], a_vel[T], a_out[kOutSum ? 1 : T], m_out[T], m_dph[T], m_sto[T];
+    float hgt[NL][T];
+    double sum[2 * NGLB * (T / 64)];
+    // dam and kinematic cells (slot_of_dam), levee cells
+    double dam[DAM ? ND : 1], daminf[DAM ? ND : 1], vk[DAM ? ND : 1], vf[DAM ? ND : 1];
+    R a_inf[DAM ? ND : 1], ro[DAM ? ND : 1], fo[DAM ? ND : 1];   // average of DAMINF; limited flows, read downstream
+    int32_t drow[DAM ? ND : 1], dcode[DAM ? ND : 1];
+    double lev[LEV ? NS : 1];
+    int32_t lrow[LEV ? NS : 1];
+};
+enum { DAM_CODE = 15, DAM_KINE = 16, DAM_ACTIVE = 32, DAM_BALANCE = 64 };   // bits of dcode (I1DAM below)
+__device__ __forceinline__ int slot_of_dam(int l, int T) { return l < BLK_KINE_AT ? l : l - BLK_KINE_AT + blk_dams(T); }
+template <int NL, int T>
+struct BlockHgt {
+    const float *s, *h;
+    int n;
+    __device__ __forceinline__ float operator()(int l) const {
+        return l <= NL ? s[(l - 1) * T] : h[(size_t)(l - 1) * n];
+    }
+};
+
+template <class R>
+struct BlockArgs {
+    DevMap M;
+    DevState<R> S;
+    BlockState<R> O;
+    BlockTab P;
+    StepArgs A;
+    InstStep I;
+    int it0, nsub;
+    const R* vel0;
+};
+
+// The kernel's arguments, re-read through an opaque pointer: the substep loop is
+// long, and pointers and constants loaded once for all of it would not fit the
+// scalar registers (they would spill into vector lanes); a scalar load where one
+// is used hits the constant cache.
+template <class R>
+__device__ __forceinline__ const BlockArgs<R>& block_args() {
+    typedef const __attribute__((address_space(4))) BlockArgs<R>* cptr;
+    cptr p = (cptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const BlockArgs<R>*)p;
+}
+
+template <class R, int T, bool LEV, bool DAM>
+__global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block(BlockArgs<R> args_) {
+    constexpr bool kOutSum = sizeof(R) == sizeof(float);
+    constexpr int NW = T / 64;
+    // budget terms formed before the stage inversion (STOPRE2 is STONEW in FP64) and after it
+    constexpr int NA = kOutSum ? G_STOPRE2 + 1 : G_STOPRE2, NB = (LEV ? NGLB : G_LEVSTO) - G_STONEW2;
+    __shared__ BlockLds<R, T, LEV, DAM> L;
+    int l = threadIdx.x;
+    const int b = blockIdx.x;
+    int g;
+    uint32_t w0, w1;
+    const R zero = R(0);
+    double rs = 0.0, fs = 0.0, zdn = 0.0;
+    R ro = zero, fo = zero;
+    float f_elevtn = 0.f, f_nxtdst = 1.f, f_rivman = 1.f, f_rivlen = 1.f, f_rivwth = 1.f, f_grarea = 1.f, f_rivhgt = 1.f;
+    {
+        const BlockArgs<R>& a = block_args<R>();
+        const DevMap& M = a.M;
+        const DevState<R>& S = a.S;
+        const BlockTab& P = a.P;
+        const int pl = b * T + l;
+        g = P.cell[pl];
+        w0 = P.topo[pl];
+        w1 = P.topo[(size_t)P.nblk * T + pl];
+        const bool mouth = (w0 & TOPO_MOUTH) == TOPO_MOUTH;
+        if (g >= 0) {
+            rs = S.rivsto[g]; fs = S.fldsto[g];
+            ro = S.rivout[g]; fo = S.fldout[g];
+            L.dph[l] = S.rivdph[g]; L.dphp[l] = S.rivdph_pre[g];
+            L.fpre[l] = S.fldsto_pre[g]; L.fdph[l] = S.flddph[g]; L.ffrc[l] = S.fldfrc[g];
+            f_rivlen = M.rivlen[g]; f_rivwth = M.rivwth[g]; f_grarea = M.grarea[g]; f_rivhgt = M.rivhgt[g];
+            f_elevtn = M.elevtn[g]; f_nxtdst = M.nxtdst[g]; f_rivman = M.rivman[g];
+            if (mouth) zdn = M.dwnelv[g];
+            using Lds = BlockLds<R, T, LEV, DAM>;
+#pragma unroll
+            for (int k = 0; k < Lds::NL; ++k)
+                if (k < M.nlfp) L.hgt[k][l] = M.fldhgt[(size_t)k * M.n + g];
+            if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) { L.lev[l] = S.levsto[g]; L.lrow[l] = M.lev_idx[g]; }
+            if (DAM && (w0 & (BLK_DAM << TOPO_FLAGS))) {
+                const int e = slot_of_dam(l, T);
+                const int c = M.i1dam[g], d = M.dam_of_cell[g];
+                int bits = c > 0 ? c & DAM_CODE : 0;
+                if (c == 10 && !mouth) {
+                    bits |= DAM_KINE;
+                    double vk, vf;
+                    dam_kine_factors(M, a.A.pminslp, a.A.pmanfld, g, M.next[g], vk, vf);
+                    L.vk[e] = vk; L.vf[e] = vf;
+                }
+                if (d >= 0 && M.damstat[d] > 0) bits |= DAM_ACTIVE;
+                if (d >= 0 && M.damstat[d] != -9999) bits |= DAM_BALANCE;
+                L.dcode[e] = bits; L.drow[e] = d;
+                const bool mine = (w1 >> TOPO_CODE) == 0;
+                L.dam[e] = S.damsto[g]; L.daminf[e] = mine ? S.daminf[g] : 0.0;
+                L.a_inf[e] = mine && a.it0 > 0 ? S.daminf_avg[g] : zero;
+                L.ro[e] = ro; L.fo[e] = fo;
+            }
+        }
+        const bool cont = (w1 >> TOPO_CODE) == 0 && a.it0 > 0;
+        L.a_riv[l] = cont ? S.rivout_avg[g] : zero;
+        L.a_fld[l] = cont ? S.fldout_avg[g] : zero;
+        L.a_vel[l] = cont ? S.rivvel_avg[g] : zero;
+        if (!kOutSum) L.a_out[l] = cont ? S.outflw_avg[g] : zero;
+        L.m_out[l] = cont ? S.outflw_max[g] : zero;
+        L.m_dph[l] = cont ? S.rivdph_max[g] : zero;
+        L.m_sto[l] = cont ? S.storge_max[g] : zero;
+        // the downstream cell's bed, through LDS
+        L.q[l] = R(f_elevtn); L.f[l] = R(f_rivhgt);
+        __syncthreads();
+        if (!mouth) {
+            const int nx = (int)(w0 & TOPO_MOUTH);
+            zdn = (double)L.q[nx] - (double)L.f[nx];
+        }
+    }
+    const int nsub = args_.nsub, it0 = args_.it0, nt = args_.I.nt;
+    const double dt = args_.I.dt, gdt = args_.I.gdt;
+    __syncthreads();
+    for (int s = 0; s < nsub; ++s) {
+        // what follows from these is formed anew in every substep: kept across the
+        // loop it would take twice the registers there are
+        asm volatile("" : "+v"(f_elevtn), "+v"(f_nxtdst), "+v"(f_rivman), "+v"(f_rivlen), "+v"(f_rivwth), "+v"(f_grarea),
+                     "+v"(f_rivhgt), "+v"(w0), "+v"(w1), "+v"(g), "+v"(l));
+        const BlockArgs<R>& a = block_args<R>();
+        const DevMap& M = a.M;
+        const DevState<R>& S = a.S;
+        const BlockTab& P = a.P;
+        const StepArgs& A = a.A;
+        const R rdt = R(dt);
+        const int nx = (int)(w0 & TOPO_MOUTH);
+        const bool river = nx != (int)TOPO_MOUTH;
+        const int u0 = (int)(w0 >> TOPO_UP0) & 0x3ff, u1 = (int)(w1 & 0x3ffu), nup = (int)(w1 >> TOPO_NUP) & 0xff;
+        // an idle lane is in no set, however many substeps remain
+        const int code = g < 0 ? 0x7fffffff : (int)(w1 >> TOPO_CODE);
+        const bool own = code == 0;
+        const bool is_dam = DAM && (w0 & (BLK_DAM << TOPO_FLAGS));
+        const int e = slot_of_dam(l, T);
+        const bool is_lev = LEV && (w0 & (BLK_LEV << TOPO_FLAGS));
+        const int it = it0 + s, rem = nsub - 1 - s;
+        const bool last = it == nt - 1;
+        // ---- outflow (k_outflow)
+        if (code <= 3 * rem + 2) {
+            FlowIn<R> c;
+            c.rivdph = L.dph[l]; c.rivdph_pre = L.dphp[l];
+            c.qr_pre = ro;
+            c.qr_old = s == 0 && a.vel0 ? a.vel0[g] : c.qr_pre;
+            c.fldsto = R(fs); c.flddph = L.fdph[l]; c.fldsto_pre = L.fpre[l];
+            c.fldout_pre = fo;
+            double stg = rs + fs;
+            if (is_lev) stg = stg + L.lev[l];
+            c.storge = R(stg);
+            c.elevtn = f_elevtn; c.rivhgt = f_rivhgt; c.rivwth = f_rivwth; c.rivman = f_rivman;
+            c.nxtdst = f_nxtdst; c.rivlen = f_rivlen;
+            c.river = river;
+            c.dj = river ? L.dph[nx] : zero;
+            c.dj_pre = river ? L.dphp[nx] : zero;
+            c.zdn = zdn;
+            const Surface<R> sf = surface_of<R>(c);
+            R q_r, q_f, vel = river_vel<R>(c, sf);
+            const int bits = is_dam ? L.dcode[e] : 0;
+            if (!DAM || !(bits & DAM_CODE)) {
+                local_inertial<R>(c, sf, A.lfldout, A.pmanfld, A.pdstmth, dt, gdt, q_r, q_f);
+            } else {
+                const BlockArgs<R>& ad = block_args<R>();
+                double inf = (double)ad.S.runoff[g];                      // damout:447-464
+                const int nd = ad.P.ndam[b];
+                for (int k = 0; k < nup; ++k) {
+                    const int u = k == 0 ? u0 : (k == 1 ? u1 : (int)ad.P.upx[ad.P.upx_ptr[b * T + l] + k - 2]);
+                    const bool dam_up = u < (nd & 0xffff) || (u >= BLK_KINE_AT && u < BLK_KINE_AT + (nd >> 16));
+                    const int eu = dam_up ? slot_of_dam(u, T) : 0;
+                    const int cu = dam_up ? L.dcode[eu] & DAM_CODE : 0;
+                    if (cu == 10 || cu == 11) inf = (inf + (double)L.ro[eu]) + (double)L.fo[eu];
+                }
+                L.daminf[e] = inf;
+                dam_outflow<R>(ad.M, (bits & DAM_KINE) != 0, L.vk[e], L.vf[e], f_rivwth, f_rivlen,
+                               (bits & DAM_ACTIVE) != 0, L.drow[e], inf, dt, L.dph[l], L.fdph[l], rs, fs, L.dam[e],
+                               q_r, q_f, vel);
+            }
+            L.q[l] = q_r;
+            L.f[l] = q_f;
+            if (own) {
+                if (last) S.rivvel[g] = vel;
+                L.a_vel[l] = L.a_vel[l] + vel * rdt;
+            }
+        }
+        __syncthreads();
+        const bool upd = code <= 3 * rem;
+        const R runoff = upd ? S.runoff[g] : zero;                        // in flight during the rate phase
+        // ---- limiter rate (k_rate)
+        if (code <= 3 * rem + 1) {
+            double so = (double)vmax(L.q[l], zero) + (double)vmax(L.f[l], zero);
+            if (nup > 0) so = (so + (double)vmax(-L.q[u0], zero)) + (double)vmax(-L.f[u0], zero);
+            if (nup > 1) so = (so + (double)vmax(-L.q[u1], zero)) + (double)vmax(-L.f[u1], zero);
+            for (int k = 2; k < nup; ++k) {
+                const int u = P.upx[P.upx_ptr[b * T + l] + k - 2];
+                so = (so + (double)vmax(-L.q[u], zero)) + (double)vmax(-L.f[u], zero);
+            }
+            so = so * dt;
+            const R dout = vmax(R(so), R(1.e-10));
+            L.rate[l] = vmin(R(rs + fs) / dout, R(1));
+        }
+        __syncthreads();
+        // ---- limit, inflow, dam balance, storages (k_update)
+        {
+            double gb[NGLB];
+#pragma unroll
+            for (int k = 0; k < NGLB; ++k) gb[k] = 0.0;
+            if (upd) {
+                const R qr = L.q[l], qf = L.f[l], ri = L.rate[l];
+                const R r = (river && !(qr > zero)) ? L.rate[nx] : ri;
+                const R qrl = qr * r, qfl = qf * r;
+                double rivinf = 0.0, fldinf = 0.0;
+                auto inflow = [&](int u) {
+                    const R qu = L.q[u], fu = L.f[u];
+                    const R ru = (qu > zero) ? L.rate[u] : ri;
+                    rivinf = rivinf + (double)(qu * ru);
+                    fldinf = fldinf + (double)(fu * ru);
+                };
+                if (nup > 0) inflow(u0);
+                if (nup > 1) inflow(u1);
+                for (int k = 2; k < nup; ++k) inflow(P.upx[P.upx_ptr[b * T + l] + k - 2]);
+                if (is_dam && (L.dcode[e] & DAM_BALANCE))
+                    L.dam[e] = (L.dam[e] + ((rivinf + fldinf) + (double)runoff) * dt) - ((double)qrl + (double)qfl) * dt;
+                L.fpre[l] = R(fs);
+                const R outflw = qrl + qfl;
+                storage_next<R>(rs, fs, rivinf, fldinf, 0.0, qrl, qfl, dt, runoff, L.ffrc[l], A.lupsinf,
+                                A.lupsinf ? S.upsinf[g] : zero, gb);
+                double st = rs + fs;
+                if (is_lev) st = st + L.lev[l];
+                gb[G_STONEW] = (double)R(st);
+                gb[G_STOPRE2] = st;
+                ro = qrl; fo = qfl;
+                if (is_dam) { L.ro[e] = qrl; L.fo[e] = qfl; }
+                if (own) {
+                    L.a_riv[l] = L.a_riv[l] + qrl * rdt;
+                    L.a_fld[l] = L.a_fld[l] + qfl * rdt;
+                    if (!kOutSum) L.a_out[l] = L.a_out[l] + outflw * rdt;
+                    L.m_out[l] = vmax(L.m_out[l], vabs(outflw));
+                    if (is_dam) L.a_inf[e] = L.a_inf[e] + R(L.daminf[e] * dt);
+                    if (last) {
+                        S.rivinf[g] = rivinf; S.fldinf[g] = fldinf; S.pthout[g] = 0.0;
+                        S.outflw[g] = outflw;
+                    }
+                }
+            }
+            if (A.budget) {
+                double ga[NA];
+#pragma unroll
+                for (int k = 0; k < NA; ++k) ga[k] = own ? gb[k] : 0.0;      // the owner counts a cell
+                wave_sum_comp<NA>(ga, L.sum, L.sum + NGLB * NW, NW, l >> 6);
+            }
+        }
+        // ---- stage inversion, maxima
+        {
+            double gs[NB];
+#pragma unroll
+            for (int k = 0; k < NB; ++k) gs[k] = 0.0;
+            if (upd) {
+                Stage o;
+                const Geom geo{(double)f_rivlen, (double)f_rivwth, (double)f_grarea, (double)f_rivhgt};
+                using Lds = BlockLds<R, T, LEV, DAM>;
+                const BlockHgt<Lds::NL, T> hgt{&L.hgt[0][l], M.fldhgt + g, M.n};
+                if (is_lev) stage_levee(M, hgt, geo, load_lev_row(M, L.lrow[l]), rs, fs, L.lev[l], o);
+                else stage_def<!LEV>(M, hgt, geo, rs, fs, o);
+                rs = o.rivsto;
+                fs = o.fldsto;
+                double stg = rs + fs;
+                if (is_lev) L.lev[l] = o.levsto;
+                if (LEV) stg = stg + o.levsto;
+                const R rivdph = R(o.rivdph), storge = R(stg);
+                L.dphp[l] = L.dph[l];
+                L.dph[l] = rivdph;
+                L.fdph[l] = R(o.flddph);
+                L.ffrc[l] = R(o.fldfrc);
+                if (own) {
+                    gs[0] = stg;
+                    gs[G_RIVSTO - G_STONEW2] = rs;
+                    gs[G_FLDSTO - G_STONEW2] = fs;
+                    gs[G_FLDARE - G_STONEW2] = o.fldare;
+                    if (LEV) gs[NB - 1] = o.levsto;
+                    L.m_dph[l] = vmax(L.m_dph[l], rivdph);
+                    L.m_sto[l] = vmax(L.m_sto[l], storge);
+                    if (last) {
+                        S.fldare[g] = R(o.fldare);
+                        S.sfcelv[g] = R((double)f_elevtn - (double)f_rivhgt) + rivdph;
+                        S.storge[g] = storge;
+                        if (is_lev) S.levdph[g] = R(o.levdph);
+                    }
+                }
+            }
+            if (A.budget) wave_sum_comp<NB>(gs, L.sum, L.sum + NGLB * NW, NW, l >> 6, G_STONEW2);
+        }
+        __syncthreads();
+        // the wavefront sums stay until the next update, two barriers from here
+        if (A.budget && l < NGLB) {
+            const int k = l == G_STOPRE2 && !kOutSum ? (int)G_STONEW : l;
+            double hi = 0.0, lo = 0.0;
+            if (LEV || k != G_LEVSTO) comp_total(L.sum, L.sum + NGLB * NW, NW, k, hi, lo);
+            double* part = S.partials + ((size_t)it * P.nblk + b) * NPART;
+            part[l] = hi;
+            part[NGLB + l] = lo;
+        }
+    }
+    if (g < 0 || (w1 >> TOPO_CODE) != 0) return;
+    const BlockArgs<R>& a = block_args<R>();
+    const DevState<R>& S = a.S;
+    const BlockState<R>& O = a.O;
+    const R rdt = R(dt);
+    O.rivsto[g] = rs; O.fldsto[g] = fs;
+    O.rivout[g] = ro; O.fldout[g] = fo;
+    O.rivdph[g] = L.dph[l]; O.rivdph_pre[g] = L.dphp[l];
+    O.fldsto_pre[g] = L.fpre[l]; O.flddph[g] = L.fdph[l]; O.fldfrc[g] = L.ffrc[l];
+    if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) O.levsto[g] = L.lev[l];
+    const bool is_dam = DAM && (w0 & (BLK_DAM << TOPO_FLAGS));
+    const int e = slot_of_dam(l, T);
+    if (is_dam) { O.damsto[g] = L.dam[e]; S.daminf[g] = L.daminf[e]; }
+    R a4 = is_dam ? L.a_inf[e] : zero;                                     // daminf_sparse: zero elsewhere
+    S.outflw_max[g] = L.m_out[l]; S.rivdph_max[g] = L.m_dph[l]; S.storge_max[g] = L.m_sto[l];
+    R a1 = L.a_riv[l], a2 = L.a_fld[l], av = L.a_vel[l], a3 = kOutSum ? zero : L.a_out[l];
+    if (it0 + nsub == nt) {                                               // GETAVE, diag:179-186
+        const R nadd = R(a.I.nadd);
+        a1 = a1 / nadd; a2 = a2 / nadd; av = av / nadd;
+        a3 = kOutSum ? a1 + a2 : a3 / nadd;
+        const R runoff = S.runoff[g];
+        R a5 = zero;
+        for (int k = 0; k < nt; ++k) a5 = a5 + runoff * rdt;
+        S.runoff_avg[g] = a5 / nadd;
+        S.pthout_avg[g] = zero;
+        a4 = a4 / nadd;
+        S.outflw_avg[g] = a3;
+    } else if (!kOutSum) {
+        S.outflw_avg[g] = a3;
+    }
+    if (is_dam || (DAM && it0 + nsub == nt)) S.daminf_avg[g] = a4;
+    S.rivout_avg[g] = a1; S.fldout_avg[g] = a2; S.rivvel_avg[g] = av;
+}
+
+template <class R, int T>
+static hipError_t launch_block_t(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
+                                 const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st) {
+    const dim3 g(P.nblk), t(T);
+    const BlockArgs<R> a{M, S, O, P, A, I, it0, nsub, vel0};
+    if (A.llevee && A.ldamout) hipLaunchKernelGGL((k_block<R, T, true, true>), g, t, 0, st, a);
+    else if (A.llevee) hipLaunchKernelGGL((k_block<R, T, true, false>), g, t, 0, st, a);
+    else if (A.ldamout) hipLaunchKernelGGL((k_block<R, T, false, true>), g, t, 0, st, a);
+    else hipLaunchKernelGGL((k_block<R, T, false, false>), g, t, 0, st, a);
+    return hipGetLastError();
+}
+
+template <class R>
+hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
+                        const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st) {
+    switch (P.T) {
+        case 256: return launch_block_t<R, 256>(M, S, O, P, A, I, it0, nsub, vel0, st);
+        case 512: return launch_block_t<R, 512>(M, S, O, P, A, I, it0, nsub, vel0, st);
+        default: return launch_block_t<R, 1024>(M, S, O, P, A, I, it0, nsub, vel0, st);
+    }
+}
+template hipError_t launch_block<double>(const DevMap&, const DevState<double>&, const BlockState<double>&,
+                                         const BlockTab&, const StepArgs&, const InstStep&, int, int, const double*,
+                                         hipStream_t);
+template hipError_t launch_block<float>(const DevMap&, const DevState<float>&, const BlockState<float>&,
+                                        const BlockTab&, const StepArgs&, const InstStep&, int, int, const float*,
+                                        hipStream_t);
+
+}  // namespace cmf

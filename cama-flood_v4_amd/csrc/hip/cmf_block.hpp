@@ -1,0 +1,69 @@
+// cmf_block.hpp -- several substeps of a single model in one launch (cmf_block.hip):
+// the partition of the river network into blocks and its launch.
+#pragma once
+#include "cmf_device.hpp"
+#include <vector>
+
+namespace cmf {
+
+// Partition of the network (host): nblk blocks of T local cells. A block owns
+// some cells (whole basins, and connected parts of basins larger than a block)
+// and holds beside them the cells its owned ones depend on over kmax substeps.
+struct BlockPlan {
+    int T = 0, kmax = 0, nblk = 0;
+    bool closed = false;                       // no block holds a cell of another: any number of substeps
+    std::vector<int32_t> cell;                 // [nblk*T] device cell of each local cell, -1 idle
+    std::vector<uint32_t> topo;                // [2][nblk*T], the fields below
+    std::vector<int32_t> upx_ptr;              // [nblk*T] start of the list in upx of cells with more than two
+    std::vector<uint16_t> upx;
+    std::vector<int32_t> ndam;                 // [nblk] dam cells | kinematic cells << 16
+};
+// False when the network cannot be cut into such blocks (a cell with too many
+// upstream cells, or whose surroundings alone overfill a block).
+// special: BLK_* flags of every cell (NULL: none).
+// dam cell (any), levee cell, reads its upstream cells' flows, dam cell on the kinematic wave
+enum : uint8_t { BLK_DAM = 1, BLK_LEV = 2, BLK_DAMUP = 4, BLK_KINE = 8 };
+bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
+                      const uint8_t* special, int T, int kmax, BlockPlan& out);
+
+// Order of the cells of a block: dam cells from 0, kinematic cells (above a dam)
+// from BLK_KINE_AT, so that the two rare flow rules are computed by different
+// wavefronts; levee cells take the lowest places left. Their extra state has LDS
+// slots for so many of each.
+constexpr int BLK_KINE_AT = 64;
+constexpr int blk_dams(int T) { return T / 32; }
+constexpr int blk_kines(int T) { return 3 * T / 32; }
+constexpr int blk_special(int T) { return 3 * T / 8; }
+
+// fields of the two topology words of a local cell (local indices < 1024)
+constexpr uint32_t TOPO_MOUTH = 0x7ff;         // word 0: downstream (11 bits), first upstream (10), flags (2)
+constexpr int TOPO_UP0 = 11, TOPO_FLAGS = 21;
+constexpr int TOPO_NUP = 10, TOPO_CODE = 18;   // word 1: second upstream (10 bits), upstream count (8), code (8)
+
+// device copy of a plan
+struct BlockTab {
+    int T, kmax, nblk, closed;
+    const int32_t* cell;
+    const uint32_t* topo;
+    const int32_t* upx_ptr;
+    const uint16_t* upx;
+    const int32_t* ndam;
+};
+
+// the arrays a launch hands to the next one: written by the owner of a cell while
+// other blocks may still read the previous values
+template <class R>
+struct BlockState {
+    double *rivsto, *fldsto, *levsto, *damsto;
+    R *rivout, *fldout, *rivdph, *rivdph_pre, *fldsto_pre, *flddph, *fldfrc;
+};
+
+// substeps it0 .. it0+nsub-1 of the outer step I, nsub <= kmax unless the plan is
+// closed. S carries the values at it0; O receives those after the last substep
+// (may alias S with a closed plan). vel0: D2RIVOUT of the first substep where it
+// differs from D2RIVOUT_PRE, or NULL. Budget sums go to S.partials[it][block][NPART].
+template <class R>
+hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
+                        const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st);
+
+}  // namespace cmf

@@ -2,6 +2,7 @@
 // upload and validation, and the outer-step driver that replaces
 // CMF_PHYSICS_ADVANCE / CMF_PHYSICS_FLDSTG (src/cmf_ctrl_physics_mod.F90).
 #include "cmf_hip.h"
+#include "cmf_block.hpp"
 #include "cmf_kernels.hpp"
 
 #include <chrono>
@@ -113,6 +114,11 @@ struct cmf_hip_ctx {
     size_t stage_cap = 0;             // bytes
     // host index of every device slot: cells (ns), path levels (npthlev*nsp), paths (nsp)
     std::vector<int64_t> hx_cell, hx_pthl, hx_pth;
+    // several substeps per launch (cmf_block.hip): the device copy of the partition
+    // (nblk = 0: none) and the second set of the arrays its launches hand on
+    BlockTab block{};
+    BlockState<double> alt64{};
+    BlockState<float> alt32{};
     // launch configuration
     cmf_tune tune{};
     int coop_max = 0;                 // co-resident blocks of the fused kernel at tune.bs_fused
@@ -671,8 +677,8 @@ void drop_graphs(cmf_hip_ctx* h) {
 }
 
 template <class R>
-int grow_partials(cmf_hip_ctx* h, DevState<R>& S, int nrun) {
-    const size_t need = (size_t)nrun * tiles_cells(h->M, upd_bs(h)) * NPART;
+int grow_partials(cmf_hip_ctx* h, DevState<R>& S, int nrun, int ntiles) {
+    const size_t need = (size_t)nrun * ntiles * NPART;
     if (need > h->partial_cap) {
         // k_update of a cached graph writes into S.partials: the old buffer is freed here
         drop_graphs(h);
@@ -761,6 +767,52 @@ int run_substeps_graph(cmf_hip_ctx* h, DevState<R>& S, int32_t ntmax) {
     return 0;
 }
 
+template <class R>
+BlockState<R>& alt_of(cmf_hip_ctx* h);
+template <>
+BlockState<double>& alt_of<double>(cmf_hip_ctx* h) { return h->alt64; }
+template <>
+BlockState<float>& alt_of<float>(cmf_hip_ctx* h) { return h->alt32; }
+
+// Whether an outer step of nt substeps runs as block launches: the handle has a
+// partition (a single model without bifurcation paths), the scheme is the default
+// one, DAMINF is zero outside the dam cells, and no other form of the substep is
+// asked for (graph replay, the persistent kernel, per-phase timing). Open
+// partitions need two launches at least (below).
+bool use_blocks(const cmf_hip_ctx* h, int32_t nt) {
+    return h->block.nblk > 0 && !h->lkine && !h->lslpmix && (!h->o.ldamout || h->daminf_sparse) && !h->tune.graph &&
+           !h->tune.fused && !h->timing && (h->block.closed || nt >= 2);
+}
+
+// NT substeps as block launches. A closed partition takes all of them in one
+// launch, in place. Otherwise the launches alternate between the state and its
+// second set of arrays, an even number of them, so that the state ends where it
+// began and no pointer moves.
+template <class R>
+int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t nt, bool vel_first) {
+    const StepArgs A = base_args(h);
+    const BlockTab& P = h->block;
+    const int nl = P.closed ? 1 : 2 * ((nt + 2 * P.kmax - 1) / (2 * P.kmax));
+    const BlockState<R> home{S.rivsto, S.fldsto, S.levsto, S.damsto, S.rivout, S.fldout, S.rivdph, S.rivdph_pre,
+                             S.fldsto_pre, S.flddph, S.fldfrc};
+    const BlockState<R>& alt = alt_of<R>(h);
+    int it0 = 0;
+    for (int j = 0; j < nl; ++j) {
+        const int it1 = (int)((long long)nt * (j + 1) / nl);
+        DevState<R> Sk = S;
+        if (j & 1) {
+            Sk.rivsto = alt.rivsto; Sk.fldsto = alt.fldsto; Sk.levsto = alt.levsto; Sk.damsto = alt.damsto;
+            Sk.rivout = alt.rivout; Sk.fldout = alt.fldout; Sk.rivdph = alt.rivdph; Sk.rivdph_pre = alt.rivdph_pre;
+            Sk.fldsto_pre = alt.fldsto_pre; Sk.flddph = alt.flddph; Sk.fldfrc = alt.fldfrc;
+        }
+        const R* vel0 = vel_first && j == 0 ? (const R*)h->vel_buf : nullptr;
+        HIPCHK(launch_block<R>(h->M, Sk, P.closed || (j & 1) ? home : alt, P, A, h->h_inst[0], it0, it1 - it0,
+                               vel0, h->stream));
+        it0 = it1;
+    }
+    return 0;
+}
+
 // NT and DT of every instance from the CFL bounds in h->h_cfl (CALC_ADPSTP,
 // physics:205-206), written to the host step table h->h_inst; returns the
 // largest substep count and whether an instance needs its RIVDPH pair swapped back
@@ -818,16 +870,20 @@ int advance_t(cmf_hip_ctx* h, double dt_def, int32_t nt_cap, int32_t* nt_out, do
     bool anyfix = false;
     TRY(plan_step(h, dt_def, nt_cap, &ntmax, &anyfix));
     HIPCHK(hipMemcpyAsync(h->d_inst, h->h_inst, (size_t)ni * sizeof(InstStep), hipMemcpyHostToDevice, h->stream));
-    if (A.budget) TRY(grow_partials<R>(h, S, ntmax));
+    const bool blocks = use_blocks(h, ntmax);
+    const int ntiles = blocks ? h->block.nblk : tiles_cells(h->M, upd_bs(h));
+    if (A.budget) TRY(grow_partials<R>(h, S, ntmax, ntiles));
     const bool vel_first = h->vel_pending;
-    if (h->tune.graph && !h->tune.fused && !h->timing && !vel_first) {
+    if (blocks) {
+        TRY(enqueue_blocks<R>(h, S, ntmax, vel_first));
+    } else if (h->tune.graph && !h->tune.fused && !h->timing && !vel_first) {
         TRY(run_substeps_graph<R>(h, S, ntmax));
     } else {
         TRY(enqueue_substeps<R>(h, S, ntmax, vel_first, &ne));
     }
     if (anyfix) launch_swapfix<R>(h->M, S, h->stream);
     if (A.budget)                                                    // CALC_WATBAL sums, all substeps
-        launch_budget(S.partials, tiles_cells(h->M, upd_bs(h)), ntmax, S.glb_hist, h->stream);
+        launch_budget(S.partials, ntiles, ntmax, S.glb_hist, h->stream);
     HIPCHK(hipGetLastError());
     h->vel_pending = false;
     h->fld_pending = false;
@@ -1091,6 +1147,79 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
     (void)hipFree(h->snapshot);
     h->snapshot = nullptr;
     return nrep;
+}
+
+// Block sizes and substeps per launch to try, in order. The chip holds 256 blocks of
+// 1024 cells (512 of 512 in the mixed form, 768), one round of them. What decides is
+// how many rounds a launch takes, the ring a block steps redundantly (it grows with
+// kmax and shrinks with T) and, with few cells, the time of one substep of a block,
+// which is latency: 5.3 us with one wavefront per SIMD (T = 256), 11 us with four.
+//  * whole basins only, T = 256: one launch for all substeps (15,001 cells at 1 degree,
+//    204 substeps: 1.36 ms; T = 512 1.77, 1024 2.54; three-phase kernels 3.4)
+//  * up to one round of T = 512: 60,005 cells with levees and dams, mixed, 1023
+//    substeps: 11.1 ms with kmax 6 (kmax 4 12.0; T = 256 13.5; T = 1024, all basins
+//    whole, 11.9; three-phase 23.4)
+//  * up to one round of T = 1024: 239,520 cells, FP64, 1275 substeps: 22.0 ms with
+//    kmax 4 (kmax 6, two rounds, 33.6; T = 512 28.0; three-phase 43.7)
+//  * many rounds, 1,500,120 cells with levees and dams, 680 substeps: FP64 T = 1024,
+//    kmax 5 89.6 ms (kmax 4 95.1; T = 512, kmax 3 95.6; three-phase 136.2); mixed T =
+//    512, kmax 3 70.7 ms (kmax 4 72.4; T = 1024, kmax 5 75.3; three-phase 96.0)
+struct BlockShape { int T, kmax; bool closed_only; };
+std::vector<BlockShape> block_shapes(int n, bool mixed) {
+    std::vector<BlockShape> v;
+    if (n <= 256 * 256) v.push_back({256, 2, true});
+    if (n <= 240 * 512) { v.push_back({512, 6, false}); v.push_back({512, 4, false}); }
+    if (mixed && n > 240 * 1024) v.push_back({512, 3, false});
+    if (n > 240 * 1024) v.push_back({1024, 5, false});
+    v.push_back({1024, 4, false});
+    v.push_back({1024, 2, false});
+    return v;
+}
+
+// partition of the network for block launches, its device copy and the second set
+// of the arrays the launches hand on
+template <class R>
+int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
+                 const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
+                 const std::vector<int32_t>& lev_of) {
+    const int n = h->d.nseqall;
+    std::vector<uint8_t> special;
+    if (h->o.ldamout || h->o.llevee) special.assign((size_t)n, 0);
+    for (int p = 0; p < n && h->o.ldamout; ++p)
+        special[(size_t)p] |= (uint8_t)((i1d[(size_t)p] > 0 ? BLK_DAM | BLK_DAMUP : 0) | (dam_of[(size_t)p] != -1 ? BLK_DAM : 0) |
+                                        (i1d[(size_t)p] == 10 ? BLK_KINE : 0));
+    for (int p = 0; p < n && h->o.llevee; ++p)
+        if (lev_of[(size_t)p] >= 0) special[(size_t)p] |= BLK_LEV;
+    BlockPlan bp;
+    bool ok = false;
+    for (const BlockShape& b : block_shapes(n, sizeof(R) == sizeof(float))) {
+        ok = build_block_plan(n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(),
+                              b.T, b.kmax, bp) && (bp.closed || !b.closed_only);
+        if (ok) break;
+    }
+    if (!ok) return 0;                                    // the three-phase kernels serve every network
+    BlockTab P{};
+    P.T = bp.T; P.kmax = bp.kmax; P.closed = bp.closed;
+    int32_t* p32 = nullptr;
+    uint32_t* pu = nullptr;
+    uint16_t* ph = nullptr;
+    TRY(put_raw(h, &p32, bp.cell.data(), bp.cell.size())); P.cell = p32;
+    TRY(put_raw(h, &pu, bp.topo.data(), bp.topo.size())); P.topo = pu;
+    TRY(put_raw(h, &p32, bp.upx_ptr.data(), bp.upx_ptr.size())); P.upx_ptr = p32;
+    TRY(put_raw(h, &ph, bp.upx.data(), bp.upx.size())); P.upx = ph;
+    TRY(put_raw(h, &p32, bp.ndam.data(), bp.ndam.size())); P.ndam = p32;
+    if (!bp.closed) {
+        BlockState<R>& B = alt_of<R>(h);
+        const size_t ns = (size_t)n;
+        TRY(dalloc(h, &B.rivsto, ns)); TRY(dalloc(h, &B.fldsto, ns));
+        TRY(dalloc(h, &B.levsto, h->o.llevee ? ns : 1)); TRY(dalloc(h, &B.damsto, h->o.ldamout ? ns : 1));
+        TRY(dalloc(h, &B.rivout, ns)); TRY(dalloc(h, &B.fldout, ns)); TRY(dalloc(h, &B.rivdph, ns));
+        TRY(dalloc(h, &B.rivdph_pre, ns)); TRY(dalloc(h, &B.fldsto_pre, ns)); TRY(dalloc(h, &B.flddph, ns));
+        TRY(dalloc(h, &B.fldfrc, ns));
+    }
+    P.nblk = bp.nblk;
+    h->block = P;
+    return 0;
 }
 
 }  // namespace
@@ -1363,10 +1492,11 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         TRY(put_raw(h, &pd, mp->pth_man, (size_t)nlv)); M.pth_man = pd;
     }
     // levee: compact table of the cells that carry a levee (levee:184-259)
+    std::vector<int32_t> lidx;
     if (h->o.llevee) {
         const double* L[7] = {mp->levhgt, mp->levfrc, mp->bashgt, mp->levdst, mp->levbassto, mp->levtopsto, mp->levfilsto};
         for (int k = 0; k < 7; ++k) if (!L[k]) return fail(CMF_EINVAL, "LLEVEE: levee tables missing");
-        std::vector<int32_t> lidx(n, -1);
+        lidx.assign((size_t)n, -1);
         std::vector<int32_t> cells;
         for (int p = 0; p < n; ++p) {                                   // device order
             const int i = P[(size_t)p];
@@ -1384,6 +1514,7 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         TRY(put_raw(h, &pd, tab.data(), tab.size())); M.lev_tab = pd;
     }
     // dams (damout:123-308)
+    std::vector<int32_t> i1d, doc;
     if (h->o.ldamout) {
         const int nd = h->d.ndam;
         M.ndam = nd;
@@ -1392,14 +1523,14 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
             !mp->dam_qf || (!h22 && (!mp->dam_adjvol || !mp->dam_qa)) ||
             (h22 && (!mp->dam_norvol || !mp->dam_r_volupa)))
             return fail(CMF_EINVAL, "LDAMOUT: dam tables missing (LDAMH22=%d)", (int)h22);
-        std::vector<int32_t> doc(n, -1);
+        doc.assign((size_t)n, -1);
         for (int d = 0; d < nd; ++d) {
             if (mp->damstat[d] == -9999) continue;
             const int s = mp->damseq[d] - 1;
             if (s < 0 || s >= n) return fail(CMF_EMAP, "DamSeq(%d)=%d outside NSEQALL", d + 1, mp->damseq[d]);
             doc[(size_t)IP[(size_t)s]] = d;
         }
-        std::vector<int32_t> i1d = to_dev(h, mp->i1dam, (size_t)n);
+        i1d = to_dev(h, mp->i1dam, (size_t)n);
         // the other cells whose DAMINF the dam module sets (I1DAM > 0, damout:444-465)
         for (int p = 0; p < n; ++p)
             if (i1d[(size_t)p] > 0 && doc[(size_t)p] == -1) doc[(size_t)p] = -2;
@@ -1426,6 +1557,9 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
             if (ddom[(size_t)p] < ddom[(size_t)p - 1]) return fail(CMF_EMAP, "domains are not contiguous in device order");
         TRY(put_raw(h, &h->d_dom_off, doff.data(), doff.size()));
     }
+    if (h->ninst == 1 && h->permuted && !h->o.lpthout)
+        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx)
+                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx));
     h->map_set = true;
     return 0;
 }
