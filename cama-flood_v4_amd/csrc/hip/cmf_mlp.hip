@@ -12,6 +12,9 @@
 //   backward: G_Y = bf16(dL/dY); dW_l = H_{l-1}^T G_l (FP32); db_l = sum G_l (FP32);
 //             G_{l-1} = bf16((G_l W_l^T) * [H_{l-1} > 0])
 // The CPU oracle restates the same quantisation points.
+//
+// Networks of 256 hidden units (and at most 32 inputs, 16 outputs: the surrogate's
+// own 24-256-256-256-2 among them) run as fused kernels, other sizes layer by layer.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -230,6 +233,405 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
     p[i] = p[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
 }
 
+// ---------------------------------------------------------------------------
+// Fused kernels for H = 256. Every layer but the weight gradients maps rows to rows,
+// so one workgroup takes a tile of RT rows through the whole network, forward and,
+// for a gradient, back again, with the activations in LDS: nothing but the inputs,
+// the outputs and what the weight gradients need touches HBM. The products are
+// formed transposed (features x rows): a wavefront owns 64 features, its weight
+// fragments come straight from L2 with 16-byte loads (two layouts of the weights are
+// kept, k contiguous for either direction), and a lane ends with four consecutive
+// features of a row, one 8-byte LDS store for the next layer's operand. Each output
+// is one accumulator over ascending k in steps of 32, as in k_gemm_bf16.
+constexpr int FH = 256, FKI = 32, FNO = 16;     // hidden units, padded inputs and outputs
+constexpr int LDX = FKI + 8, LDH = FH + 8;      // LDS rows, padded against bank conflicts
+
+struct FusedNet {
+    const uint16_t *wt[4];                      // W_l transposed [dout][din]: forward (rows >= dout and k >= din zero)
+    const uint16_t *w[4];                       // W_l [din][dout]: backward (w[3] padded to 32 columns)
+    const float* b[4];
+    int n_in, n_out;
+};
+struct FusedTrain {
+    const float* t;                             // targets
+    const int64_t* idx;                         // rows of x and t, or NULL
+    float w_over;
+    float* y;                                   // outputs [rows][n_out]
+    uint16_t *xt, *ht[3], *gt[4];               // transposed [feature][ld]: inputs, hidden values, gradients
+    int ld;
+};
+
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// acc[i][j] = A(16 features i) x B(16 rows j) over NK steps of 32 k. The weights of the
+// next D steps are in flight: all of a layer's for the small tiles, whose products
+// would otherwise wait for one L2 round trip each.
+template <int NJ, int NK>
+__device__ __forceinline__ void tile_product(const uint16_t* __restrict__ A, int lda, const uint16_t* Bs, int ldb,
+                                             f32x4 (&acc)[4][NJ]) {
+    constexpr int D = NK == 1 ? 1 : (NJ <= 2 ? 8 : (NJ == 4 ? 2 : 1));
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int lane = threadIdx.x & 63, fr = lane & 15, fk = (lane >> 4) * 8;
+    const uint16_t* a0 = A + (size_t)fr * lda + fk;
+    const uint16_t* b0 = Bs + fr * ldb + fk;
+    bf16x8 a[D][4];
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[d][i] = *reinterpret_cast<const bf16x8*>(a0 + (size_t)16 * i * lda + 32 * d);
+    if (D > 1) asm volatile("" ::: "memory");                       // the loads stay here, ahead of their uses
+#pragma unroll
+    for (int kb = 0; kb < NK; kb += D) {
+        bf16x8 an[D][4];
+        if (kb + D < NK)
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    an[d][i] = *reinterpret_cast<const bf16x8*>(a0 + (size_t)16 * i * lda + 32 * (kb + D + d));
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8*>(b0 + 16 * j * ldb + 32 * (kb + d));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i][j] = mfma(a[d][i], b, acc[i][j]);
+            }
+        if (kb + D < NK)
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) a[d][i] = an[d][i];
+    }
+}
+
+// Workgroup barrier for data in LDS only: the stores of the transposed activations
+// stay in flight across it (no other thread of the launch reads them)
+__device__ __forceinline__ void sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Measured (24-256-256-256-2): inference of 262144 rows 224 us, 321 TFLOP/s, bound by the
+// products and their LDS operands (layer kernels: 1.8 ms); a gradient's pass over 1024
+// rows 29 us and over 4099 rows 38 us, bound by the chain of seven layers on one
+// wavefront per SIMD (layer kernels, forward and backward with k_mlp_dw's part: 860 us
+// and 2.4 ms).
+template <int RT, bool TRAIN>
+__global__ __launch_bounds__(256) void k_mlp_fused(FusedNet N, FusedTrain G, const float* __restrict__ x, int rows,
+                                                   float* __restrict__ yout) {
+    constexpr int NJ = RT / 16, NM = (NJ * 16 + 31) / 32;
+    __shared__ __attribute__((aligned(16))) uint16_t Xs[RT * LDX];
+    __shared__ __attribute__((aligned(16))) uint16_t Hs[RT * LDH];
+    __shared__ __attribute__((aligned(16))) uint16_t Ys[TRAIN ? RT * LDX : 8];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r0 = blockIdx.x * RT, f0 = 64 * wave;
+    const int row_l = lane & 15, q4 = (lane >> 4) * 4;
+    // inputs: 8 threads a row, 4 columns each
+    for (int e = tid; e < RT * 8; e += 256) {
+        const int r = e >> 3, c0 = (e & 7) * 4, gr = r0 + r;
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        if (gr < rows) {
+            const float* src = x + (size_t)(TRAIN && G.idx ? G.idx[gr] : gr) * N.n_in + c0;
+            if ((N.n_in & 3) == 0) {
+                if (c0 < N.n_in) {
+                    const float4 u = *reinterpret_cast<const float4*>(src);
+                    v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+                }
+            } else {
+                for (int k = 0; k < 4; ++k) if (c0 + k < N.n_in) v[k] = src[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint16_t u = f2bf(v[k]);
+            Xs[r * LDX + c0 + k] = u;
+            if (TRAIN) {
+                if (c0 + k < N.n_in) G.xt[(size_t)(c0 + k) * G.ld + gr] = u;
+                Ys[r * LDX + c0 + k] = 0;
+            }
+        }
+    }
+    sync_lds();
+    f32x4 acc[4][NJ];
+    uint32_t mask[3][NM];
+    // forward, hidden layers
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        float4 bias[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[i] = *reinterpret_cast<const float4*>(N.b[l] + f0 + 16 * i + q4);
+        asm volatile("" ::: "memory");
+        if (l == 0) tile_product<NJ, 1>(N.wt[0] + (size_t)f0 * FKI, FKI, Xs, LDX, acc);
+        else tile_product<NJ, FH / 32>(N.wt[l] + (size_t)f0 * FH, FH, Hs, LDH, acc);
+        if (l > 0) sync_lds();                                // every wavefront has read the old values
+#pragma unroll
+        for (int m = 0; m < NM; ++m) mask[l][m] = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n0 = f0 + 16 * i + q4;
+            const float4 b = bias[i];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int r = 16 * j + row_l;
+                const float v[4] = {acc[i][j][0] + b.x, acc[i][j][1] + b.y, acc[i][j][2] + b.z, acc[i][j][3] + b.w};
+                uint16_t u[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    u[k] = f2bf(v[k] > 0.f ? v[k] : 0.f);
+                    if (TRAIN) {
+                        const int bit = (i * NJ + j) * 4 + k;
+                        if ((u[k] & 0x7fffu) != 0 && !(u[k] & 0x8000u)) mask[l][bit >> 5] |= 1u << (bit & 31);
+                        G.ht[l][(size_t)(n0 + k) * G.ld + r0 + r] = r0 + r < rows ? u[k] : (uint16_t)0;
+                    }
+                }
+                uint2 p;
+                p.x = (uint32_t)u[0] | ((uint32_t)u[1] << 16);
+                p.y = (uint32_t)u[2] | ((uint32_t)u[3] << 16);
+                *reinterpret_cast<uint2*>(&Hs[r * LDH + n0]) = p;
+            }
+        }
+        sync_lds();
+    }
+    // output layer: a wavefront takes every fourth tile of rows
+    for (int j = wave; j < NJ; j += 4) {
+        f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int fk = (lane >> 4) * 8;
+#pragma unroll
+        for (int k = 0; k < FH / 32; ++k)
+            o = mfma(*reinterpret_cast<const bf16x8*>(N.wt[3] + row_l * FH + 32 * k + fk),
+                     *reinterpret_cast<const bf16x8*>(&Hs[(16 * j + row_l) * LDH + 32 * k + fk]), o);
+        const int r = 16 * j + row_l, gr = r0 + r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int n = q4 + k;
+            if (n < N.n_out) {
+                const float yv = o[k] + N.b[3][n];
+                if (gr < rows) yout[(size_t)gr * N.n_out + n] = yv;
+                if (TRAIN) {
+                    uint16_t u = 0;
+                    if (gr < rows) {
+                        const float d = yv - G.t[(size_t)(G.idx ? G.idx[gr] : gr) * N.n_out + n];
+                        const float w = d > 0.f ? G.w_over : 1.f;
+                        u = f2bf((2.f * w) * d / (float)(rows * N.n_out));
+                    }
+                    Ys[r * LDX + n] = u;
+                    G.gt[3][(size_t)n * G.ld + gr] = u;
+                }
+            }
+        }
+    }
+    if (!TRAIN) return;
+    // backward: G_(l-1) = (W_l G_l) where H_(l-1) > 0
+    sync_lds();
+#pragma unroll
+    for (int l = 3; l > 0; --l) {
+        if (l == 3) tile_product<NJ, 1>(N.w[3] + (size_t)f0 * FKI, FKI, Ys, LDX, acc);
+        else tile_product<NJ, FH / 32>(N.w[l] + (size_t)f0 * FH, FH, Hs, LDH, acc);
+        sync_lds();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n0 = f0 + 16 * i + q4;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int r = 16 * j + row_l;
+                uint16_t u[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int bit = (i * NJ + j) * 4 + k;
+                    const bool on = (mask[l - 1][bit >> 5] >> (bit & 31)) & 1u;
+                    u[k] = on && r0 + r < rows ? f2bf(acc[i][j][k]) : (uint16_t)0;
+                    G.gt[l - 1][(size_t)(n0 + k) * G.ld + r0 + r] = u[k];
+                }
+                if (l > 1) {
+                    uint2 p;
+                    p.x = (uint32_t)u[0] | ((uint32_t)u[1] << 16);
+                    p.y = (uint32_t)u[2] | ((uint32_t)u[3] << 16);
+                    *reinterpret_cast<uint2*>(&Hs[r * LDH + n0]) = p;
+                }
+            }
+        }
+        sync_lds();
+    }
+}
+
+// Gradients of the weights and biases and the loss, one wavefront per block:
+//  * dW_l = H_(l-1)^T G_l, a 32 x 32 tile each; both operands are stored with the rows
+//    (the k of this product) contiguous, so fragments are 16-byte loads and need no
+//    LDS. Batches of more than DW_ROWS rows are split (blockIdx.y) and summed after.
+//  * db_l: chunk sums of COLSUM_CHUNK rows, then the chunk sums in chunk order
+//  * partial sums of the loss over 256 values
+// 9 us for 1024 rows, 26 us for 4099: bound by the serial sum over the rows on 144
+// wavefronts, which keeps the order of the sums; longer batches are split.
+constexpr int DW_ROWS = 8192;
+constexpr int DW_TILES = 8 + 64 + 64 + 8;
+__global__ __launch_bounds__(64) void k_mlp_dw(FusedNet N, FusedTrain G, int rows, int rows_per, float* __restrict__ gw,
+                                               size_t g_stride, float* __restrict__ g, const int* __restrict__ off /* w0 b0 w1 ... */,
+                                               float* __restrict__ part) {
+    const int lane = threadIdx.x, ndb = (3 * FH + N.n_out + 1) / 2;
+    if (blockIdx.x < DW_TILES) {
+        int t = blockIdx.x, l = 0;
+        if (t >= 136) { l = 3; t -= 136; }
+        else if (t >= 72) { l = 2; t -= 72; }
+        else if (t >= 8) { l = 1; t -= 8; }
+        const int nt = l == 3 ? 1 : 8;                              // tiles along the columns
+        const int m0 = 32 * (t / nt), n0 = 32 * (t % nt);
+        const int din = l == 0 ? N.n_in : FH, dout = l == 3 ? N.n_out : FH;
+        const uint16_t* A = l == 0 ? G.xt : G.ht[l - 1];
+        const uint16_t* B = G.gt[l];
+        const int k0 = blockIdx.y * rows_per;
+        const int k1 = k0 + rows_per < rows ? k0 + rows_per : (rows + 31) & ~31;
+        const int fr = lane & 15, fk = (lane >> 4) * 8;
+        const bool two = l != 3;                                    // 16 output columns at most
+        const uint16_t* a0 = A + (size_t)(m0 + fr) * G.ld + fk;
+        const uint16_t* b0 = B + (size_t)(n0 + fr) * G.ld + fk;
+        const size_t step = (size_t)16 * G.ld, step_b = two ? step : 0;
+        f32x4 acc[2][2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        constexpr int U = 8;                                        // steps in flight
+        bf16x8 a[U][2], b[U][2];
+        auto fetch = [&](int k, bf16x8 (&fa)[2], bf16x8 (&fb)[2]) {
+            const int kk = k < k1 ? k : k0;                         // past the end: loaded, not used
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                fa[i] = *reinterpret_cast<const bf16x8*>(a0 + i * step + kk);
+                fb[i] = *reinterpret_cast<const bf16x8*>(b0 + i * step_b + kk);
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < U; ++u) fetch(k0 + 32 * u, a[u], b[u]);
+        for (int k = k0; k < k1; k += 32 * U) {
+            bf16x8 an[U][2], bn[U][2];
+#pragma unroll
+            for (int u = 0; u < U; ++u) fetch(k + 32 * (U + u), an[u], bn[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + 32 * u < k1) {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) acc[i][j] = mfma(a[u][i], b[u][j], acc[i][j]);
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) { a[u][i] = an[u][i]; b[u][i] = bn[u][i]; }
+        }
+        float* C = gw + blockIdx.y * g_stride + off[2 * l];
+        const int rq = (lane >> 4) * 4;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int gm = m0 + 16 * i + rq + r, gn = n0 + 16 * j + fr;
+                    if (gm < din && gn < dout && (two || j == 0)) C[(size_t)gm * dout + gn] = acc[i][j][r];
+                }
+        return;
+    }
+    if (blockIdx.y != 0) return;
+    const int q = blockIdx.x - DW_TILES;
+    if (q < ndb) {                                                  // two features, 32 chunks at a time
+        const int f = 2 * q + (lane >> 5), c = lane & 31;
+        const int l = f < 3 * FH ? f / FH : 3, n = f - l * FH;
+        const bool on = l < 3 || n < N.n_out;
+        const uint16_t* src = G.gt[l] + (size_t)(on ? n : 0) * G.ld;
+        const int nchunk = (rows + COLSUM_CHUNK - 1) / COLSUM_CHUNK;
+        float total = 0.f;
+        for (int cb = 0; cb < nchunk; cb += 32) {
+            float s = 0.f;
+            const int ch = cb + c;
+            if (ch < nchunk) {
+                const int ra = ch * COLSUM_CHUNK, rb = ra + COLSUM_CHUNK < rows ? ra + COLSUM_CHUNK : rows;
+                int r = ra;
+                for (; r + 8 <= rb; r += 8) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(src + r);
+                    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        s += __uint_as_float(w[k] << 16);
+                        s += __uint_as_float(w[k] & 0xffff0000u);
+                    }
+                }
+                for (; r < rb; ++r) s += bf2f(src[r]);
+            }
+            const int last = nchunk - cb < 32 ? nchunk - cb : 32;
+            for (int k = 0; k < last; ++k) total += __shfl(s, (lane & 32) + k, 64);
+        }
+        if (c == 0 && on) g[off[2 * l + 1] + n] = total;
+        return;
+    }
+    // loss: the pairwise tree of k_mse over 256 values, four of them per lane
+    const int i0 = (q - ndb) * 256, ny = rows * N.n_out;
+    float e[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int i = i0 + 64 * k + lane;
+        e[k] = 0.f;
+        if (i < ny) {
+            const int r = i / N.n_out, n = i % N.n_out;
+            const float d = G.y[i] - G.t[(size_t)(G.idx ? G.idx[r] : r) * N.n_out + n];
+            const float w = d > 0.f ? G.w_over : 1.f;
+            e[k] = w * (d * d);
+        }
+    }
+    float s = (e[0] + e[2]) + (e[1] + e[3]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+    if (lane == 0) part[q - ndb] = s;
+}
+
+// the split weight gradients in order
+__global__ void k_sum_splits(const float* __restrict__ p, size_t stride, int ns, const int* __restrict__ off, int n_in,
+                             int n_out, float* __restrict__ g, long long np) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    for (int l = 0; l < 4; ++l)
+        if (i >= off[2 * l + 1] && i < off[2 * l + 1] + (l == 3 ? n_out : FH)) return;   // biases are not split
+    float s = 0.f;
+    for (int k = 0; k < ns; ++k) s += p[(size_t)k * stride + i];
+    g[i] = s;
+}
+
+// BF16 copies of the weights in the layouts of the fused kernels; with m1: after an
+// Adam step (bias correction c1, c2)
+__global__ void k_adam_fused(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
+                             float* __restrict__ m2, long long n, float lr, float b1, float b2, float eps, float c1,
+                             float c2, const int* __restrict__ off, int n_in, int n_out, uint16_t* __restrict__ wbf,
+                             uint16_t* __restrict__ wt, uint16_t* __restrict__ w3) {
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float v = p[i];
+    if (m1) {
+        const float gi = g[i];
+        const float a = b1 * m1[i] + (1.f - b1) * gi;
+        const float b = b2 * m2[i] + (1.f - b2) * gi * gi;
+        m1[i] = a;
+        m2[i] = b;
+        v = v - lr * (a / c1) / (sqrtf(b / c2) + eps);
+        p[i] = v;
+    }
+    const uint16_t u = f2bf(v);
+    wbf[i] = u;
+    const int l = i < off[2] ? 0 : (i < off[4] ? 1 : (i < off[6] ? 2 : 3));
+    const int e = (int)i - off[2 * l], dout = l == 3 ? n_out : FH, din = l == 0 ? n_in : FH;
+    if (e >= din * dout) return;                                     // a bias
+    const int k = e / dout, m = e % dout;
+    const int base = l == 0 ? 0 : FH * FKI + (l - 1) * FH * FH;
+    wt[base + m * (l == 0 ? FKI : FH) + k] = u;
+    if (l == 3) w3[k * FKI + m] = u;
+}
+
 inline unsigned nblk(long long n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
 
 }  // namespace
@@ -260,6 +662,20 @@ struct cmf_mlp {
     long long tn = 0;
     float* h_scratch = nullptr;            // pinned
     float w_over = 1.f;                    // loss weight of over-predictions
+    // fused kernels (256 hidden units)
+    bool fused = false;
+    int ld = 0;                            // row length of the transposed arrays
+    uint16_t *wt = nullptr, *w3 = nullptr; // weights transposed; W_4 padded to 32 columns
+    int* off = nullptr;                    // offsets of W and b in the packed parameters (device)
+    uint16_t *xt = nullptr, *ht[3] = {nullptr, nullptr, nullptr};
+    uint16_t* gt[4] = {nullptr, nullptr, nullptr, nullptr};
+    float* gsplit = nullptr;               // split weight gradients
+    int nsplit_cap = 0;
+    float* xd = nullptr;                   // FP32 inputs of a host call
+    float* lossbuf = nullptr;              // loss partial sums of every batch of a training call
+    size_t loss_cap = 0;
+    int64_t* order = nullptr;              // row order of a training call
+    size_t order_cap = 0;
 };
 
 namespace {
@@ -296,7 +712,109 @@ void forward(cmf_mlp* h, int rows) {
                        h->p + h->off_b[3], rows, h->n_out);
 }
 
+// device buffer of at least n values kept with the handle
+template <class T>
+int grow(cmf_mlp* h, T** p, size_t* cap, size_t n) {
+    if (n <= *cap) return 0;
+    if (*p) {
+        MCHK(hipStreamSynchronize(h->stream));
+        for (void*& q : h->allocs) if (q == (void*)*p) { (void)hipFree(q); q = nullptr; }
+        *p = nullptr;
+        *cap = 0;
+    }
+    MTRY(malloc_t(h, p, n));
+    *cap = n;
+    return 0;
+}
+
+int loss_parts(const cmf_mlp* h, int rows) { return (int)nblk((long long)rows * h->n_out); }
+
+FusedNet fused_net(const cmf_mlp* h) {
+    FusedNet N{};
+    const size_t o[4] = {0, FH * FKI, FH * FKI + FH * FH, FH * FKI + 2 * FH * FH};
+    for (int l = 0; l < 4; ++l) {
+        N.wt[l] = h->wt + o[l];
+        N.w[l] = l == 3 ? h->w3 : h->wbf + h->off_w[l];
+        N.b[l] = h->p + h->off_b[l];
+    }
+    N.n_in = h->n_in; N.n_out = h->n_out;
+    return N;
+}
+
+// Rows per workgroup: small batches need many workgroups more than large tiles
+// (1024 rows fill 64 of them with 16 rows); from 32768 rows on, 128-row tiles keep
+// the matrix cores busy and read the weights once per 128 rows (a gradient stops at
+// 64: its masks and accumulators would spill).
+template <bool TRAIN>
+void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, float* y) {
+    const FusedNet N = fused_net(h);
+    const int pad = TRAIN ? (rows + 31) & ~31 : rows;                // the weight gradients read whole 32-row steps
+    auto blocks = [&](int rt) { return dim3((pad + rt - 1) / rt); };
+    if (rows <= 4096)
+        hipLaunchKernelGGL((k_mlp_fused<16, TRAIN>), blocks(16), dim3(256), 0, h->stream, N, G, x, rows, y);
+    else if (rows <= 8192)
+        hipLaunchKernelGGL((k_mlp_fused<32, TRAIN>), blocks(32), dim3(256), 0, h->stream, N, G, x, rows, y);
+    else if (rows <= 32768)
+        hipLaunchKernelGGL((k_mlp_fused<64, TRAIN>), blocks(64), dim3(256), 0, h->stream, N, G, x, rows, y);
+    else
+        hipLaunchKernelGGL((k_mlp_fused<TRAIN ? 64 : 128, TRAIN>), blocks(TRAIN ? 64 : 128), dim3(256), 0, h->stream, N, G,
+                           x, rows, y);
+}
+
+int dw_splits(int rows) {
+    const int ns = (rows + DW_ROWS - 1) / DW_ROWS;
+    return ns < 64 ? ns : 64;
+}
+
+// forward and backward of a batch by the fused kernels; gradients into h->g, loss
+// partial sums into part. x, t: device arrays, rows picked by idx (NULL: in order)
+int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, int rows, float* part) {
+    if (!h->xt) {
+        // whole tiles, and an odd number of 256-byte pieces a row: with a power of two the
+        // same rows of all features would meet in one or two L2 channels
+        h->ld = (h->max_batch + 127) & ~127;
+        if (h->ld / 128 % 2 == 0) h->ld += 128;
+        const size_t ld = (size_t)h->ld;
+        MTRY(malloc_t(h, &h->xt, FKI * ld));
+        for (auto& q : h->ht) MTRY(malloc_t(h, &q, FH * ld));
+        for (int l = 0; l < 4; ++l) MTRY(malloc_t(h, &h->gt[l], (l == 3 ? FNO : FH) * ld));
+    }
+    FusedTrain G{};
+    G.t = t; G.idx = idx; G.w_over = h->w_over; G.y = h->y;
+    G.xt = h->xt; G.ld = h->ld;
+    for (int l = 0; l < 3; ++l) G.ht[l] = h->ht[l];
+    for (int l = 0; l < 4; ++l) G.gt[l] = h->gt[l];
+    const int ns = dw_splits(rows);
+    const int per = ((rows + ns - 1) / ns + 31) & ~31;
+    if (ns > 1 && ns > h->nsplit_cap) {
+        h->nsplit_cap = dw_splits(h->max_batch);
+        MTRY(malloc_t(h, &h->gsplit, (size_t)h->nsplit_cap * (size_t)h->np));
+    }
+    launch_fused<true>(h, G, x, rows, h->y);
+    const unsigned nb = DW_TILES + (unsigned)((3 * FH + h->n_out + 1) / 2) + (unsigned)loss_parts(h, rows);
+    float* dst = ns > 1 ? h->gsplit : h->g;
+    hipLaunchKernelGGL(k_mlp_dw, dim3(nb, ns), dim3(64), 0, h->stream, fused_net(h), G, rows, per, dst, (size_t)h->np,
+                       h->g, h->off, part);
+    if (ns > 1)
+        hipLaunchKernelGGL(k_sum_splits, dim3(nblk(h->np)), dim3(256), 0, h->stream, h->gsplit, (size_t)h->np, ns, h->off,
+                           h->n_in, h->n_out, h->g, h->np);
+    MCHK(hipGetLastError());
+    return 0;
+}
+
+double loss_of(const float* part, int n) {
+    double s = 0.0;
+    for (int b = 0; b < n; ++b) s += part[b];
+    return s;
+}
+
 void refresh_bf16(cmf_mlp* h) {
+    if (h->fused) {
+        hipLaunchKernelGGL(k_adam_fused, dim3(nblk(h->np)), dim3(256), 0, h->stream, h->p, (const float*)nullptr,
+                           (float*)nullptr, (float*)nullptr, h->np, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f, h->off, h->n_in, h->n_out,
+                           h->wbf, h->wt, h->w3);
+        return;
+    }
     hipLaunchKernelGGL(k_to_bf16, dim3(nblk(h->np)), dim3(256), 0, h->stream, h->p, h->wbf, h->np);
 }
 
@@ -365,15 +883,33 @@ int cmf_mlp_create(int32_t n_in, int32_t hidden, int32_t n_out, int32_t max_batc
         return mfail(CMF_MLP_EHIP, "hipStreamCreate failed");
     }
     const size_t B = (size_t)max_batch, H = (size_t)hidden, wide = (size_t)(hidden > n_out ? hidden : n_out);
-    if ((rc = malloc_t(h, &h->p, h->np)) || (rc = malloc_t(h, &h->g, h->np)) || (rc = malloc_t(h, &h->m1, h->np)) ||
-        (rc = malloc_t(h, &h->m2, h->np)) || (rc = malloc_t(h, &h->wbf, h->np)) ||
-        (rc = malloc_t(h, &h->xb, B * n_in)) || (rc = malloc_t(h, &h->hb[0], B * H)) ||
-        (rc = malloc_t(h, &h->hb[1], B * H)) || (rc = malloc_t(h, &h->hb[2], B * H)) ||
-        (rc = malloc_t(h, &h->z, B * wide)) || (rc = malloc_t(h, &h->y, B * n_out)) ||
-        (rc = malloc_t(h, &h->t, B * n_out)) || (rc = malloc_t(h, &h->gy, B * n_out)) ||
-        (rc = malloc_t(h, &h->gh[0], B * H)) || (rc = malloc_t(h, &h->gh[1], B * H)) ||
-        (rc = malloc_t(h, &h->part, (B * n_out + 255) / 256)) || (rc = malloc_t(h, &h->idx, B)) ||
-        (rc = malloc_t(h, &h->colpart, ((B + COLSUM_CHUNK - 1) / COLSUM_CHUNK) * wide))) {
+    h->fused = hidden == FH && n_in <= FKI && n_out <= FNO;
+    rc = malloc_t(h, &h->p, h->np);
+    if (!rc) rc = malloc_t(h, &h->g, h->np);
+    if (!rc) rc = malloc_t(h, &h->m1, h->np);
+    if (!rc) rc = malloc_t(h, &h->m2, h->np);
+    if (!rc) rc = malloc_t(h, &h->wbf, h->np);
+    if (!rc) rc = malloc_t(h, &h->y, B * n_out);
+    if (!rc) rc = malloc_t(h, &h->t, B * n_out);
+    if (!rc) rc = malloc_t(h, &h->part, (B * n_out + 255) / 256);
+    if (!rc && !h->fused) {                                         // batch buffers of the layer kernels
+        if ((rc = malloc_t(h, &h->xb, B * n_in)) || (rc = malloc_t(h, &h->hb[0], B * H)) ||
+            (rc = malloc_t(h, &h->hb[1], B * H)) || (rc = malloc_t(h, &h->hb[2], B * H)) ||
+            (rc = malloc_t(h, &h->z, B * wide)) || (rc = malloc_t(h, &h->gy, B * n_out)) ||
+            (rc = malloc_t(h, &h->gh[0], B * H)) || (rc = malloc_t(h, &h->gh[1], B * H)) ||
+            (rc = malloc_t(h, &h->idx, B)) ||
+            (rc = malloc_t(h, &h->colpart, ((B + COLSUM_CHUNK - 1) / COLSUM_CHUNK) * wide))) {}
+    }
+    if (!rc && h->fused) {                                          // weight layouts of the fused kernels
+        int o[8];
+        for (int l = 0; l < 4; ++l) { o[2 * l] = (int)h->off_w[l]; o[2 * l + 1] = (int)h->off_b[l]; }
+        rc = malloc_t(h, &h->wt, (size_t)FH * FKI + 2 * FH * FH + FNO * FH);
+        if (!rc) rc = malloc_t(h, &h->w3, (size_t)FH * FKI);
+        if (!rc) rc = malloc_t(h, &h->off, 8);
+        if (!rc && hipMemcpy(h->off, o, sizeof o, hipMemcpyHostToDevice) != hipSuccess)
+            rc = mfail(CMF_MLP_EHIP, "hipMemcpy failed");
+    }
+    if (rc) {
         std::string keep = m_err;
         cmf_mlp_destroy(h);
         m_err = keep;
@@ -390,7 +926,7 @@ int cmf_mlp_create(int32_t n_in, int32_t hidden, int32_t n_out, int32_t max_batc
 void cmf_mlp_destroy(cmf_mlp_handle h) {
     if (!h) return;
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    for (void* q : h->allocs) (void)hipFree(q);
+    for (void* q : h->allocs) if (q) (void)hipFree(q);
     if (h->h_scratch) (void)hipHostFree(h->h_scratch);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -425,39 +961,47 @@ int cmf_mlp_get_params(cmf_mlp_handle h, float* params, float* grads) {
 
 int cmf_mlp_forward(cmf_mlp_handle h, const float* x, int64_t n, float* y) {
     if (!h || !x || !y || n < 0) return mfail(CMF_MLP_EINVAL, "bad argument");
-    float* xd = nullptr;
-    MCHK(hipMalloc(&xd, (size_t)h->max_batch * h->n_in * sizeof(float)));
-    int rc = 0;
-    for (int64_t r0 = 0; r0 < n && rc == 0; r0 += h->max_batch) {
+    if (!h->xd) MTRY(malloc_t(h, &h->xd, (size_t)h->max_batch * h->n_in));
+    for (int64_t r0 = 0; r0 < n; r0 += h->max_batch) {
         const int rows = (int)((n - r0) < h->max_batch ? (n - r0) : h->max_batch);
-        hipError_t e = hipMemcpyAsync(xd, x + (size_t)r0 * h->n_in, (size_t)rows * h->n_in * sizeof(float),
-                                      hipMemcpyHostToDevice, h->stream);
-        if (e != hipSuccess) { rc = mfail(CMF_MLP_EHIP, "copy: %s", hipGetErrorString(e)); break; }
-        hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, xd, h->xb,
-                           (long long)rows * h->n_in);
-        forward(h, rows);
-        e = hipMemcpyAsync(y + (size_t)r0 * h->n_out, h->y, (size_t)rows * h->n_out * sizeof(float),
-                           hipMemcpyDeviceToHost, h->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-        if (e != hipSuccess) rc = mfail(CMF_MLP_EHIP, "forward: %s", hipGetErrorString(e));
+        MCHK(hipMemcpyAsync(h->xd, x + (size_t)r0 * h->n_in, (size_t)rows * h->n_in * sizeof(float),
+                            hipMemcpyHostToDevice, h->stream));
+        if (h->fused) {
+            launch_fused<false>(h, FusedTrain{}, h->xd, rows, h->y);
+        } else {
+            hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, h->xd, h->xb,
+                               (long long)rows * h->n_in);
+            forward(h, rows);
+        }
+        MCHK(hipGetLastError());
+        MCHK(hipMemcpyAsync(y + (size_t)r0 * h->n_out, h->y, (size_t)rows * h->n_out * sizeof(float),
+                            hipMemcpyDeviceToHost, h->stream));
+        MCHK(hipStreamSynchronize(h->stream));
     }
-    (void)hipFree(xd);
-    return rc;
+    return 0;
 }
 
 int cmf_mlp_grad(cmf_mlp_handle h, const float* x, const float* t, int32_t rows, float* loss) {
     if (!h || !x || !t || rows <= 0 || rows > h->max_batch) return mfail(CMF_MLP_EINVAL, "bad argument");
-    float* xd = nullptr;
-    MCHK(hipMalloc(&xd, (size_t)rows * h->n_in * sizeof(float)));
-    hipError_t e = hipMemcpyAsync(xd, x, (size_t)rows * h->n_in * sizeof(float), hipMemcpyHostToDevice, h->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(h->t, t, (size_t)rows * h->n_out * sizeof(float), hipMemcpyHostToDevice, h->stream);
-    if (e != hipSuccess) { (void)hipFree(xd); return mfail(CMF_MLP_EHIP, "copy: %s", hipGetErrorString(e)); }
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, xd, h->xb,
-                       (long long)rows * h->n_in);
-    const int rc = grad_batch(h, rows, loss);
-    (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(xd);
+    if (!h->xd) MTRY(malloc_t(h, &h->xd, (size_t)h->max_batch * h->n_in));
+    MCHK(hipMemcpyAsync(h->xd, x, (size_t)rows * h->n_in * sizeof(float), hipMemcpyHostToDevice, h->stream));
+    MCHK(hipMemcpyAsync(h->t, t, (size_t)rows * h->n_out * sizeof(float), hipMemcpyHostToDevice, h->stream));
+    int rc = 0;
+    if (h->fused) {
+        MTRY(fused_grad(h, h->xd, h->t, nullptr, rows, h->part));
+        if (loss) {
+            const int nb = loss_parts(h, rows);
+            std::vector<float> part((size_t)nb);
+            MCHK(hipMemcpyAsync(part.data(), h->part, (size_t)nb * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+            MCHK(hipStreamSynchronize(h->stream));
+            *loss = (float)(loss_of(part.data(), nb) / (rows * h->n_out));
+        }
+    } else {
+        hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, h->xd, h->xb,
+                           (long long)rows * h->n_in);
+        rc = grad_batch(h, rows, loss);
+    }
+    MCHK(hipStreamSynchronize(h->stream));
     return rc;
 }
 
@@ -488,6 +1032,30 @@ int cmf_mlp_train(cmf_mlp_handle h, const int64_t* order, int64_t n_order, int32
     double lsum = 0.0;
     int32_t step = step0;
     int64_t nb = 0;
+    if (h->fused) {
+        // the whole order and the loss of every batch stay on the device, so the batches
+        // follow each other without a word to the host: three launches each
+        const int np = loss_parts(h, batch);
+        const size_t nbatch = (size_t)(n_order / batch), need = nbatch * (size_t)np;
+        MTRY(grow(h, &h->order, &h->order_cap, (size_t)n_order));
+        MTRY(grow(h, &h->lossbuf, &h->loss_cap, need));
+        MCHK(hipMemcpyAsync(h->order, order, (size_t)n_order * sizeof(int64_t), hipMemcpyHostToDevice, h->stream));
+        for (int64_t r0 = 0; r0 + batch <= n_order; r0 += batch) {
+            MTRY(fused_grad(h, h->tx, h->tt, h->order + r0, batch, h->lossbuf + (size_t)nb * np));
+            ++step;
+            const float c1 = 1.f - powf(beta1, (float)step), c2 = 1.f - powf(beta2, (float)step);
+            hipLaunchKernelGGL(k_adam_fused, dim3(nblk(h->np)), dim3(256), 0, h->stream, h->p, h->g, h->m1, h->m2, h->np, lr,
+                               beta1, beta2, eps, c1, c2, h->off, h->n_in, h->n_out, h->wbf, h->wt, h->w3);
+            ++nb;
+        }
+        MCHK(hipGetLastError());
+        std::vector<float> part(need);
+        if (need) MCHK(hipMemcpyAsync(part.data(), h->lossbuf, need * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+        MCHK(hipStreamSynchronize(h->stream));
+        for (size_t k = 0; k < nbatch; ++k) lsum += (float)(loss_of(&part[k * (size_t)np], np) / (batch * h->n_out));
+        if (loss_out) *loss_out = nb ? (float)(lsum / nb) : 0.f;
+        return (int)nb;
+    }
     for (int64_t r0 = 0; r0 + batch <= n_order; r0 += batch) {
         MCHK(hipMemcpyAsync(h->idx, order + r0, (size_t)batch * sizeof(int64_t), hipMemcpyHostToDevice, h->stream));
         hipLaunchKernelGGL(k_gather_bf16, dim3(nblk((long long)batch * h->n_in)), dim3(256), 0, h->stream, h->tx,
