@@ -1,4 +1,4 @@
-// cmf_block.hip -- many substeps of a single model per launch.
+// cmf_block.hip -- many substeps of a model per launch.
 //
 // The three-phase kernels (cmf_kernels.hip) stream the whole state through HBM on
 // every substep and meet the grid between phases. River networks do not need
@@ -31,7 +31,7 @@ namespace cmf {
 // (a dam's inflow is the previous flow of its upstream cells). code = position of
 // the first set a cell is in: U_r <= 3r, R_r <= 3r+1, Q_r <= 3r+2.
 bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
-                      const uint8_t* special, int T, int kmax, BlockPlan& out) {
+                      const uint8_t* special, const int32_t* domain, int T, int kmax, BlockPlan& out) {
     out = BlockPlan();
     if (n <= 0 || T > 1024 || kmax < 1 || 3 * kmax > 200) return false;
     const int cap = std::max(T / 4, T - 48 * kmax);
@@ -77,7 +77,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     }
     // local cells (owned first) and codes of every piece; a piece whose
     // surroundings overfill a block is halved
-    struct Piece { int32_t beg, size, spec, dams, kines; };        // into loc / codes; special cells
+    struct Piece { int32_t beg, size, spec, dams, kines, dom; };   // into loc / codes; special cells
     std::vector<Piece> done;
     std::vector<int32_t> loc, mark((size_t)n, -1), cur;
     std::vector<uint8_t> codes, curc;
@@ -86,7 +86,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     const int max_spec = blk_special(T);
     const int max_dams = blk_dams(T), max_kines = blk_kines(T);
     auto piece_of = [&](const std::vector<int32_t>& c, size_t from, int count) {
-        Piece p{(int32_t)loc.size(), count, 0, 0, 0};
+        Piece p{(int32_t)loc.size(), count, 0, 0, 0, domain ? domain[c[from]] : 0};
         for (int j = 0; special && j < count; ++j) {
             const uint8_t f = special[(size_t)c[from + j]];
             p.spec += (f & (BLK_DAM | BLK_LEV)) != 0;
@@ -172,13 +172,14 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     std::vector<Piece> room;                                       // what is left in each
     {
         auto holds = [](const Piece& r, const Piece& p) {
-            return r.size >= p.size && r.spec >= p.spec && r.dams >= p.dams && r.kines >= p.kines;
+            return r.dom == p.dom && r.size >= p.size && r.spec >= p.spec && r.dams >= p.dams && r.kines >= p.kines;
         };
         auto put = [&](int b, size_t k) {
             if (b < 0) {
                 b = (int)bins.size();
                 bins.emplace_back();
-                room.push_back({0, T, max_spec, max_dams, max_kines});
+                room.push_back({0, T, max_spec, max_dams, max_kines, done[k].dom});
+                out.dom.push_back(done[k].dom);
             }
             const Piece& p = done[k];
             Piece& r = room[(size_t)b];
@@ -186,26 +187,37 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
             r.size -= p.size; r.spec -= p.spec; r.dams -= p.dams; r.kines -= p.kines;
             return b;
         };
+        // domain by domain (the pieces were cut in descending cell order)
+        std::vector<int32_t> ord(done.size());
+        for (size_t k = 0; k < ord.size(); ++k) ord[k] = (int32_t)k;
+        std::stable_sort(ord.begin(), ord.end(), [&](int32_t x, int32_t y) { return done[(size_t)x].dom < done[(size_t)y].dom; });
         std::vector<std::vector<int32_t>> by_size((size_t)T + 1), by_room((size_t)T + 1);
         const int small = T / 16;
-        for (size_t k = 0; k < done.size(); ++k)
-            if (done[k].size > small) by_size[(size_t)done[k].size].push_back((int32_t)k);
-        for (int s = T; s > small; --s)
-            for (int32_t k : by_size[(size_t)s]) {
-                int b = -1;
-                for (int r = s; r <= T && b < 0; ++r)
-                    if (!by_room[(size_t)r].empty() && holds(room[(size_t)by_room[(size_t)r].back()], done[(size_t)k])) {
-                        b = by_room[(size_t)r].back();
-                        by_room[(size_t)r].pop_back();
-                    }
-                b = put(b, (size_t)k);
-                by_room[(size_t)room[(size_t)b].size].push_back(b);
+        for (size_t o0 = 0, o1 = 0; o0 < ord.size(); o0 = o1) {
+            while (o1 < ord.size() && done[(size_t)ord[o1]].dom == done[(size_t)ord[o0]].dom) ++o1;
+            for (auto& v : by_size) v.clear();
+            for (auto& v : by_room) v.clear();
+            const size_t first = bins.size();
+            for (size_t o = o0; o < o1; ++o)
+                if (done[(size_t)ord[o]].size > small) by_size[(size_t)done[(size_t)ord[o]].size].push_back(ord[o]);
+            for (int s = T; s > small; --s)
+                for (int32_t k : by_size[(size_t)s]) {
+                    int b = -1;
+                    for (int r = s; r <= T && b < 0; ++r)
+                        if (!by_room[(size_t)r].empty() && holds(room[(size_t)by_room[(size_t)r].back()], done[(size_t)k])) {
+                            b = by_room[(size_t)r].back();
+                            by_room[(size_t)r].pop_back();
+                        }
+                    b = put(b, (size_t)k);
+                    by_room[(size_t)room[(size_t)b].size].push_back(b);
+                }
+            size_t b = first;
+            for (size_t o = o0; o < o1; ++o) {
+                const size_t k = (size_t)ord[o];
+                if (done[k].size > small) continue;
+                while (b < bins.size() && !holds(room[b], done[k])) ++b;
+                put(b < bins.size() ? (int)b : -1, k);
             }
-        size_t b = 0;
-        for (size_t k = 0; k < done.size(); ++k) {
-            if (done[k].size > small) continue;
-            while (b < bins.size() && !holds(room[b], done[k])) ++b;
-            put(b < bins.size() ? (int)b : -1, k);
         }
     }
     const int nb = (int)bins.size();
@@ -332,7 +344,7 @@ struct BlockArgs {
     BlockTab P;
     StepArgs A;
     InstStep I;
-    int it0, nsub;
+    int j;
     const R* vel0;
 };
 
@@ -348,16 +360,39 @@ __device__ __forceinline__ const BlockArgs<R>& block_args() {
     return *(const BlockArgs<R>*)p;
 }
 
-template <class R, int T, bool LEV, bool DAM>
+// Workgroup barrier for data in LDS only: loads and stores of global memory stay in
+// flight across it (a full barrier waits for them, the runoff of the update and the
+// budget sums among them).
+__device__ __forceinline__ void sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class R, int T, bool LEV, bool DAM, bool MB>
 __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block(BlockArgs<R> args_) {
     constexpr bool kOutSum = sizeof(R) == sizeof(float);
     constexpr int NW = T / 64;
     // budget terms formed before the stage inversion (STOPRE2 is STONEW in FP64) and after it
     constexpr int NA = kOutSum ? G_STOPRE2 + 1 : G_STOPRE2, NB = (LEV ? NGLB : G_LEVSTO) - G_STONEW2;
     __shared__ BlockLds<R, T, LEV, DAM> L;
-    int l = threadIdx.x;
-    const int b = blockIdx.x;
-    int g;
+    int l = threadIdx.x, b = blockIdx.x, m = 0;
+    int nt = args_.I.nt;
+    double dt = args_.I.dt, gdt = args_.I.gdt;
+    if (MB) {
+        // the members of a block of cells follow each other on one XCD (consecutive
+        // workgroups go round the eight), as they share the lines of its state
+        const int lgm = args_.M.lgm, r = b >> 3;
+        m = r & ((1 << lgm) - 1);
+        b = ((r >> lgm) << 3) + (b & 7);
+        if (b >= args_.P.nblk) return;
+        const InstStep& I = args_.S.inst[(args_.P.dom[b] << lgm) + m];
+        nt = I.nt; dt = I.dt; gdt = I.gdt;
+    }
+    const int nl = block_launches(nt, args_.P.kmax, args_.P.closed);
+    if (MB && args_.j >= nl) return;
+    const int it0 = (int)((long long)nt * args_.j / nl), nsub = (int)((long long)nt * (args_.j + 1) / nl) - it0;
+    int g, s0;                                                            // cell, state slot
     uint32_t w0, w1;
     const R zero = R(0);
     double rs = 0.0, fs = 0.0, zdn = 0.0;
@@ -370,14 +405,15 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         const BlockTab& P = a.P;
         const int pl = b * T + l;
         g = P.cell[pl];
+        s0 = MB ? (g << M.lgm) | m : g;
         w0 = P.topo[pl];
         w1 = P.topo[(size_t)P.nblk * T + pl];
         const bool mouth = (w0 & TOPO_MOUTH) == TOPO_MOUTH;
         if (g >= 0) {
-            rs = S.rivsto[g]; fs = S.fldsto[g];
-            ro = S.rivout[g]; fo = S.fldout[g];
-            L.dph[l] = S.rivdph[g]; L.dphp[l] = S.rivdph_pre[g];
-            L.fpre[l] = S.fldsto_pre[g]; L.fdph[l] = S.flddph[g]; L.ffrc[l] = S.fldfrc[g];
+            rs = S.rivsto[s0]; fs = S.fldsto[s0];
+            ro = S.rivout[s0]; fo = S.fldout[s0];
+            L.dph[l] = S.rivdph[s0]; L.dphp[l] = S.rivdph_pre[s0];
+            L.fpre[l] = S.fldsto_pre[s0]; L.fdph[l] = S.flddph[s0]; L.ffrc[l] = S.fldfrc[s0];
             f_rivlen = M.rivlen[g]; f_rivwth = M.rivwth[g]; f_grarea = M.grarea[g]; f_rivhgt = M.rivhgt[g];
             f_elevtn = M.elevtn[g]; f_nxtdst = M.nxtdst[g]; f_rivman = M.rivman[g];
             if (mouth) zdn = M.dwnelv[g];
@@ -385,7 +421,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
 #pragma unroll
             for (int k = 0; k < Lds::NL; ++k)
                 if (k < M.nlfp) L.hgt[k][l] = M.fldhgt[(size_t)k * M.n + g];
-            if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) { L.lev[l] = S.levsto[g]; L.lrow[l] = M.lev_idx[g]; }
+            if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) { L.lev[l] = S.levsto[s0]; L.lrow[l] = M.lev_idx[g]; }
             if (DAM && (w0 & (BLK_DAM << TOPO_FLAGS))) {
                 const int e = slot_of_dam(l, T);
                 const int c = M.i1dam[g], d = M.dam_of_cell[g];
@@ -400,35 +436,34 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 if (d >= 0 && M.damstat[d] != -9999) bits |= DAM_BALANCE;
                 L.dcode[e] = bits; L.drow[e] = d;
                 const bool mine = (w1 >> TOPO_CODE) == 0;
-                L.dam[e] = S.damsto[g]; L.daminf[e] = mine ? S.daminf[g] : 0.0;
-                L.a_inf[e] = mine && a.it0 > 0 ? S.daminf_avg[g] : zero;
+                L.dam[e] = S.damsto[s0]; L.daminf[e] = mine ? S.daminf[s0] : 0.0;
+                L.a_inf[e] = mine && it0 > 0 ? S.daminf_avg[s0] : zero;
                 L.ro[e] = ro; L.fo[e] = fo;
             }
         }
-        const bool cont = (w1 >> TOPO_CODE) == 0 && a.it0 > 0;
-        L.a_riv[l] = cont ? S.rivout_avg[g] : zero;
-        L.a_fld[l] = cont ? S.fldout_avg[g] : zero;
-        L.a_vel[l] = cont ? S.rivvel_avg[g] : zero;
-        if (!kOutSum) L.a_out[l] = cont ? S.outflw_avg[g] : zero;
-        L.m_out[l] = cont ? S.outflw_max[g] : zero;
-        L.m_dph[l] = cont ? S.rivdph_max[g] : zero;
-        L.m_sto[l] = cont ? S.storge_max[g] : zero;
+        const bool cont = (w1 >> TOPO_CODE) == 0 && it0 > 0;
+        L.a_riv[l] = cont ? S.rivout_avg[s0] : zero;
+        L.a_fld[l] = cont ? S.fldout_avg[s0] : zero;
+        L.a_vel[l] = cont ? S.rivvel_avg[s0] : zero;
+        if (!kOutSum) L.a_out[l] = cont ? S.outflw_avg[s0] : zero;
+        L.m_out[l] = cont ? S.outflw_max[s0] : zero;
+        L.m_dph[l] = cont ? S.rivdph_max[s0] : zero;
+        L.m_sto[l] = cont ? S.storge_max[s0] : zero;
         // the downstream cell's bed, through LDS
         L.q[l] = R(f_elevtn); L.f[l] = R(f_rivhgt);
-        __syncthreads();
+        sync_lds();
         if (!mouth) {
             const int nx = (int)(w0 & TOPO_MOUTH);
             zdn = (double)L.q[nx] - (double)L.f[nx];
         }
     }
-    const int nsub = args_.nsub, it0 = args_.it0, nt = args_.I.nt;
-    const double dt = args_.I.dt, gdt = args_.I.gdt;
-    __syncthreads();
+    sync_lds();
     for (int s = 0; s < nsub; ++s) {
         // what follows from these is formed anew in every substep: kept across the
         // loop it would take twice the registers there are
         asm volatile("" : "+v"(f_elevtn), "+v"(f_nxtdst), "+v"(f_rivman), "+v"(f_rivlen), "+v"(f_rivwth), "+v"(f_grarea),
                      "+v"(f_rivhgt), "+v"(w0), "+v"(w1), "+v"(g), "+v"(l));
+        if (MB) asm volatile("" : "+v"(s0));
         const BlockArgs<R>& a = block_args<R>();
         const DevMap& M = a.M;
         const DevState<R>& S = a.S;
@@ -451,7 +486,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             FlowIn<R> c;
             c.rivdph = L.dph[l]; c.rivdph_pre = L.dphp[l];
             c.qr_pre = ro;
-            c.qr_old = s == 0 && a.vel0 ? a.vel0[g] : c.qr_pre;
+            c.qr_old = it == 0 && a.vel0 ? a.vel0[s0] : c.qr_pre;
             c.fldsto = R(fs); c.flddph = L.fdph[l]; c.fldsto_pre = L.fpre[l];
             c.fldout_pre = fo;
             double stg = rs + fs;
@@ -470,7 +505,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 local_inertial<R>(c, sf, A.lfldout, A.pmanfld, A.pdstmth, dt, gdt, q_r, q_f);
             } else {
                 const BlockArgs<R>& ad = block_args<R>();
-                double inf = (double)ad.S.runoff[g];                      // damout:447-464
+                double inf = (double)ad.S.runoff[s0];                      // damout:447-464
                 const int nd = ad.P.ndam[b];
                 for (int k = 0; k < nup; ++k) {
                     const int u = k == 0 ? u0 : (k == 1 ? u1 : (int)ad.P.upx[ad.P.upx_ptr[b * T + l] + k - 2]);
@@ -487,13 +522,13 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             L.q[l] = q_r;
             L.f[l] = q_f;
             if (own) {
-                if (last) S.rivvel[g] = vel;
+                if (last) S.rivvel[s0] = vel;
                 L.a_vel[l] = L.a_vel[l] + vel * rdt;
             }
         }
-        __syncthreads();
+        sync_lds();
         const bool upd = code <= 3 * rem;
-        const R runoff = upd ? S.runoff[g] : zero;                        // in flight during the rate phase
+        const R runoff = upd ? S.runoff[s0] : zero;                        // in flight during the rate phase
         // ---- limiter rate (k_rate)
         if (code <= 3 * rem + 1) {
             double so = (double)vmax(L.q[l], zero) + (double)vmax(L.f[l], zero);
@@ -507,7 +542,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             const R dout = vmax(R(so), R(1.e-10));
             L.rate[l] = vmin(R(rs + fs) / dout, R(1));
         }
-        __syncthreads();
+        sync_lds();
         // ---- limit, inflow, dam balance, storages (k_update)
         {
             double gb[NGLB];
@@ -532,7 +567,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 L.fpre[l] = R(fs);
                 const R outflw = qrl + qfl;
                 storage_next<R>(rs, fs, rivinf, fldinf, 0.0, qrl, qfl, dt, runoff, L.ffrc[l], A.lupsinf,
-                                A.lupsinf ? S.upsinf[g] : zero, gb);
+                                A.lupsinf ? S.upsinf[s0] : zero, gb);
                 double st = rs + fs;
                 if (is_lev) st = st + L.lev[l];
                 gb[G_STONEW] = (double)R(st);
@@ -546,12 +581,12 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                     L.m_out[l] = vmax(L.m_out[l], vabs(outflw));
                     if (is_dam) L.a_inf[e] = L.a_inf[e] + R(L.daminf[e] * dt);
                     if (last) {
-                        S.rivinf[g] = rivinf; S.fldinf[g] = fldinf; S.pthout[g] = 0.0;
-                        S.outflw[g] = outflw;
+                        S.rivinf[s0] = rivinf; S.fldinf[s0] = fldinf; S.pthout[s0] = 0.0;
+                        S.outflw[s0] = outflw;
                     }
                 }
             }
-            if (A.budget) {
+            if (!MB && A.budget) {
                 double ga[NA];
 #pragma unroll
                 for (int k = 0; k < NA; ++k) ga[k] = own ? gb[k] : 0.0;      // the owner counts a cell
@@ -589,18 +624,18 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                     L.m_dph[l] = vmax(L.m_dph[l], rivdph);
                     L.m_sto[l] = vmax(L.m_sto[l], storge);
                     if (last) {
-                        S.fldare[g] = R(o.fldare);
-                        S.sfcelv[g] = R((double)f_elevtn - (double)f_rivhgt) + rivdph;
-                        S.storge[g] = storge;
-                        if (is_lev) S.levdph[g] = R(o.levdph);
+                        S.fldare[s0] = R(o.fldare);
+                        S.sfcelv[s0] = R((double)f_elevtn - (double)f_rivhgt) + rivdph;
+                        S.storge[s0] = storge;
+                        if (is_lev) S.levdph[s0] = R(o.levdph);
                     }
                 }
             }
-            if (A.budget) wave_sum_comp<NB>(gs, L.sum, L.sum + NGLB * NW, NW, l >> 6, G_STONEW2);
+            if (!MB && A.budget) wave_sum_comp<NB>(gs, L.sum, L.sum + NGLB * NW, NW, l >> 6, G_STONEW2);
         }
-        __syncthreads();
+        sync_lds();
         // the wavefront sums stay until the next update, two barriers from here
-        if (A.budget && l < NGLB) {
+        if (!MB && A.budget && l < NGLB) {
             const int k = l == G_STOPRE2 && !kOutSum ? (int)G_STONEW : l;
             double hi = 0.0, lo = 0.0;
             if (LEV || k != G_LEVSTO) comp_total(L.sum, L.sum + NGLB * NW, NW, k, hi, lo);
@@ -614,61 +649,68 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
     const DevState<R>& S = a.S;
     const BlockState<R>& O = a.O;
     const R rdt = R(dt);
-    O.rivsto[g] = rs; O.fldsto[g] = fs;
-    O.rivout[g] = ro; O.fldout[g] = fo;
-    O.rivdph[g] = L.dph[l]; O.rivdph_pre[g] = L.dphp[l];
-    O.fldsto_pre[g] = L.fpre[l]; O.flddph[g] = L.fdph[l]; O.fldfrc[g] = L.ffrc[l];
-    if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) O.levsto[g] = L.lev[l];
+    O.rivsto[s0] = rs; O.fldsto[s0] = fs;
+    O.rivout[s0] = ro; O.fldout[s0] = fo;
+    O.rivdph[s0] = L.dph[l]; O.rivdph_pre[s0] = L.dphp[l];
+    O.fldsto_pre[s0] = L.fpre[l]; O.flddph[s0] = L.fdph[l]; O.fldfrc[s0] = L.ffrc[l];
+    if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) O.levsto[s0] = L.lev[l];
     const bool is_dam = DAM && (w0 & (BLK_DAM << TOPO_FLAGS));
     const int e = slot_of_dam(l, T);
-    if (is_dam) { O.damsto[g] = L.dam[e]; S.daminf[g] = L.daminf[e]; }
+    if (is_dam) { O.damsto[s0] = L.dam[e]; S.daminf[s0] = L.daminf[e]; }
     R a4 = is_dam ? L.a_inf[e] : zero;                                     // daminf_sparse: zero elsewhere
-    S.outflw_max[g] = L.m_out[l]; S.rivdph_max[g] = L.m_dph[l]; S.storge_max[g] = L.m_sto[l];
+    S.outflw_max[s0] = L.m_out[l]; S.rivdph_max[s0] = L.m_dph[l]; S.storge_max[s0] = L.m_sto[l];
     R a1 = L.a_riv[l], a2 = L.a_fld[l], av = L.a_vel[l], a3 = kOutSum ? zero : L.a_out[l];
     if (it0 + nsub == nt) {                                               // GETAVE, diag:179-186
-        const R nadd = R(a.I.nadd);
+        const R nadd = R(MB ? S.inst[(a.P.dom[b] << a.M.lgm) + m].nadd : a.I.nadd);
         a1 = a1 / nadd; a2 = a2 / nadd; av = av / nadd;
         a3 = kOutSum ? a1 + a2 : a3 / nadd;
-        const R runoff = S.runoff[g];
+        const R runoff = S.runoff[s0];
         R a5 = zero;
         for (int k = 0; k < nt; ++k) a5 = a5 + runoff * rdt;
-        S.runoff_avg[g] = a5 / nadd;
-        S.pthout_avg[g] = zero;
+        S.runoff_avg[s0] = a5 / nadd;
+        S.pthout_avg[s0] = zero;
         a4 = a4 / nadd;
-        S.outflw_avg[g] = a3;
+        S.outflw_avg[s0] = a3;
     } else if (!kOutSum) {
-        S.outflw_avg[g] = a3;
+        S.outflw_avg[s0] = a3;
     }
-    if (is_dam || (DAM && it0 + nsub == nt)) S.daminf_avg[g] = a4;
-    S.rivout_avg[g] = a1; S.fldout_avg[g] = a2; S.rivvel_avg[g] = av;
+    if (is_dam || (DAM && it0 + nsub == nt)) S.daminf_avg[s0] = a4;
+    S.rivout_avg[s0] = a1; S.fldout_avg[s0] = a2; S.rivvel_avg[s0] = av;
 }
 
-template <class R, int T>
+template <class R, int T, bool MB>
 static hipError_t launch_block_t(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
-                                 const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st) {
-    const dim3 g(P.nblk), t(T);
-    const BlockArgs<R> a{M, S, O, P, A, I, it0, nsub, vel0};
-    if (A.llevee && A.ldamout) hipLaunchKernelGGL((k_block<R, T, true, true>), g, t, 0, st, a);
-    else if (A.llevee) hipLaunchKernelGGL((k_block<R, T, true, false>), g, t, 0, st, a);
-    else if (A.ldamout) hipLaunchKernelGGL((k_block<R, T, false, true>), g, t, 0, st, a);
-    else hipLaunchKernelGGL((k_block<R, T, false, false>), g, t, 0, st, a);
+                                 const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
+    const dim3 g(MB ? ((P.nblk + 7) / 8 * 8) << M.lgm : P.nblk), t(T);
+    const BlockArgs<R> a{M, S, O, P, A, I, j, vel0};
+    if (A.llevee && A.ldamout) hipLaunchKernelGGL((k_block<R, T, true, true, MB>), g, t, 0, st, a);
+    else if (A.llevee) hipLaunchKernelGGL((k_block<R, T, true, false, MB>), g, t, 0, st, a);
+    else if (A.ldamout) hipLaunchKernelGGL((k_block<R, T, false, true, MB>), g, t, 0, st, a);
+    else hipLaunchKernelGGL((k_block<R, T, false, false, MB>), g, t, 0, st, a);
     return hipGetLastError();
+}
+
+template <class R, bool MB>
+static hipError_t launch_block_mb(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
+                                  const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
+    switch (P.T) {
+        case 256: return launch_block_t<R, 256, MB>(M, S, O, P, A, I, j, vel0, st);
+        case 512: return launch_block_t<R, 512, MB>(M, S, O, P, A, I, j, vel0, st);
+        default: return launch_block_t<R, 1024, MB>(M, S, O, P, A, I, j, vel0, st);
+    }
 }
 
 template <class R>
 hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
-                        const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st) {
-    switch (P.T) {
-        case 256: return launch_block_t<R, 256>(M, S, O, P, A, I, it0, nsub, vel0, st);
-        case 512: return launch_block_t<R, 512>(M, S, O, P, A, I, it0, nsub, vel0, st);
-        default: return launch_block_t<R, 1024>(M, S, O, P, A, I, it0, nsub, vel0, st);
-    }
+                        const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
+    if (M.nmem > 1 || M.cell_dom) return launch_block_mb<R, true>(M, S, O, P, A, I, j, vel0, st);
+    return launch_block_mb<R, false>(M, S, O, P, A, I, j, vel0, st);
 }
 template hipError_t launch_block<double>(const DevMap&, const DevState<double>&, const BlockState<double>&,
-                                         const BlockTab&, const StepArgs&, const InstStep&, int, int, const double*,
+                                         const BlockTab&, const StepArgs&, const InstStep&, int, const double*,
                                          hipStream_t);
 template hipError_t launch_block<float>(const DevMap&, const DevState<float>&, const BlockState<float>&,
-                                        const BlockTab&, const StepArgs&, const InstStep&, int, int, const float*,
+                                        const BlockTab&, const StepArgs&, const InstStep&, int, const float*,
                                         hipStream_t);
 
 }  // namespace cmf

@@ -1,4 +1,4 @@
-// cmf_block.hpp -- several substeps of a single model in one launch (cmf_block.hip):
+// cmf_block.hpp -- several substeps of a model in one launch (cmf_block.hip):
 // the partition of the river network into blocks and its launch.
 #pragma once
 #include "cmf_device.hpp"
@@ -17,14 +17,16 @@ struct BlockPlan {
     std::vector<int32_t> upx_ptr;              // [nblk*T] start of the list in upx of cells with more than two
     std::vector<uint16_t> upx;
     std::vector<int32_t> ndam;                 // [nblk] dam cells | kinematic cells << 16
+    std::vector<int32_t> dom;                  // [nblk] domain of the block's cells
 };
 // False when the network cannot be cut into such blocks (a cell with too many
 // upstream cells, or whose surroundings alone overfill a block).
 // special: BLK_* flags of every cell (NULL: none).
 // dam cell (any), levee cell, reads its upstream cells' flows, dam cell on the kinematic wave
 enum : uint8_t { BLK_DAM = 1, BLK_LEV = 2, BLK_DAMUP = 4, BLK_KINE = 8 };
+// domain: of every cell, ascending (NULL: one); a block's cells share theirs.
 bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
-                      const uint8_t* special, int T, int kmax, BlockPlan& out);
+                      const uint8_t* special, const int32_t* domain, int T, int kmax, BlockPlan& out);
 
 // Order of the cells of a block: dam cells from 0, kinematic cells (above a dam)
 // from BLK_KINE_AT, so that the two rare flow rules are computed by different
@@ -48,6 +50,7 @@ struct BlockTab {
     const int32_t* upx_ptr;
     const uint16_t* upx;
     const int32_t* ndam;
+    const int32_t* dom;
 };
 
 // the arrays a launch hands to the next one: written by the owner of a cell while
@@ -58,12 +61,20 @@ struct BlockState {
     R *rivout, *fldout, *rivdph, *rivdph_pre, *fldsto_pre, *flddph, *fldfrc;
 };
 
-// substeps it0 .. it0+nsub-1 of the outer step I, nsub <= kmax unless the plan is
-// closed. S carries the values at it0; O receives those after the last substep
-// (may alias S with a closed plan). vel0: D2RIVOUT of the first substep where it
-// differs from D2RIVOUT_PRE, or NULL. Budget sums go to S.partials[it][block][NPART].
+// Launches of an instance of nt substeps: one with a closed plan, else an even number
+// of at most kmax substeps each, so that the state ends in the arrays it began in.
+__host__ __device__ inline int block_launches(int nt, int kmax, int closed) {
+    return closed ? 1 : 2 * ((nt + 2 * kmax - 1) / (2 * kmax));
+}
+
+// Launch j of an outer step: substeps nt*j/L .. nt*(j+1)/L of every instance with its
+// own nt (S.inst) and L = block_launches(nt); instances with L <= j are done. S carries
+// the values before it, O receives those after it (may alias S with a closed plan).
+// I: the step of a single model. vel0: D2RIVOUT of the first substep where it differs
+// from D2RIVOUT_PRE, or NULL. Budget sums of a single model go to
+// S.partials[it][block][NPART].
 template <class R>
 hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
-                        const StepArgs& A, const InstStep& I, int it0, int nsub, const R* vel0, hipStream_t st);
+                        const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st);
 
 }  // namespace cmf

@@ -774,11 +774,11 @@ BlockState<double>& alt_of<double>(cmf_hip_ctx* h) { return h->alt64; }
 template <>
 BlockState<float>& alt_of<float>(cmf_hip_ctx* h) { return h->alt32; }
 
-// Whether an outer step of nt substeps runs as block launches: the handle has a
-// partition (a single model without bifurcation paths), the scheme is the default
-// one, DAMINF is zero outside the dam cells, and no other form of the substep is
-// asked for (graph replay, the persistent kernel, per-phase timing). Open
-// partitions need two launches at least (below).
+// Whether an outer step of up to nt substeps runs as block launches: the handle has a
+// partition (no bifurcation paths; setup_blocks), the scheme is the default one,
+// DAMINF is zero outside the dam cells, and no other form of the substep is asked
+// for (graph replay, the persistent kernel, per-phase timing). One substep of an open
+// partition would take two launches that move the state for it.
 bool use_blocks(const cmf_hip_ctx* h, int32_t nt) {
     return h->block.nblk > 0 && !h->lkine && !h->lslpmix && (!h->o.ldamout || h->daminf_sparse) && !h->tune.graph &&
            !h->tune.fused && !h->timing && (h->block.closed || nt >= 2);
@@ -786,29 +786,25 @@ bool use_blocks(const cmf_hip_ctx* h, int32_t nt) {
 
 // NT substeps as block launches. A closed partition takes all of them in one
 // launch, in place. Otherwise the launches alternate between the state and its
-// second set of arrays, an even number of them, so that the state ends where it
-// began and no pointer moves.
+// second set of arrays, an even number of them for every instance, so that the state
+// ends where it began and no pointer moves.
 template <class R>
-int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t nt, bool vel_first) {
+int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t ntmax, bool vel_first) {
     const StepArgs A = base_args(h);
     const BlockTab& P = h->block;
-    const int nl = P.closed ? 1 : 2 * ((nt + 2 * P.kmax - 1) / (2 * P.kmax));
+    const int nl = block_launches(ntmax, P.kmax, P.closed);
     const BlockState<R> home{S.rivsto, S.fldsto, S.levsto, S.damsto, S.rivout, S.fldout, S.rivdph, S.rivdph_pre,
                              S.fldsto_pre, S.flddph, S.fldfrc};
     const BlockState<R>& alt = alt_of<R>(h);
-    int it0 = 0;
     for (int j = 0; j < nl; ++j) {
-        const int it1 = (int)((long long)nt * (j + 1) / nl);
         DevState<R> Sk = S;
         if (j & 1) {
             Sk.rivsto = alt.rivsto; Sk.fldsto = alt.fldsto; Sk.levsto = alt.levsto; Sk.damsto = alt.damsto;
             Sk.rivout = alt.rivout; Sk.fldout = alt.fldout; Sk.rivdph = alt.rivdph; Sk.rivdph_pre = alt.rivdph_pre;
             Sk.fldsto_pre = alt.fldsto_pre; Sk.flddph = alt.flddph; Sk.fldfrc = alt.fldfrc;
         }
-        const R* vel0 = vel_first && j == 0 ? (const R*)h->vel_buf : nullptr;
-        HIPCHK(launch_block<R>(h->M, Sk, P.closed || (j & 1) ? home : alt, P, A, h->h_inst[0], it0, it1 - it0,
-                               vel0, h->stream));
-        it0 = it1;
+        const R* vel0 = vel_first ? (const R*)h->vel_buf : nullptr;
+        HIPCHK(launch_block<R>(h->M, Sk, P.closed || (j & 1) ? home : alt, P, A, h->h_inst[0], j, vel0, h->stream));
     }
     return 0;
 }
@@ -881,7 +877,7 @@ int advance_t(cmf_hip_ctx* h, double dt_def, int32_t nt_cap, int32_t* nt_out, do
     } else {
         TRY(enqueue_substeps<R>(h, S, ntmax, vel_first, &ne));
     }
-    if (anyfix) launch_swapfix<R>(h->M, S, h->stream);
+    if (anyfix && !blocks) launch_swapfix<R>(h->M, S, h->stream);
     if (A.budget)                                                    // CALC_WATBAL sums, all substeps
         launch_budget(S.partials, ntiles, ntmax, S.glb_hist, h->stream);
     HIPCHK(hipGetLastError());
@@ -1149,30 +1145,42 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
     return nrep;
 }
 
-// Block sizes and substeps per launch to try, in order. The chip holds 256 blocks of
-// 1024 cells (512 of 512 in the mixed form, 768), one round of them. What decides is
-// how many rounds a launch takes, the ring a block steps redundantly (it grows with
-// kmax and shrinks with T) and, with few cells, the time of one substep of a block,
-// which is latency: 5.3 us with one wavefront per SIMD (T = 256), 11 us with four.
+// Block sizes and substeps per launch to try, in order, for ns cells (members counted)
+// in ninst instances. The chip holds 256 blocks of 1024 cells (512 of 512 in FP64, 768
+// in the mixed form), one round of them. What decides is how many rounds a launch
+// takes, the ring a block steps redundantly (it grows with kmax and shrinks with T)
+// and, with few cells, the time of one substep of a block, which is latency: 5.3 us
+// with one wavefront per SIMD (T = 256), 11 us with four.
 //  * whole basins only, T = 256: one launch for all substeps (15,001 cells at 1 degree,
 //    204 substeps: 1.36 ms; T = 512 1.77, 1024 2.54; three-phase kernels 3.4)
 //  * up to one round of T = 512: 60,005 cells with levees and dams, mixed, 1023
 //    substeps: 11.1 ms with kmax 6 (kmax 4 12.0; T = 256 13.5; T = 1024, all basins
-//    whole, 11.9; three-phase 23.4)
+//    whole, 11.9; three-phase 23.4); 4 members of them, FP64: 7.9 ms with kmax 6 (kmax
+//    4 9.2, kmax 3 10.0; T = 1024, kmax 6 8.5; three-phase 19.9)
 //  * up to one round of T = 1024: 239,520 cells, FP64, 1275 substeps: 22.0 ms with
 //    kmax 4 (kmax 6, two rounds, 33.6; T = 512 28.0; three-phase 43.7)
-//  * many rounds, 1,500,120 cells with levees and dams, 680 substeps: FP64 T = 1024,
-//    kmax 5 89.6 ms (kmax 4 95.1; T = 512, kmax 3 95.6; three-phase 136.2); mixed T =
-//    512, kmax 3 70.7 ms (kmax 4 72.4; T = 1024, kmax 5 75.3; three-phase 96.0)
-struct BlockShape { int T, kmax; bool closed_only; };
-std::vector<BlockShape> block_shapes(int n, bool mixed) {
+//  * many rounds, a single model, 1,500,120 cells with levees and dams, 680 substeps:
+//    FP64 T = 1024, kmax 5 89.6 ms (kmax 4 95.1; T = 512, kmax 3 95.6; three-phase
+//    136.2); mixed T = 512, kmax 3 70.7 ms (kmax 4 72.4; T = 1024, kmax 5 75.3;
+//    three-phase 96.0)
+//  * many rounds, ensembles: 16 domains of 4 members, 5,950,000 cells, mixed: T = 512,
+//    kmax 4 46.4 ms (kmax 3 48.6, kmax 6 50.4; T = 1024, kmax 4 58.4; three-phase
+//    71.6); FP64 65.4 (kmax 3 70.8; T = 1024 73.8; three-phase 107.1). 16 members,
+//    mixed: 44.2 (three-phase 54.8). With 64 the three-phase kernels have a line of
+//    memory per cell and are level (203.6; blocks 201.4): they keep it beyond 16.
+// max_blocks: a plan with more of them is refused.
+constexpr int BLOCK_MEMBERS = 16;
+struct BlockShape { int T, kmax; bool closed_only; int max_blocks; };
+std::vector<BlockShape> block_shapes(int64_t ns, int ninst, bool mixed) {
+    const int any = 0x7fffffff, round512 = mixed ? 768 : 512;
     std::vector<BlockShape> v;
-    if (n <= 256 * 256) v.push_back({256, 2, true});
-    if (n <= 240 * 512) { v.push_back({512, 6, false}); v.push_back({512, 4, false}); }
-    if (mixed && n > 240 * 1024) v.push_back({512, 3, false});
-    if (n > 240 * 1024) v.push_back({1024, 5, false});
-    v.push_back({1024, 4, false});
-    v.push_back({1024, 2, false});
+    if (ns <= 256 * 256) v.push_back({256, 2, true, any});
+    if (ns <= (ninst > 1 ? 480 : 240) * 512) v.push_back({512, 6, false, round512});   // one model this large does not fit
+    if (ns <= 240 * 512) v.push_back({512, 4, false, any});
+    if (ns > 240 * 1024 && (mixed || ninst > 1)) v.push_back({512, ninst > 1 ? 4 : 3, false, any});
+    if (ns > 240 * 1024) v.push_back({1024, 5, false, any});
+    v.push_back({1024, 4, false, any});
+    v.push_back({1024, 2, false, any});
     return v;
 }
 
@@ -1181,7 +1189,7 @@ std::vector<BlockShape> block_shapes(int n, bool mixed) {
 template <class R>
 int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
                  const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
-                 const std::vector<int32_t>& lev_of) {
+                 const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of) {
     const int n = h->d.nseqall;
     std::vector<uint8_t> special;
     if (h->o.ldamout || h->o.llevee) special.assign((size_t)n, 0);
@@ -1192,9 +1200,12 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
         if (lev_of[(size_t)p] >= 0) special[(size_t)p] |= BLK_LEV;
     BlockPlan bp;
     bool ok = false;
-    for (const BlockShape& b : block_shapes(n, sizeof(R) == sizeof(float))) {
+    for (const BlockShape& b : block_shapes(h->M.ns, h->ninst, sizeof(R) == sizeof(float))) {
         ok = build_block_plan(n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(),
-                              b.T, b.kmax, bp) && (bp.closed || !b.closed_only);
+                              dom_of.data(), b.T, b.kmax, bp) &&
+             (bp.closed || !b.closed_only) && (int64_t)bp.nblk * h->nmem <= b.max_blocks;
+        // blocks hold cells of one domain: many small domains would leave them empty
+        ok = ok && ((int64_t)bp.nblk * h->nmem <= 256 || (int64_t)bp.nblk * bp.T <= 2 * (int64_t)n);
         if (ok) break;
     }
     if (!ok) return 0;                                    // the three-phase kernels serve every network
@@ -1208,14 +1219,22 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
     TRY(put_raw(h, &p32, bp.upx_ptr.data(), bp.upx_ptr.size())); P.upx_ptr = p32;
     TRY(put_raw(h, &ph, bp.upx.data(), bp.upx.size())); P.upx = ph;
     TRY(put_raw(h, &p32, bp.ndam.data(), bp.ndam.size())); P.ndam = p32;
+    TRY(put_raw(h, &p32, bp.dom.data(), bp.dom.size())); P.dom = p32;
     if (!bp.closed) {
         BlockState<R>& B = alt_of<R>(h);
-        const size_t ns = (size_t)n;
-        TRY(dalloc(h, &B.rivsto, ns)); TRY(dalloc(h, &B.fldsto, ns));
-        TRY(dalloc(h, &B.levsto, h->o.llevee ? ns : 1)); TRY(dalloc(h, &B.damsto, h->o.ldamout ? ns : 1));
-        TRY(dalloc(h, &B.rivout, ns)); TRY(dalloc(h, &B.fldout, ns)); TRY(dalloc(h, &B.rivdph, ns));
-        TRY(dalloc(h, &B.rivdph_pre, ns)); TRY(dalloc(h, &B.fldsto_pre, ns)); TRY(dalloc(h, &B.flddph, ns));
-        TRY(dalloc(h, &B.fldfrc, ns));
+        const size_t ns = ((size_t)h->M.ns + 63) / 64 * 64, nlev = h->o.llevee ? ns : 0, ndm = h->o.ldamout ? ns : 0;
+        double* d = nullptr;                              // the doubles, then the fields in R, which is no larger
+        if (dalloc(h, &d, 2 * ns + nlev + ndm + 7 * ns * sizeof(R) / sizeof(double)) != 0) {
+            (void)hipGetLastError();                      // no memory for it: the three-phase kernels need none
+            return 0;
+        }
+        auto dbl = [&](double*& p, size_t k) { p = d; d += k; };
+        dbl(B.rivsto, ns); dbl(B.fldsto, ns); dbl(B.levsto, nlev); dbl(B.damsto, ndm);
+        R* r = reinterpret_cast<R*>(d);
+        for (R** p : {&B.rivout, &B.fldout, &B.rivdph, &B.rivdph_pre, &B.fldsto_pre, &B.flddph, &B.fldfrc}) {
+            *p = r;
+            r += ns;
+        }
     }
     P.nblk = bp.nblk;
     h->block = P;
@@ -1557,9 +1576,9 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
             if (ddom[(size_t)p] < ddom[(size_t)p - 1]) return fail(CMF_EMAP, "domains are not contiguous in device order");
         TRY(put_raw(h, &h->d_dom_off, doff.data(), doff.size()));
     }
-    if (h->ninst == 1 && h->permuted && !h->o.lpthout)
-        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx)
-                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx));
+    if (h->permuted && !h->o.lpthout && h->nmem <= BLOCK_MEMBERS)
+        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx, ddom)
+                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx, ddom));
     h->map_set = true;
     return 0;
 }

@@ -90,3 +90,47 @@ def test_upstream_inflow():
     m, st, ro = big_basins(9000, 0.0, 0)
     u = np.random.default_rng(2).uniform(0.0, 5.0, m.n)
     compare(m, st, ro, "fp64", [14], prep=lambda x: x.set_upsinf(u))
+
+
+# every instance its own number of substeps, some of them one; domains of blocks cut
+# from basins and of whole ones (1200 cells), a small and a large chip share
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("sizes, members, lev, dam", [
+    ([9000, 1200, 5000], 1, 0.2, 60), ([9000, 1200, 5000], 2, 0.0, 0), ([9000, 1200], 4, 0.3, 0),
+    ([1200, 700], 16, 0.0, 40), ([1500, 900], 2, 0.0, 0), ([60000, 40000], 4, 0.0, 0), ([6000], 32, 0.0, 0)])
+def test_ensemble(sizes, members, lev, dam, prec):
+    doms = []
+    for d, net in enumerate(synth.regional_networks(sizes, 11, land_frac=0.9)):
+        if lev:
+            synth.add_levees(net, lev, d, hmin=0.5, hmax=3.0, fmin=0.05, fmax=0.5)
+        if dam:
+            synth.add_dams(net, max(3, net.ncells // dam), d)
+        m = maps.build_map(net, maps.Options(llevee=lev > 0, ldamout=dam > 0, pdstmth=4.0e5))
+        st = maps.cold_start(m)
+        st["rivsto"] = m.rivstomax * np.random.default_rng(d).uniform(0.0, 0.4 + d, m.n)
+        if dam:
+            maps.init_dams(m, net, st)
+        doms.append((m, upload_keys(st), m.vec(synth.make_runoff(net, 1, d, mean_mm_day=20.0)[0])))
+    cm, dom_cells = maps.concat_maps([d[0] for d in doms])
+    init = {k: np.stack([np.concatenate([d[1][k] for d in doms])] * members) for k in doms[0][1]}
+    level = np.random.default_rng(4).uniform(0.02, 1.0, size=(members, 1))
+    init["rivsto"] = init["rivsto"] * level
+    ro = np.concatenate([d[2] for d in doms])
+    g = {k: CMFModel(cm, prec, members=members, dom_cells=dom_cells) for k in ("blocks", "phases")}
+    g["phases"].set_tune(graph=1)
+    fac = np.exp(np.random.default_rng(5).normal(0.0, 1.5, size=len(sizes) * members))
+    for x in g.values():
+        x.set_state(init)
+        x.set_runoff_scaled(ro, fac)
+    names = [k for k in STATE_KEYS + ["levsto", "levdph", "damsto", "daminf", "daminf_avg"] if g["blocks"]._available(k)]
+    spread = set()
+    for dt, cap in ((900.0, 0), (3600.0, 0), (86400.0, 9), (86400.0, 26)):
+        nt = {k: x.ensemble_advance(dt, nt_cap=cap)[0] for k, x in g.items()}
+        assert np.array_equal(nt["blocks"], nt["phases"])
+        spread |= set(np.minimum(nt["blocks"], cap or 10**6).tolist())
+        a, b = (x.get_state(names) for x in g.values())
+        for k in names:
+            assert np.array_equal(a[k], b[k]), (k, dt, cap, rel_err(a[k], b[k]))
+    print("substeps", sorted(spread), flush=True)
+    for x in g.values():
+        x.close()
