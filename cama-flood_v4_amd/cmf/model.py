@@ -162,7 +162,7 @@ class CMFModel:
             elif k in ("pthflwsum", "pthflwsum_avg"):
                 a = np.zeros(lead + (m.npth,))
             else:
-                a = np.zeros(lead + (m.n,))
+                a = np.empty(lead + (m.n,))           # every value of a cell field is written
             out[k] = a
             setattr(s, k, a.ctypes.data)
         self._check(self.lib.cmf_hip_get_state(self.h, C.byref(s)))
@@ -306,7 +306,7 @@ class CMFModel:
         lead = (self.members,) if self.members > 1 else ()
         out, s = {}, cmf_output()
         for k in names:
-            a = np.zeros(lead + ((m.npthlev, m.npth) if k == "pthflw" else (m.n,)))
+            a = np.zeros(lead + (m.npthlev, m.npth)) if k == "pthflw" else np.empty(lead + (m.n,))
             out[k] = a
             setattr(s, k, a.ctypes.data)
         self._check(self.lib.cmf_hip_get_output(self.h, C.byref(s)))

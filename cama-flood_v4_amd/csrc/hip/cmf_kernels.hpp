@@ -29,8 +29,22 @@ const void* substep_kernel(const DevMap& M, int bs);
 template <class R, class H>
 void launch_cells_from_host(R* dst, const H* src, const int32_t* perm, int n, int lgm, int ns, int shared,
                             hipStream_t st);
-template <class R, class H>
-void launch_cells_to_host(H* dst, const R* src, const int32_t* perm, int n, int lgm, int ns, hipStream_t st);
+// parts of up to FETCH_SEGS arrays, converted to double, into dst (pinned host memory)
+constexpr int FETCH_SEGS = 48;
+struct FetchSeg {
+    const void* src;          // device array of the members' values
+    uint32_t first, count;    // elements first .. first+count-1 of the host array
+    uint32_t at;              // its place in dst
+    uint32_t plane;           // values per member
+    int32_t cells, f32;       // in device cell order; floats
+};
+struct FetchArgs {
+    FetchSeg seg[FETCH_SEGS];
+    const int32_t* iperm;     // device position of a cell, NULL: identity
+    int lgm;
+    double* dst;
+};
+void launch_fetch(const FetchArgs& a, int nseg, hipStream_t st);
 // CMF_CALC_OUTPRE: RIVOUT_PRE, FLDOUT_PRE, RIVDPH_PRE, SFCELV (and D1PTHFLW_PRE with paths)
 template <class R>
 void launch_outpre(const DevMap& M, const DevState<R>& S, int lfldout, int lpthout, double pmanfld, double pdstmth,

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -26,6 +27,7 @@
 #include <vector>
 
 #include "cmf_mlp.h"
+#include "cmf_xfer.hpp"
 
 namespace {
 
@@ -672,6 +674,10 @@ struct cmf_mlp {
     float* gsplit = nullptr;               // split weight gradients
     int nsplit_cap = 0;
     float* xd = nullptr;                   // FP32 inputs of a host call
+    cmf::Pinned fwd_pin;                   // slots of the chunked inference: x and y; x on the device
+    float* fwd_x = nullptr;
+    int fwd_slots = 0;
+    hipStream_t fwd_stream[4] = {nullptr, nullptr, nullptr, nullptr};
     float* lossbuf = nullptr;              // loss partial sums of every batch of a training call
     size_t loss_cap = 0;
     int64_t* order = nullptr;              // row order of a training call
@@ -746,18 +752,18 @@ FusedNet fused_net(const cmf_mlp* h) {
 // the matrix cores busy and read the weights once per 128 rows (a gradient stops at
 // 64: its masks and accumulators would spill).
 template <bool TRAIN>
-void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, float* y) {
+void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, float* y, hipStream_t st) {
     const FusedNet N = fused_net(h);
     const int pad = TRAIN ? (rows + 31) & ~31 : rows;                // the weight gradients read whole 32-row steps
     auto blocks = [&](int rt) { return dim3((pad + rt - 1) / rt); };
     if (rows <= 4096)
-        hipLaunchKernelGGL((k_mlp_fused<16, TRAIN>), blocks(16), dim3(256), 0, h->stream, N, G, x, rows, y);
+        hipLaunchKernelGGL((k_mlp_fused<16, TRAIN>), blocks(16), dim3(256), 0, st, N, G, x, rows, y);
     else if (rows <= 8192)
-        hipLaunchKernelGGL((k_mlp_fused<32, TRAIN>), blocks(32), dim3(256), 0, h->stream, N, G, x, rows, y);
+        hipLaunchKernelGGL((k_mlp_fused<32, TRAIN>), blocks(32), dim3(256), 0, st, N, G, x, rows, y);
     else if (rows <= 32768)
-        hipLaunchKernelGGL((k_mlp_fused<64, TRAIN>), blocks(64), dim3(256), 0, h->stream, N, G, x, rows, y);
+        hipLaunchKernelGGL((k_mlp_fused<64, TRAIN>), blocks(64), dim3(256), 0, st, N, G, x, rows, y);
     else
-        hipLaunchKernelGGL((k_mlp_fused<TRAIN ? 64 : 128, TRAIN>), blocks(TRAIN ? 64 : 128), dim3(256), 0, h->stream, N, G,
+        hipLaunchKernelGGL((k_mlp_fused<TRAIN ? 64 : 128, TRAIN>), blocks(TRAIN ? 64 : 128), dim3(256), 0, st, N, G,
                            x, rows, y);
 }
 
@@ -790,7 +796,7 @@ int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, i
         h->nsplit_cap = dw_splits(h->max_batch);
         MTRY(malloc_t(h, &h->gsplit, (size_t)h->nsplit_cap * (size_t)h->np));
     }
-    launch_fused<true>(h, G, x, rows, h->y);
+    launch_fused<true>(h, G, x, rows, h->y, h->stream);
     const unsigned nb = DW_TILES + (unsigned)((3 * FH + h->n_out + 1) / 2) + (unsigned)loss_parts(h, rows);
     float* dst = ns > 1 ? h->gsplit : h->g;
     hipLaunchKernelGGL(k_mlp_dw, dim3(nb, ns), dim3(64), 0, h->stream, fused_net(h), G, rows, per, dst, (size_t)h->np,
@@ -799,6 +805,67 @@ int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, i
         hipLaunchKernelGGL(k_sum_splits, dim3(nblk(h->np)), dim3(256), 0, h->stream, h->gsplit, (size_t)h->np, ns, h->off,
                            h->n_in, h->n_out, h->g, h->np);
     MCHK(hipGetLastError());
+    return 0;
+}
+
+// Inference over any number of rows in chunks of FWD_ROWS: copied into a pinned slot
+// by one of several threads, sent, computed, written by the kernel into the slot and
+// copied out, chunks in flight on FWD_STREAMS streams. Bound by the host's copies and
+// PCIe (96 bytes a row): 1,500,120 rows 2.9 ms, 51 GB/s (one pageable copy, kernel and
+// copy back after another 7.1; chunks of 8,192 rows 3.9, of 4,096 6.2: the launches of
+// a chunk cost about 20 us).
+constexpr int FWD_ROWS = 16384, FWD_STREAMS = 4;
+int forward_fused(cmf_mlp* h, const float* x, int64_t n, float* y) {
+    const int64_t nc = (n + FWD_ROWS - 1) / FWD_ROWS;
+    if (nc > 0x7fffffff) return mfail(CMF_MLP_EINVAL, "too many rows");
+    const int slots = (int)std::min<int64_t>(nc, cmf::XFER_SLOTS);
+    const size_t nx = (size_t)FWD_ROWS * h->n_in, ny = (size_t)FWD_ROWS * h->n_out;
+    if (slots > h->fwd_slots) {
+        MCHK(h->fwd_pin.grow((size_t)slots * (nx + ny) * sizeof(float)));
+        float* q = nullptr;
+        MTRY(malloc_t(h, &q, (size_t)slots * nx));
+        if (h->fwd_x) {
+            (void)hipFree(h->fwd_x);
+            for (size_t k = 0; k < h->allocs.size(); ++k)
+                if (h->allocs[k] == (void*)h->fwd_x) { h->allocs.erase(h->allocs.begin() + (long)k); break; }
+        }
+        h->fwd_x = q;
+        h->fwd_slots = slots;
+    }
+    float* const pin = reinterpret_cast<float*>(h->fwd_pin.p);
+    auto rows_of = [n](int64_t c) { return (int)std::min<int64_t>(FWD_ROWS, n - c * FWD_ROWS); };
+    auto start_on = [&](int c, int slot, hipStream_t st) -> hipError_t {
+        const int rows = rows_of(c);
+        float *px = pin + (size_t)slot * (nx + ny), *dx = h->fwd_x + (size_t)slot * nx;
+        const size_t bytes = (size_t)rows * h->n_in * sizeof(float);
+        std::memcpy(px, x + (size_t)c * nx, bytes);
+        const hipError_t e = hipMemcpyAsync(dx, px, bytes, hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) return e;
+        launch_fused<false>(h, FusedTrain{}, dx, rows, px + nx, st);
+        return hipGetLastError();
+    };
+    auto finish = [&](int c, int slot) {
+        std::memcpy(y + (size_t)c * ny, pin + (size_t)slot * (nx + ny) + nx, (size_t)rows_of(c) * h->n_out * sizeof(float));
+    };
+    if (nc == 1) {
+        MCHK(start_on(0, 0, h->stream));
+        MCHK(hipStreamSynchronize(h->stream));
+        finish(0, 0);
+        return 0;
+    }
+    for (hipStream_t& st : h->fwd_stream)
+        if (!st) MCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    int device = 0;
+    MCHK(hipGetDevice(&device));
+    MCHK(hipStreamSynchronize(h->stream));                            // the weights
+    const hipError_t e = cmf::run_chunks((int)nc, device, [&](int c, int slot, hipEvent_t ev) -> hipError_t {
+        const hipStream_t st = h->fwd_stream[slot % FWD_STREAMS];
+        const hipError_t r = start_on(c, slot, st);
+        return r != hipSuccess ? r : hipEventRecord(ev, st);
+    }, finish);
+    if (e != hipSuccess)
+        for (hipStream_t st : h->fwd_stream) (void)hipStreamSynchronize(st);   // the slots are the next call's
+    MCHK(e);
     return 0;
 }
 
@@ -928,6 +995,9 @@ void cmf_mlp_destroy(cmf_mlp_handle h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (void* q : h->allocs) if (q) (void)hipFree(q);
     if (h->h_scratch) (void)hipHostFree(h->h_scratch);
+    h->fwd_pin.release();
+    for (hipStream_t st : h->fwd_stream)
+        if (st) (void)hipStreamDestroy(st);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
@@ -961,18 +1031,15 @@ int cmf_mlp_get_params(cmf_mlp_handle h, float* params, float* grads) {
 
 int cmf_mlp_forward(cmf_mlp_handle h, const float* x, int64_t n, float* y) {
     if (!h || !x || !y || n < 0) return mfail(CMF_MLP_EINVAL, "bad argument");
+    if (h->fused) return n > 0 ? forward_fused(h, x, n, y) : 0;
     if (!h->xd) MTRY(malloc_t(h, &h->xd, (size_t)h->max_batch * h->n_in));
     for (int64_t r0 = 0; r0 < n; r0 += h->max_batch) {
         const int rows = (int)((n - r0) < h->max_batch ? (n - r0) : h->max_batch);
         MCHK(hipMemcpyAsync(h->xd, x + (size_t)r0 * h->n_in, (size_t)rows * h->n_in * sizeof(float),
                             hipMemcpyHostToDevice, h->stream));
-        if (h->fused) {
-            launch_fused<false>(h, FusedTrain{}, h->xd, rows, h->y);
-        } else {
-            hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, h->xd, h->xb,
-                               (long long)rows * h->n_in);
-            forward(h, rows);
-        }
+        hipLaunchKernelGGL(k_to_bf16, dim3(nblk((long long)rows * h->n_in)), dim3(256), 0, h->stream, h->xd, h->xb,
+                           (long long)rows * h->n_in);
+        forward(h, rows);
         MCHK(hipGetLastError());
         MCHK(hipMemcpyAsync(y + (size_t)r0 * h->n_out, h->y, (size_t)rows * h->n_out * sizeof(float),
                             hipMemcpyDeviceToHost, h->stream));
