@@ -12,9 +12,15 @@
 // waits for another. State lives in registers and LDS between the substeps; HBM
 // sees it once per launch. Every value is computed by the statements of the
 // three-phase kernels on the same inputs, so results are the same bits.
+//
+// The levels of a bifurcation path are computed by neighbouring lanes, each keeping
+// its flow in a register; the lanes add them up in the order of the levels. That adds
+// about a tenth to a substep of a block with 80 paths of 5 levels (as one thread per
+// path the five powers and divides in a row would be the longest chain of it).
 #include "cmf_block.hpp"
 
 #include <algorithm>
+#include <queue>
 
 namespace cmf {
 
@@ -30,11 +36,24 @@ namespace cmf {
 //   U_(r+1) = Q_r + downstream(Q_r) + upstream(dam cells of Q_r)
 // (a dam's inflow is the previous flow of its upstream cells). code = position of
 // the first set a cell is in: U_r <= 3r, R_r <= 3r+1, Q_r <= 3r+2.
-bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
-                      const uint8_t* special, const int32_t* domain, int T, int kmax, BlockPlan& out) {
+//
+// Bifurcation paths join cells of different basins: R_r also holds the other ends of
+// the paths of U_r (a path is limited at either end), U_(r+1) those of the paths of R_r,
+// whose flows R_r needs. The rivers are then cut into small pieces, and a block is
+// grown from them along the links, so that most paths stay inside: of 240,019 cells with
+// 20,000 paths, blocks of 512 load 1.07 times as many for kmax = 1, 1.28 for 2 and 1.58
+// for 3 (their outflows are computed 1.06, 1.16 and 1.30 times).
+bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
+    const int n = net.n;
+    const int32_t *next = net.next, *up_ptr = net.up_ptr, *up_idx = net.up_idx, *domain = net.domain;
+    const uint8_t* special = net.special;
+    const bool paths = net.npth > 0;
     out = BlockPlan();
-    if (n <= 0 || T > 1024 || kmax < 1 || 3 * kmax > 200) return false;
-    const int cap = std::max(T / 4, T - 48 * kmax);
+    if (n <= 0 || T > 1024 || kmax < 1 || 3 * kmax > (paths ? 60 : 200)) return false;
+    if (paths && (net.npthlev < 1 || net.npthlev > 64)) return false;
+    const int per_wave = paths ? 64 / net.npthlev : 0;             // paths of a wavefront
+    const int max_paths = paths ? std::min(blk_paths(T), per_wave * (T / 64)) : 0;
+    const int cap = paths ? std::max(8, T / 32) : std::max(T / 4, T - 48 * kmax);
     std::vector<int32_t> total((size_t)n, 1), resid((size_t)n), piece((size_t)n);
     std::vector<uint8_t> root((size_t)n, 0);
     for (int p = 0; p < n; ++p) {
@@ -48,7 +67,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     for (int p = n - 1; p >= 0; --p) piece[(size_t)p] = next[p] >= 0 ? piece[(size_t)next[p]] : total[(size_t)p];
     bool closed = true;
     for (int p = 0; p < n; ++p) {
-        const int lim = piece[(size_t)p] <= T ? T : cap;
+        const int lim = !paths && piece[(size_t)p] <= T ? T : cap;
         closed = closed && lim == T;
         int r = 1;
         for (int k = up_ptr[p]; k < up_ptr[p + 1]; ++k)
@@ -77,7 +96,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     }
     // local cells (owned first) and codes of every piece; a piece whose
     // surroundings overfill a block is halved
-    struct Piece { int32_t beg, size, spec, dams, kines, dom; };   // into loc / codes; special cells
+    struct Piece { int32_t beg, size, spec, dams, kines, dom, paths; };   // into loc / codes; special cells, paths
     std::vector<Piece> done;
     std::vector<int32_t> loc, mark((size_t)n, -1), cur;
     std::vector<uint8_t> codes, curc;
@@ -86,7 +105,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     const int max_spec = blk_special(T);
     const int max_dams = blk_dams(T), max_kines = blk_kines(T);
     auto piece_of = [&](const std::vector<int32_t>& c, size_t from, int count) {
-        Piece p{(int32_t)loc.size(), count, 0, 0, 0, domain ? domain[c[from]] : 0};
+        Piece p{(int32_t)loc.size(), count, 0, 0, 0, domain ? domain[c[from]] : 0, 0};
         for (int j = 0; special && j < count; ++j) {
             const uint8_t f = special[(size_t)c[from + j]];
             p.spec += (f & (BLK_DAM | BLK_LEV)) != 0;
@@ -95,9 +114,151 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
         }
         return p;
     };
-    auto fits = [&](const Piece& p) { return p.size <= T && p.spec <= max_spec && p.dams <= max_dams && p.kines <= max_kines; };
-    std::vector<std::vector<int32_t>> work;
+    auto fits = [&](const Piece& p) {
+        return p.size <= T && p.spec <= max_spec && p.dams <= max_dams && p.kines <= max_kines && p.paths <= max_paths;
+    };
     int stamp = 0;
+    // f(the other end, path) of every path of cell x
+    auto each_path = [&](int x, auto f) {
+        for (int k = net.out_ptr[x]; k < net.out_ptr[x + 1]; ++k) f(net.pth_down[net.out_idx[k]], net.out_idx[k]);
+        for (int k = net.in_ptr[x]; k < net.in_ptr[x + 1]; ++k) f(net.pth_up[net.in_idx[k]], net.in_idx[k]);
+    };
+    // the surroundings of the owned cells in cur, with their codes
+    auto surround = [&] {
+        const int id = stamp++;
+        curc.assign(cur.size(), 0);
+        for (int x : cur) mark[(size_t)x] = id;
+        uint8_t c = 0;
+        auto add = [&](int x) {
+            if (x >= 0 && mark[(size_t)x] != id) { mark[(size_t)x] = id; cur.push_back(x); curc.push_back(c); }
+        };
+        auto add_up = [&](int x) { for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) add(up_idx[k]); };
+        auto add_ends = [&](int x) { each_path(x, [&](int y, int) { add(y); }); };
+        size_t r0 = 0, q0 = 0;                                      // members whose neighbours are already in
+        for (int r = 0; r < kmax && (int)cur.size() <= T; ++r) {
+            const size_t eu = cur.size();
+            c = (uint8_t)(3 * r + 1);
+            for (size_t j = r0; j < eu; ++j) { add_up(cur[j]); add(next[cur[j]]); if (paths) add_ends(cur[j]); }
+            const size_t er = cur.size();
+            c = (uint8_t)(3 * r + 2);
+            for (size_t j = r0; j < er; ++j) add_up(cur[j]);
+            const size_t eq = cur.size();
+            c = (uint8_t)(3 * r + 3);
+            for (size_t j = q0; j < eq; ++j) {
+                add(next[cur[j]]);
+                if (special && (special[(size_t)cur[j]] & BLK_DAMUP)) add_up(cur[j]);
+            }
+            for (size_t j = r0; paths && j < er; ++j) add_ends(cur[j]);
+            r0 = er;
+            q0 = eq;
+        }
+    };
+    // paths whose flows a cell of this code asks for, from its set R_r on (kmax: none)
+    auto path_step = [&](int code) { return std::min(kmax, code < 2 ? 0 : (code + 1) / 3); };
+    std::vector<int32_t> pmark(paths ? (size_t)net.npth : 0, -1), pslot(pmark.size());
+    auto count_paths = [&] {
+        const int id = stamp++;
+        int m = 0;
+        for (size_t j = 0; j < cur.size(); ++j)
+            if (path_step(curc[j]) < kmax)
+                each_path(cur[j], [&](int, int q) { if (pmark[(size_t)q] != id) { pmark[(size_t)q] = id; ++m; } });
+        return m;
+    };
+    auto keep = [&](Piece pc, int nown) {
+        done.push_back(pc);
+        closed = closed && (int)cur.size() == nown;
+        loc.insert(loc.end(), cur.begin(), cur.end());
+        codes.insert(codes.end(), curc.begin(), curc.end());
+    };
+    if (paths) {
+        closed = true;
+        // blocks grown from the river pieces: always the one with most links to the
+        // block for its size, from a seed with most links to the blocks before
+        std::vector<int32_t> links((size_t)npc, 0), seen((size_t)npc, -1), before((size_t)npc, 0), took, grown;
+        std::vector<uint8_t> in((size_t)npc, 0);
+        typedef std::pair<float, int32_t> Cand;
+        std::priority_queue<Cand> near, seeds;
+        int first = 0, blk = 0;
+        double share = 0.8;                                         // owned cells of a full block
+        auto size_of = [&](int i) { return off[(size_t)i + 1] - off[(size_t)i]; };
+        auto each_link = [&](int i, auto f) {                       // pieces a piece is joined to
+            for (int e = off[(size_t)i]; e < off[(size_t)i + 1]; ++e) {
+                const int x = own[(size_t)e];
+                auto to = [&](int y) { if (y >= 0 && piece[(size_t)y] != i && !in[(size_t)piece[(size_t)y]]) f(piece[(size_t)y]); };
+                to(next[x]);
+                for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) to(up_idx[k]);
+                each_path(x, [&](int y, int) { to(y); });
+            }
+        };
+        for (int left = npc; left > 0; ++blk) {
+            took.clear();
+            grown.clear();
+            while (!near.empty()) near.pop();
+            int target = std::max(1, (int)(share * T));
+            bool shrunk = false;
+            for (int tries = 0;; ++tries) {
+                while (!shrunk && (int)grown.size() < target && left > (int)took.size()) {
+                    int i = -1;
+                    while (!near.empty() && i < 0) {
+                        const int c = near.top().second;
+                        near.pop();
+                        if (!in[(size_t)c]) i = c;
+                    }
+                    while (i < 0 && took.empty() && !seeds.empty()) {
+                        if (!in[(size_t)seeds.top().second]) i = seeds.top().second;
+                        seeds.pop();
+                    }
+                    for (int f = first; i < 0; ++f)
+                        if (!in[(size_t)f]) i = f;
+                        else if (f == first) ++first;
+                    if (!grown.empty() && (int)grown.size() + size_of(i) > T) break;
+                    in[(size_t)i] = 1;
+                    took.push_back(i);
+                    grown.insert(grown.end(), own.begin() + off[(size_t)i], own.begin() + off[(size_t)i + 1]);
+                    each_link(i, [&](int c) {
+                        if (seen[(size_t)c] != blk) { seen[(size_t)c] = blk; links[(size_t)c] = 0; }
+                        links[(size_t)c] += 1;
+                        near.push({(float)links[(size_t)c] / (float)size_of(c), c});
+                    });
+                }
+                cur = grown;
+                surround();
+                Piece pc = piece_of(cur, 0, (int)cur.size());
+                pc.paths = count_paths();
+                const bool ok = fits(pc);
+                const bool full = left == (int)took.size() || cur.size() > 0.96 * T || tries >= 4 || shrunk ||
+                                  pc.spec > 0.9 * max_spec || pc.dams > 0.9 * max_dams || pc.paths > 0.94 * max_paths;
+                if (ok && full) {
+                    share = std::max(0.1, std::min(1.0, (double)grown.size() / T));
+                    keep(pc, (int)grown.size());
+                    break;
+                }
+                if (ok) {                                           // room for more
+                    target = std::max((int)grown.size() + 1, (int)((double)grown.size() * 0.985 * T / (double)cur.size()));
+                    continue;
+                }
+                // too much: the pieces taken last go back, one at least
+                if (took.size() < 2) return false;
+                target = (int)std::min((double)grown.size() * 0.96, (double)grown.size() * 0.97 * T / (double)cur.size());
+                while (took.size() > 1 && (int)grown.size() > target) {
+                    const int i = took.back();
+                    took.pop_back();
+                    grown.resize(grown.size() - (size_t)size_of(i));
+                    in[(size_t)i] = 0;
+                    first = std::min(first, i);
+                }
+                shrunk = true;
+            }
+            left -= (int)took.size();
+            for (int i : took)
+                each_link(i, [&](int c) {
+                    before[(size_t)c] += 1;
+                    seeds.push({(float)before[(size_t)c] / (float)size_of(c), c});
+                });
+        }
+    }
+    std::vector<std::vector<int32_t>> work;
+    if (paths) npc = 0;                                             // all of them are in blocks
     for (int i = 0; i < npc; ++i) {
         const int a = off[(size_t)i], b = off[(size_t)i + 1], rt = own[(size_t)b - 1];
         const Piece whole = piece_of(own, (size_t)a, b - a);
@@ -111,37 +272,11 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
         while (!work.empty()) {
             cur.swap(work.back());
             work.pop_back();
-            const int nown = (int)cur.size(), id = stamp++;
-            curc.assign((size_t)nown, 0);
-            for (int x : cur) mark[(size_t)x] = id;
-            uint8_t c = 0;
-            auto add = [&](int x) {
-                if (x >= 0 && mark[(size_t)x] != id) { mark[(size_t)x] = id; cur.push_back(x); curc.push_back(c); }
-            };
-            auto add_up = [&](int x) { for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) add(up_idx[k]); };
-            size_t r0 = 0, q0 = 0;                                  // members whose neighbours are already in
-            for (int r = 0; r < kmax && (int)cur.size() <= T; ++r) {
-                const size_t eu = cur.size();
-                c = (uint8_t)(3 * r + 1);
-                for (size_t j = r0; j < eu; ++j) { add_up(cur[j]); add(next[cur[j]]); }
-                const size_t er = cur.size();
-                c = (uint8_t)(3 * r + 2);
-                for (size_t j = r0; j < er; ++j) add_up(cur[j]);
-                const size_t eq = cur.size();
-                c = (uint8_t)(3 * r + 3);
-                for (size_t j = q0; j < eq; ++j) {
-                    add(next[cur[j]]);
-                    if (special && (special[(size_t)cur[j]] & BLK_DAMUP)) add_up(cur[j]);
-                }
-                r0 = er;
-                q0 = eq;
-            }
+            const int nown = (int)cur.size();
+            surround();
             const Piece pc = piece_of(cur, 0, (int)cur.size());
             if (fits(pc)) {
-                done.push_back(pc);
-                closed = closed && (int)cur.size() == nown;
-                loc.insert(loc.end(), cur.begin(), cur.end());
-                codes.insert(codes.end(), curc.begin(), curc.end());
+                keep(pc, nown);
                 continue;
             }
             if (nown < 2) return false;
@@ -172,19 +307,20 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     std::vector<Piece> room;                                       // what is left in each
     {
         auto holds = [](const Piece& r, const Piece& p) {
-            return r.dom == p.dom && r.size >= p.size && r.spec >= p.spec && r.dams >= p.dams && r.kines >= p.kines;
+            return r.dom == p.dom && r.size >= p.size && r.spec >= p.spec && r.dams >= p.dams && r.kines >= p.kines &&
+                   r.paths >= p.paths;
         };
         auto put = [&](int b, size_t k) {
             if (b < 0) {
                 b = (int)bins.size();
                 bins.emplace_back();
-                room.push_back({0, T, max_spec, max_dams, max_kines, done[k].dom});
+                room.push_back({0, T, max_spec, max_dams, max_kines, done[k].dom, max_paths});
                 out.dom.push_back(done[k].dom);
             }
             const Piece& p = done[k];
             Piece& r = room[(size_t)b];
             bins[(size_t)b].push_back((int32_t)k);
-            r.size -= p.size; r.spec -= p.spec; r.dams -= p.dams; r.kines -= p.kines;
+            r.size -= p.size; r.spec -= p.spec; r.dams -= p.dams; r.kines -= p.kines; r.paths -= p.paths;
             return b;
         };
         // domain by domain (the pieces were cut in descending cell order)
@@ -227,12 +363,22 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
     out.topo.assign(2 * np, 0);
     out.upx_ptr.assign(np, 0);
     out.ndam.assign((size_t)nb, 0);
+    const size_t npb = (size_t)blk_paths(T);
+    if (paths) {
+        out.path.assign(np, -1);
+        out.pword.assign(np, 0);
+        out.pcell.assign(np, 0);
+        out.ppx_ptr.assign(np, 0);
+        out.pends.assign((size_t)nb * npb, 0);
+    }
+    std::vector<std::pair<int, int>> plist;                        // code, path
     // order inside a block: dam, kinematic and levee cells in places of their own
     // (their wavefronts take the rare paths, the others never do), then the owned
     // cells, then the ring by code
     std::vector<int32_t>& pos = resid;                               // local index in the block
     std::vector<int32_t> place((size_t)T), count((size_t)3 * kmax + 6), spot((size_t)T);
     std::fill(mark.begin(), mark.end(), -1);
+    std::fill(pmark.begin(), pmark.end(), -1);
     for (int b = 0; b < nb; ++b) {
         const std::vector<int32_t>& bin = bins[(size_t)b];
         auto code_of = [&](size_t e) { return closed ? 0 : (int)codes[e]; };
@@ -258,6 +404,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
             for (int j = 0; j < done[(size_t)k].size; ++j, ++q)
                 place[(size_t)q] = spot[(size_t)count[(size_t)key_of((size_t)done[(size_t)k].beg + j)]++];
         q = 0;
+        int slots = 0;
         for (int32_t k : bin) {
             const Piece& pc = done[(size_t)k];
             // a piece's neighbours are looked up inside the piece: two pieces of one
@@ -266,6 +413,39 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
                 const int x = loc[(size_t)pc.beg + j];
                 mark[(size_t)x] = k;
                 pos[(size_t)x] = place[(size_t)(q + j)];
+            }
+            if (paths) {
+                // slots of the paths, the owner's (of the upstream end) first; two
+                // pieces of one block may both have a path
+                plist.clear();
+                for (int j = 0; j < pc.size; ++j) {
+                    const int x = loc[(size_t)pc.beg + j], step = path_step(code_of((size_t)pc.beg + j));
+                    const bool mine = codes[(size_t)pc.beg + j] == 0;
+                    if (step < kmax)
+                        each_path(x, [&](int, int w) {
+                            const int code = mine && net.pth_up[w] == x ? 0 : 3 * step + 2;
+                            if (pmark[(size_t)w] != k) {
+                                pmark[(size_t)w] = k;
+                                pslot[(size_t)w] = (int)plist.size();
+                                plist.push_back({code, w});
+                            } else {
+                                int& c = plist[(size_t)pslot[(size_t)w]].first;
+                                c = std::min(c, code);
+                            }
+                        });
+                }
+                std::stable_sort(plist.begin(), plist.end(),
+                                 [](const std::pair<int, int>& x, const std::pair<int, int>& y) { return x.first < y.first; });
+                for (const auto& cw : plist) {
+                    const int w = cw.second, sl = slots++;
+                    pslot[(size_t)w] = sl;
+                    out.pends[(size_t)b * npb + sl] = (uint32_t)pos[(size_t)net.pth_up[w]] | ((uint32_t)pos[(size_t)net.pth_down[w]] << 10);
+                    for (int v = 0; v < net.npthlev; ++v) {
+                        const size_t e = (size_t)b * T + (size_t)(T - 64 * (1 + sl / per_wave) + sl % per_wave * net.npthlev + v);
+                        out.path[e] = w;
+                        out.pword[e] = (uint32_t)v | ((uint32_t)sl << PATH_SLOT) | ((uint32_t)(closed ? 0 : cw.first) << PATH_CODE);
+                    }
+                }
             }
             for (int j = 0; j < pc.size; ++j, ++q) {
                 const int x = loc[(size_t)pc.beg + j];
@@ -290,6 +470,19 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
                 out.cell[e0] = x;
                 out.topo[e0] = nx | (u0 << TOPO_UP0) | (fl << TOPO_FLAGS);
                 out.topo[np + e0] = u1 | ((uint32_t)nup << TOPO_NUP) | ((uint32_t)code << TOPO_CODE);
+                if (paths && path_step(code) < kmax) {
+                    const int no = net.out_ptr[x + 1] - net.out_ptr[x], ni = net.in_ptr[x + 1] - net.in_ptr[x];
+                    if (no > 255 || ni > 255) return false;
+                    uint32_t w = ((uint32_t)no << 16) | ((uint32_t)ni << 24);
+                    int at = 0;
+                    out.ppx_ptr[e0] = (int32_t)out.ppx.size();
+                    each_path(x, [&](int, int p) {
+                        if (at < 2) w |= (uint32_t)pslot[(size_t)p] << (8 * at);
+                        else out.ppx.push_back((uint16_t)pslot[(size_t)p]);
+                        ++at;
+                    });
+                    out.pcell[e0] = w;
+                }
                 if (nup > 2) {
                     out.upx_ptr[e0] = (int32_t)out.upx.size();
                     for (int e = up_ptr[x] + 2; e < up_ptr[x + 1]; ++e)
@@ -301,6 +494,7 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
             if (out.cell[(size_t)b * T + l] < 0) out.topo[np + (size_t)b * T + l] = 255u << TOPO_CODE;   // idle
     }
     if (out.upx.empty()) out.upx.push_back(0);
+    if (out.ppx.empty()) out.ppx.push_back(0);
     return true;
 }
 
@@ -309,10 +503,11 @@ bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const i
 // the arrays of T cells take 120 bytes a cell and the first NL floodplain heights 20
 // more, which fills the 160 KB of a CU with 1024 cells; the mixed form has room for
 // all heights.
-template <class R, int T, bool LEV, bool DAM>
+template <class R, int T, bool LEV, bool DAM, bool PTH>
 struct BlockLds {
     static constexpr bool kOutSum = sizeof(R) == sizeof(float);
-    static constexpr int NL = kOutSum ? 8 : 5, NS = blk_special(T), ND = blk_dams(T) + blk_kines(T);
+    static constexpr int NL = kOutSum ? 8 : (PTH && (LEV || DAM) ? 1 : 5), NS = blk_special(T), ND = blk_dams(T) + blk_kines(T);
+    static constexpr int NP = PTH ? blk_paths(T) : 1;
     R dph[T], dphp[T], q[T], f[T], rate[T];    // read by neighbours
     R fpre[T], fdph[T], ffrc[T];               // own floodplain state
     R a_riv[T], a_fld[T], a_vel[T], a_out[kOutSum ? 1 : T], m_out[T], m_dph[T], m_sto[T];
@@ -324,6 +519,9 @@ struct BlockLds {
     int32_t drow[DAM ? ND : 1], dcode[DAM ? ND : 1];
     double lev[LEV ? NS : 1];
     int32_t lrow[LEV ? NS : 1];
+    // paths: STORGE of the cells, flow of a path summed over its levels and its ends, LEVDPH
+    R sto[PTH ? T : 1], psum[NP], ldph[PTH && LEV ? NS : 1];
+    uint32_t pend[NP];
 };
 enum { DAM_CODE = 15, DAM_KINE = 16, DAM_ACTIVE = 32, DAM_BALANCE = 64 };   // bits of dcode (I1DAM below)
 __device__ __forceinline__ int slot_of_dam(int l, int T) { return l < BLK_KINE_AT ? l : l - BLK_KINE_AT + blk_dams(T); }
@@ -369,13 +567,13 @@ __device__ __forceinline__ void sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-template <class R, int T, bool LEV, bool DAM, bool MB>
+template <class R, int T, bool LEV, bool DAM, bool MB, bool PTH>
 __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block(BlockArgs<R> args_) {
     constexpr bool kOutSum = sizeof(R) == sizeof(float);
     constexpr int NW = T / 64;
     // budget terms formed before the stage inversion (STOPRE2 is STONEW in FP64) and after it
     constexpr int NA = kOutSum ? G_STOPRE2 + 1 : G_STOPRE2, NB = (LEV ? NGLB : G_LEVSTO) - G_STONEW2;
-    __shared__ BlockLds<R, T, LEV, DAM> L;
+    __shared__ BlockLds<R, T, LEV, DAM, PTH> L;
     int l = threadIdx.x, b = blockIdx.x, m = 0;
     int nt = args_.I.nt;
     double dt = args_.I.dt, gdt = args_.I.gdt;
@@ -397,6 +595,9 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
     const R zero = R(0);
     double rs = 0.0, fs = 0.0, zdn = 0.0;
     R ro = zero, fo = zero;
+    int gp = -1;                                                          // path of this thread's level
+    uint32_t wp = 0, wc = 0;
+    R pf = zero;                                                          // its flow
     float f_elevtn = 0.f, f_nxtdst = 1.f, f_rivman = 1.f, f_rivlen = 1.f, f_rivwth = 1.f, f_grarea = 1.f, f_rivhgt = 1.f;
     {
         const BlockArgs<R>& a = block_args<R>();
@@ -409,6 +610,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         w0 = P.topo[pl];
         w1 = P.topo[(size_t)P.nblk * T + pl];
         const bool mouth = (w0 & TOPO_MOUTH) == TOPO_MOUTH;
+        using Lds = BlockLds<R, T, LEV, DAM, PTH>;
         if (g >= 0) {
             rs = S.rivsto[s0]; fs = S.fldsto[s0];
             ro = S.rivout[s0]; fo = S.fldout[s0];
@@ -417,7 +619,6 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             f_rivlen = M.rivlen[g]; f_rivwth = M.rivwth[g]; f_grarea = M.grarea[g]; f_rivhgt = M.rivhgt[g];
             f_elevtn = M.elevtn[g]; f_nxtdst = M.nxtdst[g]; f_rivman = M.rivman[g];
             if (mouth) zdn = M.dwnelv[g];
-            using Lds = BlockLds<R, T, LEV, DAM>;
 #pragma unroll
             for (int k = 0; k < Lds::NL; ++k)
                 if (k < M.nlfp) L.hgt[k][l] = M.fldhgt[(size_t)k * M.n + g];
@@ -439,6 +640,32 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 L.dam[e] = S.damsto[s0]; L.daminf[e] = mine ? S.daminf[s0] : 0.0;
                 L.a_inf[e] = mine && it0 > 0 ? S.daminf_avg[s0] : zero;
                 L.ro[e] = ro; L.fo[e] = fo;
+            }
+        }
+        if (PTH) {
+            if (g >= 0) {
+                wc = P.pcell[pl];
+                double st = rs + fs;
+                if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) { st = st + L.lev[l]; L.ldph[l] = S.levdph[s0]; }
+                L.sto[l] = R(st);
+            }
+            gp = P.path[pl];
+            if (gp >= 0) {
+                wp = P.pword[pl];
+                const int lev = (int)(wp & 63u), slot = (int)(wp >> PATH_SLOT) & 0xff;
+                pf = S.pthflw[(size_t)lev * M.nsp + gp];
+                if (lev == 0) {
+                    const int ip = M.pth_upst[gp], jp = M.pth_down[gp], mi = M.i2mask[ip], mj = M.i2mask[jp];
+                    uint32_t pe = P.pends[(size_t)b * Lds::NP + slot];
+                    if (LEV ? mi == 1 || mj == 1 : mi > 0 || mj > 0) pe |= END_SKIP;
+                    if (mi > 0 || mj > 0) pe |= END_NOLIM;                  // inflow_lspamat:501
+                    if (LEV) {
+                        const int u = M.lev_idx[ip], v = M.lev_idx[jp];
+                        if (u >= 0 && M.lev_tab[M.nlevcell + u] < 1.0) pe |= END_LEV_I;
+                        if (v >= 0 && M.lev_tab[M.nlevcell + v] < 1.0) pe |= END_LEV_J;
+                    }
+                    L.pend[slot] = pe;
+                }
             }
         }
         const bool cont = (w1 >> TOPO_CODE) == 0 && it0 > 0;
@@ -464,6 +691,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         asm volatile("" : "+v"(f_elevtn), "+v"(f_nxtdst), "+v"(f_rivman), "+v"(f_rivlen), "+v"(f_rivwth), "+v"(f_grarea),
                      "+v"(f_rivhgt), "+v"(w0), "+v"(w1), "+v"(g), "+v"(l));
         if (MB) asm volatile("" : "+v"(s0));
+        if (PTH) asm volatile("" : "+v"(gp), "+v"(wp), "+v"(wc));
         const BlockArgs<R>& a = block_args<R>();
         const DevMap& M = a.M;
         const DevState<R>& S = a.S;
@@ -481,6 +709,46 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         const bool is_lev = LEV && (w0 & (BLK_LEV << TOPO_FLAGS));
         const int it = it0 + s, rem = nsub - 1 - s;
         const bool last = it == nt - 1;
+        // ---- path flows, a level per lane (pthflow_path)
+        if (PTH && __any(gp >= 0 && (int)(wp >> PATH_CODE) <= 3 * rem + 2)) {
+            const bool act = gp >= 0 && (int)(wp >> PATH_CODE) <= 3 * rem + 2;
+            const int lev = (int)(wp & 63u), slot = (int)(wp >> PATH_SLOT) & 0xff;
+            const uint32_t pe = act ? L.pend[slot] : END_SKIP;
+            const int li = (int)(pe & 0x3ffu), lj = (int)(pe >> 10) & 0x3ff;
+            R qq = zero;
+            if (!(pe & END_SKIP)) {
+                const size_t np = (size_t)P.nblk * T;
+                const double* pc = P.pconst + (size_t)b * T + l;
+                PathEnds<R> pn;
+                pn.ri_d = pc[0]; pn.rj_d = pc[np];
+                pn.di = L.dph[li]; pn.dj = L.dph[lj];
+                pn.dpi = L.dphp[li]; pn.dpj = L.dphp[lj];
+                if (LEV) {
+                    pn.lev_i = pe & END_LEV_I; pn.lev_j = pe & END_LEV_J;
+                    if (pn.lev_i) { pn.ldi = L.ldph[li]; pn.ei = M.elevtn[M.pth_upst[gp]]; }
+                    if (pn.lev_j) { pn.ldj = L.ldph[lj]; pn.ej = M.elevtn[M.pth_down[gp]]; }
+                }
+                const R before = pf;
+                qq = path_level<R>(pn, path_slope<R>(pn, R(pc[4 * np])), LEV, lev, pc[2 * np], R(gdt), [&](R& w, R& man, R& pre) {
+                    w = R(pc[3 * np]);
+                    man = R(M.pth_man[lev]);
+                    pre = before;
+                });
+            }
+            R sum = zero;
+            const int lane = l & 63, base = lane - lev;
+            for (int k = 0; k < M.npthlev; ++k) sum = sum + __shfl(qq, base + k);
+            if (act) {
+                if (sum != zero) {                                        // pthout:84-95
+                    R rate = (R(0.05) * vmin(L.sto[li], L.sto[lj])) / vabs(sum * R(dt));
+                    rate = vmin(rate, R(1));
+                    qq = qq * rate;
+                    sum = sum * rate;
+                }
+                pf = qq;
+                if (lev == 0) L.psum[slot] = sum;
+            }
+        }
         // ---- outflow (k_outflow)
         if (code <= 3 * rem + 2) {
             FlowIn<R> c;
@@ -529,6 +797,16 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         sync_lds();
         const bool upd = code <= 3 * rem;
         const R runoff = upd ? S.runoff[s0] : zero;                        // in flight during the rate phase
+        const int npo = PTH ? (int)(wc >> 16) & 0xff : 0, npa = PTH ? npo + (int)(wc >> 24) : 0;
+        R pavg = zero, qavg = zero;                                       // as these
+        const bool pupd = PTH && gp >= 0 && (int)(wp >> PATH_CODE) <= 3 * rem, pown = pupd && (wp >> PATH_CODE) == 0;
+        if (PTH && it > 0) {
+            if (own && npa > 0) pavg = S.pthout_avg[s0];
+            if (pown) qavg = S.pthflw_avg[(size_t)(wp & 63u) * M.nsp + gp];
+        }
+        auto slot_at = [&](int k) {
+            return k == 0 ? (int)(wc & 0xffu) : (k == 1 ? (int)(wc >> 8) & 0xff : (int)P.ppx[P.ppx_ptr[b * T + l] + k - 2]);
+        };
         // ---- limiter rate (k_rate)
         if (code <= 3 * rem + 1) {
             double so = (double)vmax(L.q[l], zero) + (double)vmax(L.f[l], zero);
@@ -539,10 +817,36 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 so = (so + (double)vmax(-L.q[u], zero)) + (double)vmax(-L.f[u], zero);
             }
             so = so * dt;
+            for (int k = 0; k < npa; ++k) {
+                const R v = L.psum[slot_at(k)];
+                so = so + (double)vmax(k < npo ? v : -v, zero) * dt;
+            }
             const R dout = vmax(R(so), R(1.e-10));
             L.rate[l] = vmin(R(rs + fs) / dout, R(1));
         }
         sync_lds();
+        // a path's sum under the rate of the end it leaves
+        auto limited = [&](R v, uint32_t pe) {
+            return pe & END_NOLIM ? v : (v >= zero ? v * L.rate[pe & 0x3ffu] : v * L.rate[(pe >> 10) & 0x3ffu]);
+        };
+        if (PTH && pupd) {                                                // update_path
+            const int lev = (int)(wp & 63u);
+            pf = limited(pf, L.pend[(wp >> PATH_SLOT) & 0xffu]);
+            if (pown) {
+                qavg = qavg + pf * rdt;
+                if (last) qavg = qavg / R(a.I.nadd);
+                S.pthflw_avg[(size_t)lev * M.nsp + gp] = qavg;
+            }
+        }
+        if (PTH && last && __any(pown)) {
+            const int lev = (int)(wp & 63u), slot = (int)(wp >> PATH_SLOT) & 0xff, base = (l & 63) - lev;
+            R sumavg = zero;                                              // diag:206-213
+            for (int k = 0; k < M.npthlev; ++k) sumavg = sumavg + __shfl(qavg, base + k);
+            if (pown && lev == 0) {
+                S.pthflwsum[gp] = limited(L.psum[slot], L.pend[slot]);
+                S.pthflwsum_avg[gp] = sumavg;
+            }
+        }
         // ---- limit, inflow, dam balance, storages (k_update)
         {
             double gb[NGLB];
@@ -562,11 +866,17 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 if (nup > 0) inflow(u0);
                 if (nup > 1) inflow(u1);
                 for (int k = 2; k < nup; ++k) inflow(P.upx[P.upx_ptr[b * T + l] + k - 2]);
+                double pthout = 0.0;
+                for (int k = 0; k < npa; ++k) {                           // inflow_lspamat:519-535
+                    const int sl = slot_at(k);
+                    const double v = (double)limited(L.psum[sl], L.pend[sl]);
+                    pthout = k < npo ? pthout + v : pthout - v;
+                }
                 if (is_dam && (L.dcode[e] & DAM_BALANCE))
                     L.dam[e] = (L.dam[e] + ((rivinf + fldinf) + (double)runoff) * dt) - ((double)qrl + (double)qfl) * dt;
                 L.fpre[l] = R(fs);
                 const R outflw = qrl + qfl;
-                storage_next<R>(rs, fs, rivinf, fldinf, 0.0, qrl, qfl, dt, runoff, L.ffrc[l], A.lupsinf,
+                storage_next<R>(rs, fs, rivinf, fldinf, pthout, qrl, qfl, dt, runoff, L.ffrc[l], A.lupsinf,
                                 A.lupsinf ? S.upsinf[s0] : zero, gb);
                 double st = rs + fs;
                 if (is_lev) st = st + L.lev[l];
@@ -580,8 +890,13 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                     if (!kOutSum) L.a_out[l] = L.a_out[l] + outflw * rdt;
                     L.m_out[l] = vmax(L.m_out[l], vabs(outflw));
                     if (is_dam) L.a_inf[e] = L.a_inf[e] + R(L.daminf[e] * dt);
+                    if (PTH && npa > 0) {
+                        R pa = pavg + R(pthout) * rdt;
+                        if (last) pa = pa / R(a.I.nadd);
+                        S.pthout_avg[s0] = pa;
+                    }
                     if (last) {
-                        S.rivinf[s0] = rivinf; S.fldinf[s0] = fldinf; S.pthout[s0] = 0.0;
+                        S.rivinf[s0] = rivinf; S.fldinf[s0] = fldinf; S.pthout[s0] = pthout;
                         S.outflw[s0] = outflw;
                     }
                 }
@@ -601,7 +916,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             if (upd) {
                 Stage o;
                 const Geom geo{(double)f_rivlen, (double)f_rivwth, (double)f_grarea, (double)f_rivhgt};
-                using Lds = BlockLds<R, T, LEV, DAM>;
+                using Lds = BlockLds<R, T, LEV, DAM, PTH>;
                 const BlockHgt<Lds::NL, T> hgt{&L.hgt[0][l], M.fldhgt + g, M.n};
                 if (is_lev) stage_levee(M, hgt, geo, load_lev_row(M, L.lrow[l]), rs, fs, L.lev[l], o);
                 else stage_def<!LEV>(M, hgt, geo, rs, fs, o);
@@ -615,6 +930,10 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                 L.dph[l] = rivdph;
                 L.fdph[l] = R(o.flddph);
                 L.ffrc[l] = R(o.fldfrc);
+                if (PTH) {
+                    L.sto[l] = storge;
+                    if (is_lev) L.ldph[l] = R(o.levdph);
+                }
                 if (own) {
                     gs[0] = stg;
                     gs[G_RIVSTO - G_STONEW2] = rs;
@@ -627,7 +946,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
                         S.fldare[s0] = R(o.fldare);
                         S.sfcelv[s0] = R((double)f_elevtn - (double)f_rivhgt) + rivdph;
                         S.storge[s0] = storge;
-                        if (is_lev) S.levdph[s0] = R(o.levdph);
+                        if (!PTH && is_lev) S.levdph[s0] = R(o.levdph);
                     }
                 }
             }
@@ -644,6 +963,10 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
             part[NGLB + l] = lo;
         }
     }
+    if (PTH && gp >= 0 && (wp >> PATH_CODE) == 0) {
+        const BlockArgs<R>& a = block_args<R>();
+        a.O.pthflw[(size_t)(wp & 63u) * a.M.nsp + gp] = pf;
+    }
     if (g < 0 || (w1 >> TOPO_CODE) != 0) return;
     const BlockArgs<R>& a = block_args<R>();
     const DevState<R>& S = a.S;
@@ -653,7 +976,10 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
     O.rivout[s0] = ro; O.fldout[s0] = fo;
     O.rivdph[s0] = L.dph[l]; O.rivdph_pre[s0] = L.dphp[l];
     O.fldsto_pre[s0] = L.fpre[l]; O.flddph[s0] = L.fdph[l]; O.fldfrc[s0] = L.ffrc[l];
-    if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) O.levsto[s0] = L.lev[l];
+    if (LEV && (w0 & (BLK_LEV << TOPO_FLAGS))) {
+        O.levsto[s0] = L.lev[l];
+        if (PTH) O.levdph[s0] = L.ldph[l];
+    }
     const bool is_dam = DAM && (w0 & (BLK_DAM << TOPO_FLAGS));
     const int e = slot_of_dam(l, T);
     if (is_dam) { O.damsto[s0] = L.dam[e]; S.daminf[s0] = L.daminf[e]; }
@@ -668,7 +994,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         R a5 = zero;
         for (int k = 0; k < nt; ++k) a5 = a5 + runoff * rdt;
         S.runoff_avg[s0] = a5 / nadd;
-        S.pthout_avg[s0] = zero;
+        if (!PTH || (wc >> 16) == 0) S.pthout_avg[s0] = zero;
         a4 = a4 / nadd;
         S.outflw_avg[s0] = a3;
     } else if (!kOutSum) {
@@ -678,33 +1004,54 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
     S.rivout_avg[s0] = a1; S.fldout_avg[s0] = a2; S.rivvel_avg[s0] = av;
 }
 
-template <class R, int T, bool MB>
-static hipError_t launch_block_t(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
-                                 const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
-    const dim3 g(MB ? ((P.nblk + 7) / 8 * 8) << M.lgm : P.nblk), t(T);
-    const BlockArgs<R> a{M, S, O, P, A, I, j, vel0};
-    if (A.llevee && A.ldamout) hipLaunchKernelGGL((k_block<R, T, true, true, MB>), g, t, 0, st, a);
-    else if (A.llevee) hipLaunchKernelGGL((k_block<R, T, true, false, MB>), g, t, 0, st, a);
-    else if (A.ldamout) hipLaunchKernelGGL((k_block<R, T, false, true, MB>), g, t, 0, st, a);
-    else hipLaunchKernelGGL((k_block<R, T, false, false, MB>), g, t, 0, st, a);
+template <class R, int T, bool MB, bool PTH>
+static hipError_t launch_block_t(const BlockArgs<R>& a, hipStream_t st) {
+    const dim3 g(MB ? ((a.P.nblk + 7) / 8 * 8) << a.M.lgm : a.P.nblk), t(T);
+    if (a.A.llevee && a.A.ldamout) hipLaunchKernelGGL((k_block<R, T, true, true, MB, PTH>), g, t, 0, st, a);
+    else if (a.A.llevee) hipLaunchKernelGGL((k_block<R, T, true, false, MB, PTH>), g, t, 0, st, a);
+    else if (a.A.ldamout) hipLaunchKernelGGL((k_block<R, T, false, true, MB, PTH>), g, t, 0, st, a);
+    else hipLaunchKernelGGL((k_block<R, T, false, false, MB, PTH>), g, t, 0, st, a);
     return hipGetLastError();
 }
 
 template <class R, bool MB>
-static hipError_t launch_block_mb(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
-                                  const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
-    switch (P.T) {
-        case 256: return launch_block_t<R, 256, MB>(M, S, O, P, A, I, j, vel0, st);
-        case 512: return launch_block_t<R, 512, MB>(M, S, O, P, A, I, j, vel0, st);
-        default: return launch_block_t<R, 1024, MB>(M, S, O, P, A, I, j, vel0, st);
+static hipError_t launch_block_mb(const BlockArgs<R>& a, hipStream_t st) {
+    switch (a.P.T) {
+        case 256: return launch_block_t<R, 256, MB, false>(a, st);
+        case 512: return launch_block_t<R, 512, MB, false>(a, st);
+        default: return launch_block_t<R, 1024, MB, false>(a, st);
     }
+}
+
+// flows of the paths with an end outside the network, which no block holds (update_path)
+template <class R>
+__global__ void k_dead_paths(DevMap M, DevState<R> S, const int32_t* dead, int n) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int q = dead[k];
+    for (int l = 0; l < M.npthlev; ++l) {
+        S.pthflw[(size_t)l * M.nsp + q] = R(0);
+        S.pthflw_avg[(size_t)l * M.nsp + q] = R(0);
+    }
+    S.pthflwsum[q] = R(0);
+    S.pthflwsum_avg[q] = R(0);
 }
 
 template <class R>
 hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
                         const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
-    if (M.nmem > 1 || M.cell_dom) return launch_block_mb<R, true>(M, S, O, P, A, I, j, vel0, st);
-    return launch_block_mb<R, false>(M, S, O, P, A, I, j, vel0, st);
+    const BlockArgs<R> a{M, S, O, P, A, I, j, vel0};
+    if (P.npth > 0) {
+        if (j == 0 && P.ndead > 0)
+            hipLaunchKernelGGL((k_dead_paths<R>), dim3((P.ndead + 255) / 256), dim3(256), 0, st, M, S, P.dead, P.ndead);
+        switch (P.T) {
+            case 256: return launch_block_t<R, 256, false, true>(a, st);
+            case 512: return launch_block_t<R, 512, false, true>(a, st);
+            default: return launch_block_t<R, 1024, false, true>(a, st);
+        }
+    }
+    if (M.nmem > 1 || M.cell_dom) return launch_block_mb<R, true>(a, st);
+    return launch_block_mb<R, false>(a, st);
 }
 template hipError_t launch_block<double>(const DevMap&, const DevState<double>&, const BlockState<double>&,
                                          const BlockTab&, const StepArgs&, const InstStep&, int, const double*,

@@ -18,15 +18,31 @@ struct BlockPlan {
     std::vector<uint16_t> upx;
     std::vector<int32_t> ndam;                 // [nblk] dam cells | kinematic cells << 16
     std::vector<int32_t> dom;                  // [nblk] domain of the block's cells
+    // bifurcation paths (empty without): thread of a block -> path and level of its wavefront, packed
+    // with the ends and codes; path slots of a cell, the third on in ppx
+    std::vector<int32_t> path;                 // [nblk*T] path or -1
+    std::vector<uint32_t> pword, pends;        // [nblk*T] PATH_* fields; [nblk*blk_paths(T)] ends of a slot
+    std::vector<uint32_t> pcell;               // [nblk*T] first two slots (8 bits each), paths out and in (8 each)
+    std::vector<int32_t> ppx_ptr;              // [nblk*T]
+    std::vector<uint16_t> ppx;
+};
+// dam cell (any), levee cell, reads its upstream cells' flows, dam cell on the kinematic wave
+enum : uint8_t { BLK_DAM = 1, BLK_LEV = 2, BLK_DAMUP = 4, BLK_KINE = 8 };
+// The network in device cell order: downstream cells, upstream lists, BLK_* flags
+// (NULL: none), domains (ascending, NULL: one; a block's cells share theirs), and the
+// bifurcation paths with both ends in the network (lists of those out of and into a
+// cell; npth = 0: none).
+struct BlockNet {
+    int n;
+    const int32_t *next, *up_ptr, *up_idx;
+    const uint8_t* special;
+    const int32_t* domain;
+    int npth, npthlev;
+    const int32_t *pth_up, *pth_down, *out_ptr, *out_idx, *in_ptr, *in_idx;
 };
 // False when the network cannot be cut into such blocks (a cell with too many
 // upstream cells, or whose surroundings alone overfill a block).
-// special: BLK_* flags of every cell (NULL: none).
-// dam cell (any), levee cell, reads its upstream cells' flows, dam cell on the kinematic wave
-enum : uint8_t { BLK_DAM = 1, BLK_LEV = 2, BLK_DAMUP = 4, BLK_KINE = 8 };
-// domain: of every cell, ascending (NULL: one); a block's cells share theirs.
-bool build_block_plan(int n, const int32_t* next, const int32_t* up_ptr, const int32_t* up_idx,
-                      const uint8_t* special, const int32_t* domain, int T, int kmax, BlockPlan& out);
+bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out);
 
 // Order of the cells of a block: dam cells from 0, kinematic cells (above a dam)
 // from BLK_KINE_AT, so that the two rare flow rules are computed by different
@@ -36,6 +52,14 @@ constexpr int BLK_KINE_AT = 64;
 constexpr int blk_dams(int T) { return T / 32; }
 constexpr int blk_kines(int T) { return 3 * T / 32; }
 constexpr int blk_special(int T) { return 3 * T / 8; }
+constexpr int blk_paths(int T) { return T < 1024 ? T / 4 : 255; }
+
+// The levels of a path are computed by neighbouring lanes, whole paths in a wavefront,
+// from the last one of the block down (the ring's, which has least to do otherwise).
+// Word of such a thread: level (6 bits), slot (8), code (6); ends of a slot: local cells
+// (10 bits each), flags set by the kernel
+constexpr int PATH_SLOT = 6, PATH_CODE = 14;
+constexpr uint32_t END_SKIP = 1u << 20, END_NOLIM = 1u << 21, END_LEV_I = 1u << 22, END_LEV_J = 1u << 23;
 
 // fields of the two topology words of a local cell (local indices < 1024)
 constexpr uint32_t TOPO_MOUTH = 0x7ff;         // word 0: downstream (11 bits), first upstream (10), flags (2)
@@ -51,6 +75,14 @@ struct BlockTab {
     const uint16_t* upx;
     const int32_t* ndam;
     const int32_t* dom;
+    int npth;                                  // > 0: with paths
+    const int32_t* path;
+    const uint32_t *pword, *pends, *pcell;
+    const int32_t* ppx_ptr;
+    const uint16_t* ppx;
+    const double* pconst;                      // [5][nblk*T]: riverbeds of the ends, level elevation, width, distance
+    int ndead;                                 // paths with an end outside the network, in dead
+    const int32_t* dead;
 };
 
 // the arrays a launch hands to the next one: written by the owner of a cell while
@@ -59,6 +91,7 @@ template <class R>
 struct BlockState {
     double *rivsto, *fldsto, *levsto, *damsto;
     R *rivout, *fldout, *rivdph, *rivdph_pre, *fldsto_pre, *flddph, *fldfrc;
+    R *pthflw, *levdph;                        // with paths
 };
 
 // Launches of an instance of nt substeps: one with a closed plan, else an even number

@@ -813,7 +813,7 @@ template <>
 BlockState<float>& alt_of<float>(cmf_hip_ctx* h) { return h->alt32; }
 
 // Whether an outer step of up to nt substeps runs as block launches: the handle has a
-// partition (no bifurcation paths; setup_blocks), the scheme is the default one,
+// partition (setup_blocks), the scheme is the default one,
 // DAMINF is zero outside the dam cells, and no other form of the substep is asked
 // for (graph replay, the persistent kernel, per-phase timing). One substep of an open
 // partition would take two launches that move the state for it.
@@ -832,7 +832,7 @@ int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t ntmax, bool vel_first
     const BlockTab& P = h->block;
     const int nl = block_launches(ntmax, P.kmax, P.closed);
     const BlockState<R> home{S.rivsto, S.fldsto, S.levsto, S.damsto, S.rivout, S.fldout, S.rivdph, S.rivdph_pre,
-                             S.fldsto_pre, S.flddph, S.fldfrc};
+                             S.fldsto_pre, S.flddph, S.fldfrc, S.pthflw, S.levdph};
     const BlockState<R>& alt = alt_of<R>(h);
     for (int j = 0; j < nl; ++j) {
         DevState<R> Sk = S;
@@ -840,6 +840,7 @@ int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t ntmax, bool vel_first
             Sk.rivsto = alt.rivsto; Sk.fldsto = alt.fldsto; Sk.levsto = alt.levsto; Sk.damsto = alt.damsto;
             Sk.rivout = alt.rivout; Sk.fldout = alt.fldout; Sk.rivdph = alt.rivdph; Sk.rivdph_pre = alt.rivdph_pre;
             Sk.fldsto_pre = alt.fldsto_pre; Sk.flddph = alt.flddph; Sk.fldfrc = alt.fldfrc;
+            if (P.npth > 0) { Sk.pthflw = alt.pthflw; Sk.levdph = alt.levdph; }
         }
         const R* vel0 = vel_first ? (const R*)h->vel_buf : nullptr;
         HIPCHK(launch_block<R>(h->M, Sk, P.closed || (j & 1) ? home : alt, P, A, h->h_inst[0], j, vel0, h->stream));
@@ -1222,12 +1223,42 @@ std::vector<BlockShape> block_shapes(int64_t ns, int ninst, bool mixed) {
     return v;
 }
 
+// The same with bifurcation paths (single models). Blocks of 512 cells leave room for
+// the ring that paths make larger, and their second round of a launch is finer:
+//  * whole groups of basins: 938 cells, all options, 8 substeps, FP64: T = 256 186 us
+//    (T = 512 201, 1024 239; three-phase 319)
+//  * 15,001 cells, 1,000 paths, levees and dams, 222 substeps, FP64: kmax 6 3.1 ms (kmax
+//    4 3.3, 3 3.6; T = 256, kmax 2 3.6; T = 1024, kmax 4 4.5; three-phase 6.1)
+//  * 60,005 cells, 5,000 paths, 893 substeps, FP64: kmax 4 11.7 ms (kmax 3 12.5, 2 14.2;
+//    T = 1024, kmax 6 14.7; three-phase 24.9)
+//  * 240,019 cells, 20,000 paths, 2163 substeps: FP64 kmax 3 74.4 ms (kmax 2 77.2, 1
+//    110.3; T = 1024, kmax 4 75.1, 1 80.2; T = 256, kmax 2 78.1; three-phase 110.1); mixed
+//    54.0 (kmax 2 53.9; T = 1024, kmax 4 61.1; three-phase 96.4)
+//  * 583,000 cells, 50,000 paths, 1202 substeps: FP64 98.5 (T = 1024, kmax 3 97.0;
+//    three-phase 130.2); mixed 66.1 (kmax 2 67.4; T = 1024 78.2; three-phase 103.1)
+std::vector<BlockShape> path_shapes(int n) {
+    const int any = 0x7fffffff;
+    std::vector<BlockShape> v;
+    if (n <= 256 * 256) v.push_back({256, 1, true, any});
+    if (n <= 64 * 512) v.push_back({512, 6, false, any});
+    if (n <= 240 * 512) v.push_back({512, 4, false, any});
+    v.push_back({512, 3, false, any});
+    v.push_back({512, 2, false, any});
+    return v;
+}
+
+// the bifurcation paths in device cell order (-1: an end outside the network)
+struct BlockPaths {
+    std::vector<int32_t> up, down, out_ptr, out_idx, in_ptr, in_idx;
+    int live = 0;
+};
+
 // partition of the network for block launches, its device copy and the second set
 // of the arrays the launches hand on
 template <class R>
 int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
                  const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
-                 const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of) {
+                 const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of, const BlockPaths& pth, const cmf_map* mp) {
     const int n = h->d.nseqall;
     std::vector<uint8_t> special;
     if (h->o.ldamout || h->o.llevee) special.assign((size_t)n, 0);
@@ -1236,11 +1267,19 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
                                         (i1d[(size_t)p] == 10 ? BLK_KINE : 0));
     for (int p = 0; p < n && h->o.llevee; ++p)
         if (lev_of[(size_t)p] >= 0) special[(size_t)p] |= BLK_LEV;
+    BlockNet net{n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(), dom_of.data()};
+    const bool paths = pth.live > 0;
+    if (paths) {
+        net.npth = h->d.npthout; net.npthlev = h->d.npthlev;
+        net.pth_up = pth.up.data(); net.pth_down = pth.down.data();
+        net.out_ptr = pth.out_ptr.data(); net.out_idx = pth.out_idx.data();
+        net.in_ptr = pth.in_ptr.data(); net.in_idx = pth.in_idx.data();
+    }
     BlockPlan bp;
     bool ok = false;
-    for (const BlockShape& b : block_shapes(h->M.ns, h->ninst, sizeof(R) == sizeof(float))) {
-        ok = build_block_plan(n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(),
-                              dom_of.data(), b.T, b.kmax, bp) &&
+    for (const BlockShape& b : paths ? path_shapes(n)
+                                     : block_shapes(h->M.ns, h->ninst, sizeof(R) == sizeof(float))) {
+        ok = build_block_plan(net, b.T, b.kmax, bp) &&
              (bp.closed || !b.closed_only) && (int64_t)bp.nblk * h->nmem <= b.max_blocks;
         // blocks hold cells of one domain: many small domains would leave them empty
         ok = ok && ((int64_t)bp.nblk * h->nmem <= 256 || (int64_t)bp.nblk * bp.T <= 2 * (int64_t)n);
@@ -1258,11 +1297,39 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
     TRY(put_raw(h, &ph, bp.upx.data(), bp.upx.size())); P.upx = ph;
     TRY(put_raw(h, &p32, bp.ndam.data(), bp.ndam.size())); P.ndam = p32;
     TRY(put_raw(h, &p32, bp.dom.data(), bp.dom.size())); P.dom = p32;
+    if (paths) {
+        const int np = h->d.npthout;
+        const size_t nt = (size_t)bp.nblk * bp.T;
+        TRY(put_raw(h, &p32, bp.path.data(), nt)); P.path = p32;
+        TRY(put_raw(h, &pu, bp.pword.data(), nt)); P.pword = pu;
+        TRY(put_raw(h, &pu, bp.pends.data(), bp.pends.size())); P.pends = pu;
+        TRY(put_raw(h, &pu, bp.pcell.data(), nt)); P.pcell = pu;
+        TRY(put_raw(h, &p32, bp.ppx_ptr.data(), nt)); P.ppx_ptr = p32;
+        TRY(put_raw(h, &ph, bp.ppx.data(), bp.ppx.size())); P.ppx = ph;
+        std::vector<double> pc(5 * nt, 1.0);
+        auto bed = [&](int p) { return (double)(float)mp->elevtn[h->perm[(size_t)p]] - (double)(float)mp->rivhgt[h->perm[(size_t)p]]; };
+        for (size_t e = 0; e < nt; ++e) {
+            const int q = bp.path[e];
+            if (q < 0) continue;
+            const size_t lq = (size_t)(bp.pword[e] & 63u) * (size_t)np + (size_t)q;
+            pc[e] = bed(pth.up[(size_t)q]); pc[nt + e] = bed(pth.down[(size_t)q]);
+            pc[2 * nt + e] = mp->pth_elv[lq]; pc[3 * nt + e] = mp->pth_wth[lq]; pc[4 * nt + e] = mp->pth_dst[q];
+        }
+        double* pd = nullptr;
+        TRY(put_raw(h, &pd, pc.data(), pc.size())); P.pconst = pd;
+        P.npth = np;
+    }
+    std::vector<int32_t> dead;                            // no block holds these (none may, with no live path)
+    for (int q = 0; h->o.lpthout && q < h->d.npthout; ++q)
+        if (pth.up[(size_t)q] < 0 || pth.down[(size_t)q] < 0) dead.push_back(q);
+    P.ndead = (int)dead.size();
+    if (P.ndead > 0) { TRY(put_raw(h, &p32, dead.data(), dead.size())); P.dead = p32; }
     if (!bp.closed) {
         BlockState<R>& B = alt_of<R>(h);
         const size_t ns = ((size_t)h->M.ns + 63) / 64 * 64, nlev = h->o.llevee ? ns : 0, ndm = h->o.ldamout ? ns : 0;
+        const size_t npl = paths ? ((size_t)h->d.npthout * h->d.npthlev + 63) / 64 * 64 : 0, nld = paths ? nlev : 0;
         double* d = nullptr;                              // the doubles, then the fields in R, which is no larger
-        if (dalloc(h, &d, 2 * ns + nlev + ndm + 7 * ns * sizeof(R) / sizeof(double)) != 0) {
+        if (dalloc(h, &d, 2 * ns + nlev + ndm + (7 * ns + npl + nld) * sizeof(R) / sizeof(double)) != 0) {
             (void)hipGetLastError();                      // no memory for it: the three-phase kernels need none
             return 0;
         }
@@ -1273,6 +1340,8 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
             *p = r;
             r += ns;
         }
+        B.pthflw = r;
+        B.levdph = r + npl;
     }
     P.nblk = bp.nblk;
     h->block = P;
@@ -1514,6 +1583,7 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         TRY(put_raw(h, &p32, m2.data(), (size_t)n)); M.i2mask = p32;
     }
     // bifurcation paths (maps:531-639)
+    BlockPaths bpth;
     M.pth_dom = nullptr;
     M.nsp = 0;
     if (h->o.lpthout) {
@@ -1548,6 +1618,7 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         TRY(put_raw(h, &p32, iptr.data(), iptr.size())); M.pinf_ptr = p32;
         TRY(put_raw(h, &p32, iidx.data(), iidx.size())); M.pinf_idx = p32;
         if (h->ndom > 1) { TRY(put_raw(h, &p32, pdom.data(), (size_t)np)); M.pth_dom = p32; }
+        bpth = BlockPaths{pu, pdn, optr, oidx, iptr, iidx, (int)oidx.size()};
         TRY(put_raw(h, &pd, mp->pth_dst, (size_t)np)); M.pth_dst = pd;
         TRY(put_raw(h, &pd, mp->pth_elv, (size_t)np * nlv)); M.pth_elv = pd;
         TRY(put_raw(h, &pd, mp->pth_wth, (size_t)np * nlv)); M.pth_wth = pd;
@@ -1619,9 +1690,9 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
             if (ddom[(size_t)p] < ddom[(size_t)p - 1]) return fail(CMF_EMAP, "domains are not contiguous in device order");
         TRY(put_raw(h, &h->d_dom_off, doff.data(), doff.size()));
     }
-    if (h->permuted && !h->o.lpthout && h->nmem <= BLOCK_MEMBERS)
-        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx, ddom)
-                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx, ddom));
+    if (h->permuted && h->nmem <= BLOCK_MEMBERS && (!h->o.lpthout || h->ninst == 1))
+        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx, ddom, bpth, mp)
+                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx, ddom, bpth, mp));
     h->map_set = true;
     return 0;
 }

@@ -367,6 +367,68 @@ __device__ __forceinline__ double rivelv_of(const DevMap& M, int i) {
     return (double)M.elevtn[i] - (double)M.rivhgt[i];            // maps:722
 }
 
+// The two ends of a bifurcation path: riverbed elevations, depths, and for a levee end
+// (lev_*) its LEVDPH and ground elevation
+template <class R>
+struct PathEnds {
+    double ri_d, rj_d;
+    R di, dj, dpi, dpj;
+    bool lev_i = false, lev_j = false;
+    R ldi = R(0), ldj = R(0);
+    float ei = 0.f, ej = 0.f;
+};
+// Water surface slope along a path. Surface terms are in difference form with R =
+// float: each surface height relative to a level elevation is a depth plus the exact
+// FP64 elevation difference rounded once.
+template <class R>
+__device__ __forceinline__ R path_slope(const PathEnds<R>& e, R dst) {
+    constexpr bool kDiff = sizeof(R) == sizeof(float);
+    const R si = R(e.ri_d) + e.di, sj = R(e.rj_d) + e.dj;
+    const R dslp = (kDiff ? (e.di - e.dj) + R(e.ri_d - e.rj_d) : si - sj) / dst;
+    return vmax(R(-0.005), vmin(R(0.005), dslp));
+}
+// Flow of level l of a path before its limits, pthout:20-83 / levee:497-590.
+// load(w, man, pre): width, roughness and the flow before, asked for where the level is wet
+template <class R, class Load>
+__device__ __forceinline__ R path_level(const PathEnds<R>& e, R dslp, int llevee, int l, double elv_d, R gdt, Load load) {
+    constexpr bool kDiff = sizeof(R) == sizeof(float);
+    const R zero = R(0), one = R(1);
+    // max(si, sj) - elv, max(pi, pj) - elv and max(li, lj) - elv
+    R hs, hp, hl;
+    if (kDiff) {
+        const R ai = R(e.ri_d - elv_d), aj = R(e.rj_d - elv_d);
+        hs = vmax(e.di + ai, e.dj + aj);
+        hp = vmax(e.dpi + ai, e.dpj + aj);
+        const R lvi = e.lev_i ? vmin(e.ldi + R((double)e.ei - elv_d), e.di + ai) : e.di + ai;
+        const R lvj = e.lev_j ? vmin(e.ldj + R((double)e.ej - elv_d), e.dj + aj) : e.dj + aj;
+        hl = vmax(lvi, lvj);
+    } else {
+        const R elv = R(elv_d), ri = R(e.ri_d), rj = R(e.rj_d);
+        const R si = ri + e.di, sj = rj + e.dj;
+        const R li = e.lev_i ? vmin(R(e.ei) + e.ldi, si) : si, lj = e.lev_j ? vmin(R(e.ej) + e.ldj, sj) : sj;   // D2SFCELV_LEV
+        hs = vmax(si, sj) - elv;
+        hp = vmax(ri + e.dpi, rj + e.dpj) - elv;
+        hl = vmax(li, lj) - elv;
+    }
+    R dflw, dflw_im;
+    if (!llevee || l == 0) {
+        dflw = vmax(hs, zero);
+        const R dflw_pr = vmax(hp, zero);
+        dflw_im = vsqrt(dflw * dflw_pr);
+        if (llevee) { if (dflw_im <= zero) dflw_im = dflw; }
+        else dflw_im = vmax(dflw_im, vsqrt(dflw * R(0.01)));
+    } else {
+        dflw = vmax(hl, zero);
+        dflw_im = dflw;
+    }
+    if (!(dflw_im > R(1.e-5))) return zero;
+    R w, man, pre;
+    load(w, man, pre);
+    const R dout_pr = (llevee && l > 0) ? pre * (one / w) : pre / w;
+    return (w * (dout_pr + (gdt * dflw_im) * dslp)) /
+           (one + ((gdt * (man * man)) * vabs(dout_pr)) * vpow(dflw_im, R(K_P7O3)));
+}
+
 struct Stage {
     double rivsto, fldsto, levsto;
     double rivdph, flddph, fldfrc, fldare, levdph;

@@ -304,67 +304,26 @@ __device__ __forceinline__ void pthflow_path(const DevMap& M, const DevState<R>&
     const int si_ = sidx<MB>(M, ip, m), sj_ = sidx<MB>(M, jp, m);
     const R zero = R(0), one = R(1);
     const R gdt = R(I.gdt);
-    // Surface terms; with R = float in difference form (see outflow_cell): each
-    // surface height relative to a level elevation is a depth plus the exact FP64
-    // elevation difference rounded once.
-    constexpr bool kDiff = sizeof(R) == sizeof(float);
-    const double ri_d = rivelv_of(M, ip), rj_d = rivelv_of(M, jp);
-    const R di = S.rivdph[si_], dj = S.rivdph[sj_];
-    const R dpi = S.rivdph_pre[si_], dpj = S.rivdph_pre[sj_];
-    const R ri = R(ri_d), rj = R(rj_d);
-    const R si = ri + di, sj = rj + dj;
-    const R pi = ri + dpi, pj = rj + dpj;
-    R dslp = (kDiff ? (di - dj) + R(ri_d - rj_d) : si - sj) / R(M.pth_dst[p]);
-    dslp = vmax(R(-0.005), vmin(R(0.005), dslp));
-    R li = si, lj = sj;                                              // D2SFCELV_LEV
-    bool lev_i = false, lev_j = false;
-    R ldi = zero, ldj = zero;
+    PathEnds<R> e;
+    e.ri_d = rivelv_of(M, ip); e.rj_d = rivelv_of(M, jp);
+    e.di = S.rivdph[si_]; e.dj = S.rivdph[sj_];
+    e.dpi = S.rivdph_pre[si_]; e.dpj = S.rivdph_pre[sj_];
     if (A.llevee) {
         const int a = M.lev_idx[ip], b = M.lev_idx[jp];
         const int nlc = M.nlevcell;
-        lev_i = a >= 0 && M.lev_tab[nlc + a] < 1.0;
-        lev_j = b >= 0 && M.lev_tab[nlc + b] < 1.0;
-        if (lev_i) { ldi = S.levdph[si_]; li = vmin(R(M.elevtn[ip]) + ldi, si); }
-        if (lev_j) { ldj = S.levdph[sj_]; lj = vmin(R(M.elevtn[jp]) + ldj, sj); }
+        e.lev_i = a >= 0 && M.lev_tab[nlc + a] < 1.0;
+        e.lev_j = b >= 0 && M.lev_tab[nlc + b] < 1.0;
+        if (e.lev_i) { e.ldi = S.levdph[si_]; e.ei = M.elevtn[ip]; }
+        if (e.lev_j) { e.ldj = S.levdph[sj_]; e.ej = M.elevtn[jp]; }
     }
+    const R dslp = path_slope<R>(e, R(M.pth_dst[p]));
     R sum = zero;
     for (int l = 0; l < nl; ++l) {
-        const double elv_d = M.pth_elv[(size_t)l * np + p];
-        const R elv = R(elv_d);
-        // max(si, sj) - elv, max(pi, pj) - elv and max(li, lj) - elv
-        R hs, hp, hl;
-        if (kDiff) {
-            const R ai = R(ri_d - elv_d), aj = R(rj_d - elv_d);
-            hs = vmax(di + ai, dj + aj);
-            hp = vmax(dpi + ai, dpj + aj);
-            const R lvi = lev_i ? vmin(ldi + R((double)M.elevtn[ip] - elv_d), di + ai) : di + ai;
-            const R lvj = lev_j ? vmin(ldj + R((double)M.elevtn[jp] - elv_d), dj + aj) : dj + aj;
-            hl = vmax(lvi, lvj);
-        } else {
-            hs = vmax(si, sj) - elv;
-            hp = vmax(pi, pj) - elv;
-            hl = vmax(li, lj) - elv;
-        }
-        R dflw, dflw_im;
-        if (!A.llevee || l == 0) {
-            dflw = vmax(hs, zero);
-            R dflw_pr = vmax(hp, zero);
-            dflw_im = vsqrt(dflw * dflw_pr);
-            if (A.llevee) { if (dflw_im <= zero) dflw_im = dflw; }
-            else dflw_im = vmax(dflw_im, vsqrt(dflw * R(0.01)));
-        } else {
-            dflw = vmax(hl, zero);
-            dflw_im = dflw;
-        }
-        R qq = zero;
-        if (dflw_im > R(1.e-5)) {
-            const R w = R(M.pth_wth[(size_t)l * np + p]);
-            const R man = R(M.pth_man[l]);
-            const R pre = S.pthflw[(size_t)l * nsp + q];            // D1PTHFLW_PRE
-            const R dout_pr = (A.llevee && l > 0) ? pre * (one / w) : pre / w;
-            qq = (w * (dout_pr + (gdt * dflw_im) * dslp)) /
-                 (one + ((gdt * (man * man)) * vabs(dout_pr)) * vpow(dflw_im, R(K_P7O3)));
-        }
+        const R qq = path_level<R>(e, dslp, A.llevee, l, M.pth_elv[(size_t)l * np + p], gdt, [&](R& w, R& man, R& pre) {
+            w = R(M.pth_wth[(size_t)l * np + p]);
+            man = R(M.pth_man[l]);
+            pre = S.pthflw[(size_t)l * nsp + q];                        // D1PTHFLW_PRE
+        });
         S.pthflw_u[(size_t)l * nsp + q] = qq;
         sum = sum + qq;
     }

@@ -134,3 +134,62 @@ def test_ensemble(sizes, members, lev, dam, prec):
     print("substeps", sorted(spread), flush=True)
     for x in g.values():
         x.close()
+
+
+PATH_KEYS = ["pthflw", "pthflwsum", "pthflw_avg", "pthflwsum_avg", "pthout_avg", "pthout"]
+
+
+def compare_paths(m, st, runoff, prec, caps, dt=86400.0):
+    g = {k: CMFModel(m, prec) for k in ("blocks", "phases")}
+    g["phases"].set_tune(graph=1)
+    for x in g.values():
+        x.set_state(st)
+        x.set_runoff(runoff)
+    names = STATE_KEYS + PATH_KEYS + ["levsto", "levdph", "damsto", "daminf", "daminf_avg"]
+    names = [k for k in dict.fromkeys(names) if g["blocks"]._available(k)]
+    flows = 0.0
+    for cap in caps:
+        out = {k: x.physics_advance(dt, nt_cap=cap, budget=True) for k, x in g.items()}
+        assert out["blocks"][0] == out["phases"][0]
+        for k in range(11):
+            assert rel_err(out["blocks"][1][:, k], out["phases"][1][:, k]) < 1e-14, k
+        a, b = (x.get_state(names) for x in g.values())
+        for k in names:
+            assert np.array_equal(a[k], b[k]), (k, cap, rel_err(a[k], b[k]))
+        flows = max(flows, np.abs(a["pthflwsum"]).max())
+    for x in g.values():
+        x.close()
+    assert flows > 0.0                                     # the paths carry water
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("case", ["pth", "levpth", "all", "allwet"])
+def test_paths_small(case, prec):
+    m, net, st, rvec = prepare(case, 1)
+    compare_paths(m, upload_keys(st), rvec[0], prec, [0, 1, 2, 31])
+
+
+# blocks grown along the paths, with paths that leave them, cells with several paths,
+# masked cells (dams) and paths with an end outside the network; one level to ten
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("cells, per, levels, lev, dam, dead", [
+    (9000, 12, 5, 0.0, 0, 0), (9000, 8, 5, 0.3, 60, 40), (9000, 20, 1, 0.2, 0, 0), (5000, 15, 10, 0.0, 25, 7),
+    (140000, 12, 5, 0.0, 0, 0)])
+def test_paths_cut(cells, per, levels, lev, dam, dead, prec):
+    net = synth.regional_networks([cells], 3, land_frac=0.9)[0]
+    synth.add_bifurcations(net, net.ncells // per, levels, 3)
+    if lev:
+        synth.add_levees(net, lev, 3, hmin=0.5, hmax=3.0, fmin=0.05, fmax=0.5)
+    if dam:
+        synth.add_dams(net, max(3, net.ncells // dam), 3)
+    m = maps.build_map(net, maps.Options(lpthout=True, llevee=lev > 0, ldamout=dam > 0))
+    st = maps.cold_start(m)
+    st["rivsto"] = m.rivstomax * np.random.default_rng(3).uniform(0.3, 1.9, m.n)
+    if dam:
+        maps.init_dams(m, net, st)
+    if dead:
+        m.pth_upst[::dead] = -1
+        m.pth_down[1::dead] = -1
+        st["pthflw"][:, ::dead] = 3.0
+    ro = m.vec(synth.make_runoff(net, 1, 3, mean_mm_day=20.0)[0])
+    compare_paths(m, upload_keys(st), ro, prec, [1, 2, 3, 11, 12, 13] if cells < 100000 else [9])
