@@ -41,8 +41,9 @@ namespace cmf {
 // the paths of U_r (a path is limited at either end), U_(r+1) those of the paths of R_r,
 // whose flows R_r needs. The rivers are then cut into small pieces, and a block is
 // grown from them along the links, so that most paths stay inside: of 240,019 cells with
-// 20,000 paths, blocks of 512 load 1.07 times as many for kmax = 1, 1.28 for 2 and 1.58
-// for 3 (their outflows are computed 1.06, 1.16 and 1.30 times).
+// 20,000 paths, 702 blocks of 512 load 1.42 times as many for kmax = 3 and compute 1.22
+// times as many outflows (pieces of T/32 cells 780 and 1.58; T/4 710 with more room
+// left; without the small pieces put into the room at the end 714).
 bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
     const int n = net.n;
     const int32_t *next = net.next, *up_ptr = net.up_ptr, *up_idx = net.up_idx, *domain = net.domain;
@@ -53,7 +54,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
     if (paths && (net.npthlev < 1 || net.npthlev > 64)) return false;
     const int per_wave = paths ? 64 / net.npthlev : 0;             // paths of a wavefront
     const int max_paths = paths ? std::min(blk_paths(T), per_wave * (T / 64)) : 0;
-    const int cap = paths ? std::max(8, T / 32) : std::max(T / 4, T - 48 * kmax);
+    const int cap = paths ? std::max(8, T / 8) : std::max(T / 4, T - 48 * kmax);
     std::vector<int32_t> total((size_t)n, 1), resid((size_t)n), piece((size_t)n);
     std::vector<uint8_t> root((size_t)n, 0);
     for (int p = 0; p < n; ++p) {
@@ -190,6 +191,17 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
                 each_path(x, [&](int y, int) { to(y); });
             }
         };
+        auto take = [&](int i) {
+            in[(size_t)i] = 1;
+            took.push_back(i);
+            each_link(i, [&](int c) {
+                if (seen[(size_t)c] != blk) { seen[(size_t)c] = blk; links[(size_t)c] = 0; }
+                links[(size_t)c] += 1;
+                near.push({(float)links[(size_t)c] / (float)size_of(c), c});
+            });
+        };
+        std::vector<int32_t> best;
+        std::vector<uint8_t> best_codes;
         for (int left = npc; left > 0; ++blk) {
             took.clear();
             grown.clear();
@@ -212,14 +224,8 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
                         if (!in[(size_t)f]) i = f;
                         else if (f == first) ++first;
                     if (!grown.empty() && (int)grown.size() + size_of(i) > T) break;
-                    in[(size_t)i] = 1;
-                    took.push_back(i);
                     grown.insert(grown.end(), own.begin() + off[(size_t)i], own.begin() + off[(size_t)i + 1]);
-                    each_link(i, [&](int c) {
-                        if (seen[(size_t)c] != blk) { seen[(size_t)c] = blk; links[(size_t)c] = 0; }
-                        links[(size_t)c] += 1;
-                        near.push({(float)links[(size_t)c] / (float)size_of(c), c});
-                    });
+                    take(i);
                 }
                 cur = grown;
                 surround();
@@ -229,6 +235,33 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
                 const bool full = left == (int)took.size() || cur.size() > 0.96 * T || tries >= 4 || shrunk ||
                                   pc.spec > 0.9 * max_spec || pc.dams > 0.9 * max_dams || pc.paths > 0.94 * max_paths;
                 if (ok && full) {
+                    // small pieces into the room that is left
+                    for (int more = 0; more < 6 && !near.empty(); ++more) {
+                        const int room = T - pc.size;
+                        int i = -1;
+                        while (!near.empty() && i < 0 && room > T / 64) {
+                            const int c = near.top().second;
+                            near.pop();
+                            if (!in[(size_t)c] && 4 * size_of(c) <= 3 * room) i = c;
+                        }
+                        if (i < 0) break;
+                        best.swap(cur);
+                        best_codes.swap(curc);
+                        const size_t had = grown.size();
+                        grown.insert(grown.end(), own.begin() + off[(size_t)i], own.begin() + off[(size_t)i + 1]);
+                        cur = grown;
+                        surround();
+                        Piece with = piece_of(cur, 0, (int)cur.size());
+                        with.paths = count_paths();
+                        if (fits(with)) {
+                            pc = with;
+                            take(i);
+                        } else {
+                            grown.resize(had);
+                            cur.swap(best);
+                            curc.swap(best_codes);
+                        }
+                    }
                     share = std::max(0.1, std::min(1.0, (double)grown.size() / T));
                     keep(pc, (int)grown.size());
                     break;

@@ -1228,14 +1228,14 @@ std::vector<BlockShape> block_shapes(int64_t ns, int ninst, bool mixed) {
 //  * whole groups of basins: 938 cells, all options, 8 substeps, FP64: T = 256 186 us
 //    (T = 512 201, 1024 239; three-phase 319)
 //  * 15,001 cells, 1,000 paths, levees and dams, 222 substeps, FP64: kmax 6 3.1 ms (kmax
-//    4 3.3, 3 3.6; T = 256, kmax 2 3.6; T = 1024, kmax 4 4.5; three-phase 6.1)
-//  * 60,005 cells, 5,000 paths, 893 substeps, FP64: kmax 4 11.7 ms (kmax 3 12.5, 2 14.2;
+//    4 3.4; T = 256, kmax 3 3.7; T = 1024, kmax 4 4.5; three-phase 6.1)
+//  * 60,005 cells, 5,000 paths, 893 substeps, FP64: kmax 4 11.9 ms (kmax 3 12.7, 2 14.2;
 //    T = 1024, kmax 6 14.7; three-phase 24.9)
-//  * 240,019 cells, 20,000 paths, 2163 substeps: FP64 kmax 3 74.4 ms (kmax 2 77.2, 1
-//    110.3; T = 1024, kmax 4 75.1, 1 80.2; T = 256, kmax 2 78.1; three-phase 110.1); mixed
-//    54.0 (kmax 2 53.9; T = 1024, kmax 4 61.1; three-phase 96.4)
-//  * 583,000 cells, 50,000 paths, 1202 substeps: FP64 98.5 (T = 1024, kmax 3 97.0;
-//    three-phase 130.2); mixed 66.1 (kmax 2 67.4; T = 1024 78.2; three-phase 103.1)
+//  * 240,019 cells, 20,000 paths, 2163 substeps: FP64 kmax 3 67.8 ms (kmax 4 71.6, 2 77.1,
+//    1 80.0; T = 1024, kmax 4 74.1, 1 80.2; T = 256, kmax 2 78.1; three-phase 110.1);
+//    mixed 46.5 (kmax 4 52.4, 2 53.2; T = 1024, kmax 4 60.5; three-phase 96.4)
+//  * 583,000 cells, 50,000 paths, 1202 substeps: FP64 92.3 (kmax 2 99.4; T = 1024, kmax 3
+//    97.0; three-phase 130.2); mixed 61.6 (kmax 2 65.8; T = 1024 77.4; three-phase 103.1)
 std::vector<BlockShape> path_shapes(int n) {
     const int any = 0x7fffffff;
     std::vector<BlockShape> v;
