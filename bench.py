@@ -33,7 +33,8 @@ BYTES_MIXED = {"outflow": 96.0, "rate": 24.0, "update": 156.0}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "traffic_c3.json")
 # launch configuration of the single-model C3 runs: the one profiles/traffic_c3.* was
 # measured with (the autotuner's usual choice on this workload), so roofline.traffic
-# describes the launches that are timed
+# describes the phase kernels of the roofline's own pass; the timed steps of this
+# workload run block launches, which read none of it
 PINNED_TUNE = '{"bs_outflow":64,"bs_rate":256,"bs_update":128,"xcd":1}'
 
 
@@ -104,7 +105,8 @@ def run_gpu(net, m, rvec, precision, steps, warmup, dt, tune="auto"):
         gm.synchronize()
         t_total += time.perf_counter() - t0
         sum_nt += nt
-    # kernel timing pass (HIP events on the model's stream)
+    # kernel timing pass (HIP events on the model's stream): times the three phase
+    # kernels one by one; the steps above ran block launches, several substeps each
     gm.kernel_times(True)
     gm.set_runoff(rvec[rec % len(rvec)])
     gm.physics_advance(dt)

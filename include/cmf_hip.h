@@ -342,7 +342,9 @@ int cmf_hip_instance_times(cmf_handle h, double* ms);
  * kernel of grid_fused blocks (0 = all co-resident blocks) of bs_fused threads;
  * xcd = 1 gives each XCD a contiguous range of tiles; graph = 1 replays the
  * substep launches of an outer step from a captured HIP graph (phase kernels
- * only). The configuration changes no state value, only the rounding of the
+ * only). The block sizes are those of the three phase kernels; most single models
+ * and ensembles of up to 16 members step in block launches instead, unless fused or
+ * graph is set. The configuration changes no state value, only the rounding of the
  * logged budget sums. */
 typedef struct cmf_tune {
     int32_t bs_outflow, bs_rate, bs_update, fused, bs_fused, grid_fused, xcd, graph;
@@ -365,7 +367,8 @@ int cmf_hip_synchronize(cmf_handle h);
 /* Duration in milliseconds of the dominant substep kernels over the last
  * advance, measured with HIP events on the handle's stream (diagnostics for
  * benchmarking; no reference counterpart). out[0]=outflow, [1]=rate,
- * [2]=update(stage), [3]=stage+CFL, [4]=number of substeps timed. */
+ * [2]=update(stage), [3]=stage+CFL, [4]=number of substeps timed. While enabled,
+ * every model runs the three phase kernels. */
 int cmf_hip_kernel_times(cmf_handle h, int32_t enable, double* out5);
 
 #ifdef __cplusplus
