@@ -112,6 +112,7 @@ HIP_FUNCS = {
     "cmf_hip_instance_times": (I, [H, P]),
     "cmf_hip_get_dt_min": (I, [H, P]),
     "cmf_hip_instance_storage": (I, [H, P]),
+    "cmf_hip_block_info": (I, [H, P]),
     "cmf_hip_set_tune": (I, [H, C.POINTER(cmf_tune)]),
     "cmf_hip_get_tune": (I, [H, C.POINTER(cmf_tune)]),
     "cmf_hip_autotune": (I, [H, C.c_double, C.c_int32, C.POINTER(cmf_tune), P, C.c_int32]),

@@ -376,6 +376,13 @@ class CMFModel:
         self._check(self.lib.cmf_hip_instance_times(self.h, out.ctypes.data))
         return out
 
+    def block_info(self) -> dict:
+        """Block launches of the last advance (0: the phase kernels) and the partition
+        they use (cells 0: none)."""
+        out = np.zeros(6, np.int32)
+        self._check(self.lib.cmf_hip_block_info(self.h, out.ctypes.data))
+        return dict(zip(("launches", "cells", "substeps", "blocks", "closed", "paths"), out.tolist()))
+
     def set_tune(self, **kw) -> dict:
         t = self.get_tune()
         t.update(kw)

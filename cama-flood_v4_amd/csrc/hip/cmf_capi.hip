@@ -120,6 +120,7 @@ struct cmf_hip_ctx {
     // several substeps per launch (cmf_block.hip): the device copy of the partition
     // (nblk = 0: none) and the second set of the arrays its launches hand on
     BlockTab block{};
+    int32_t block_runs = 0;           // block launches of the last advance (0: the phase kernels)
     BlockState<double> alt64{};
     BlockState<float> alt32{};
     // launch configuration
@@ -844,6 +845,7 @@ int enqueue_blocks(cmf_hip_ctx* h, DevState<R>& S, int32_t ntmax, bool vel_first
         }
         const R* vel0 = vel_first ? (const R*)h->vel_buf : nullptr;
         HIPCHK(launch_block<R>(h->M, Sk, P.closed || (j & 1) ? home : alt, P, A, h->h_inst[0], j, vel0, h->stream));
+        ++h->block_runs;
     }
     return 0;
 }
@@ -911,6 +913,7 @@ int advance_t(cmf_hip_ctx* h, double dt_def, int32_t nt_cap, int32_t* nt_out, do
     const int ntiles = blocks ? h->block.nblk : tiles_cells(h->M, upd_bs(h));
     if (A.budget) TRY(grow_partials<R>(h, S, ntmax, ntiles));
     const bool vel_first = h->vel_pending;
+    h->block_runs = 0;
     if (blocks) {
         TRY(enqueue_blocks<R>(h, S, ntmax, vel_first));
     } else if (h->tune.graph && !h->tune.fused && !h->timing && !vel_first) {
@@ -1016,6 +1019,7 @@ int advance_noalloc_t(cmf_hip_ctx* h, double dt_def, int32_t* nt_out, double* gl
     HIPCHK(hipMemcpyAsync(h->d_inst, h->h_inst, sizeof(InstStep), hipMemcpyHostToDevice, h->stream));
     const int ntc = tiles_cells(h->M, h->tune.bs_update);
     const bool vel_first = h->vel_pending;
+    h->block_runs = 0;
     for (int32_t it = 0; it < ntmax; ++it) {
         A.it = it;
         A.prow = 0;
@@ -2354,6 +2358,18 @@ int cmf_hip_instance_times(cmf_handle h, double* ms) {
     if (!h || !ms) return fail(CMF_EINVAL, "NULL argument");
     if (h->inst_ms.size() != (size_t)h->ninst) return fail(CMF_ESTATE, "no timed advance yet");
     for (int k = 0; k < h->ninst; ++k) ms[k] = h->inst_ms[(size_t)k];
+    return 0;
+}
+
+int cmf_hip_block_info(cmf_handle h, int32_t* out6) {
+    if (!h || !out6) return fail(CMF_EINVAL, "NULL argument");
+    const BlockTab& P = h->block;
+    out6[0] = h->block_runs;
+    out6[1] = P.nblk > 0 ? P.T : 0;
+    out6[2] = P.nblk > 0 ? P.kmax : 0;
+    out6[3] = P.nblk;
+    out6[4] = P.nblk > 0 && P.closed;
+    out6[5] = P.nblk > 0 && P.npth > 0;
     return 0;
 }
 

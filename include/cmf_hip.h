@@ -337,6 +337,13 @@ int cmf_hip_instance_storage(cmf_handle h, double* out);
  * the end of the last substep of each instance (ms[ndom*members]). */
 int cmf_hip_instance_times(cmf_handle h, double* ms);
 
+/* How the handle's substeps run (diagnostics; no reference counterpart): out6[0] =
+ * block launches of the last advance, 0 where it ran the three phase kernels (or the
+ * fused one); the partition of the network made by cmf_hip_set_map, all 0 without one:
+ * [1] cells per block, [2] substeps per launch, [3] blocks, [4] 1 if no block holds a
+ * cell of another (all substeps in one launch), [5] 1 if it follows bifurcation paths. */
+int cmf_hip_block_info(cmf_handle h, int32_t* out6);
+
 /* Launch configuration (no reference counterpart). Block sizes 64/128/256/512
  * per substep phase; fused = 1 runs a substep as one persistent cooperative
  * kernel of grid_fused blocks (0 = all co-resident blocks) of bs_fused threads;
