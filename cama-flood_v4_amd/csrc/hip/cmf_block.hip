@@ -1085,9 +1085,9 @@ template <class R>
 hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<R>& O, const BlockTab& P,
                         const StepArgs& A, const InstStep& I, int j, const R* vel0, hipStream_t st) {
     const BlockArgs<R> a{M, S, O, P, A, I, j, vel0};
+    if (j == 0 && P.ndead > 0)                                       // also where every path is dead
+        hipLaunchKernelGGL((k_dead_paths<R>), dim3((P.ndead + 255) / 256), dim3(256), 0, st, M, S, P.dead, P.ndead);
     if (P.npth > 0) {
-        if (j == 0 && P.ndead > 0)
-            hipLaunchKernelGGL((k_dead_paths<R>), dim3((P.ndead + 255) / 256), dim3(256), 0, st, M, S, P.dead, P.ndead);
         switch (P.T) {
             case 256: return launch_block_t<R, 256, false, true>(a, st);
             case 512: return launch_block_t<R, 512, false, true>(a, st);

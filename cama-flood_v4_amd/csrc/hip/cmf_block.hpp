@@ -75,7 +75,7 @@ struct BlockTab {
     const uint16_t* upx;
     const int32_t* ndam;
     const int32_t* dom;
-    int npth;                                  // > 0: with paths
+    int npth;                                  // > 0: blocks along paths with both ends in the network
     const int32_t* path;
     const uint32_t *pword, *pends, *pcell;
     const int32_t* ppx_ptr;

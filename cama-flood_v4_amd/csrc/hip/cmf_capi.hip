@@ -1323,7 +1323,7 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
         TRY(put_raw(h, &pd, pc.data(), pc.size())); P.pconst = pd;
         P.npth = np;
     }
-    std::vector<int32_t> dead;                            // no block holds these (none may, with no live path)
+    std::vector<int32_t> dead;                            // no block holds these
     for (int q = 0; h->o.lpthout && q < h->d.npthout; ++q)
         if (pth.up[(size_t)q] < 0 || pth.down[(size_t)q] < 0) dead.push_back(q);
     P.ndead = (int)dead.size();
@@ -1622,7 +1622,7 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         TRY(put_raw(h, &p32, iptr.data(), iptr.size())); M.pinf_ptr = p32;
         TRY(put_raw(h, &p32, iidx.data(), iidx.size())); M.pinf_idx = p32;
         if (h->ndom > 1) { TRY(put_raw(h, &p32, pdom.data(), (size_t)np)); M.pth_dom = p32; }
-        bpth = BlockPaths{pu, pdn, optr, oidx, iptr, iidx, (int)oidx.size()};
+        bpth = BlockPaths{pu, pdn, optr, oidx, iptr, iidx, (int)oi.size()};
         TRY(put_raw(h, &pd, mp->pth_dst, (size_t)np)); M.pth_dst = pd;
         TRY(put_raw(h, &pd, mp->pth_elv, (size_t)np * nlv)); M.pth_elv = pd;
         TRY(put_raw(h, &pd, mp->pth_wth, (size_t)np * nlv)); M.pth_wth = pd;
