@@ -672,7 +672,6 @@ struct cmf_mlp {
     uint16_t *xt = nullptr, *ht[3] = {nullptr, nullptr, nullptr};
     uint16_t* gt[4] = {nullptr, nullptr, nullptr, nullptr};
     float* gsplit = nullptr;               // split weight gradients
-    int nsplit_cap = 0;
     float* xd = nullptr;                   // FP32 inputs of a host call
     cmf::Pinned fwd_pin;                   // slots of the chunked inference: x and y; x on the device
     float* fwd_x = nullptr;
@@ -767,24 +766,50 @@ void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, flo
                            x, rows, y);
 }
 
+// slots of the chunked inference: rows of x and y in pinned memory, x on the device
+constexpr int FWD_ROWS = 16384, FWD_STREAMS = 4;
+int grow_forward(cmf_mlp* h, int slots) {
+    if (slots <= h->fwd_slots) return 0;
+    const size_t nx = (size_t)FWD_ROWS * h->n_in, ny = (size_t)FWD_ROWS * h->n_out;
+    MCHK(h->fwd_pin.grow((size_t)slots * (nx + ny) * sizeof(float)));
+    float* q = nullptr;
+    MTRY(malloc_t(h, &q, (size_t)slots * nx));
+    if (h->fwd_x) {
+        (void)hipFree(h->fwd_x);
+        for (size_t k = 0; k < h->allocs.size(); ++k)
+            if (h->allocs[k] == (void*)h->fwd_x) { h->allocs.erase(h->allocs.begin() + (long)k); break; }
+    }
+    h->fwd_x = q;
+    h->fwd_slots = slots;
+    return 0;
+}
+
 int dw_splits(int rows) {
-    const int ns = (rows + DW_ROWS - 1) / DW_ROWS;
+    const int ns = (rows - 1) / DW_ROWS + 1;
     return ns < 64 ? ns : 64;
+}
+
+// Buffers of the fused kernels, all of them with the handle: made in the first gradient,
+// a failed allocation left some of them to the next call, and that gradient, of 64 rows,
+// took 0.25 ms with max_batch 1,024 and 0.9 ms with 65,536 (0.07 ms now)
+int alloc_fused(cmf_mlp* h) {
+    // whole tiles, and an odd number of 256-byte pieces a row: with a power of two the
+    // same rows of all features would meet in one or two L2 channels
+    size_t ld = ((size_t)h->max_batch + 127) & ~(size_t)127;
+    if (ld / 128 % 2 == 0) ld += 128;
+    for (auto& q : h->ht) MTRY(malloc_t(h, &q, FH * ld));
+    for (int l = 0; l < 4; ++l) MTRY(malloc_t(h, &h->gt[l], (l == 3 ? FNO : FH) * ld));
+    MTRY(malloc_t(h, &h->xt, FKI * ld));
+    if (ld > 0x7fffffff) return mfail(CMF_MLP_EINVAL, "max_batch too large");
+    h->ld = (int)ld;
+    const int ns = dw_splits(h->max_batch);
+    if (ns > 1) MTRY(malloc_t(h, &h->gsplit, (size_t)ns * (size_t)h->np));
+    return grow_forward(h, 1);
 }
 
 // forward and backward of a batch by the fused kernels; gradients into h->g, loss
 // partial sums into part. x, t: device arrays, rows picked by idx (NULL: in order)
 int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, int rows, float* part) {
-    if (!h->xt) {
-        // whole tiles, and an odd number of 256-byte pieces a row: with a power of two the
-        // same rows of all features would meet in one or two L2 channels
-        h->ld = (h->max_batch + 127) & ~127;
-        if (h->ld / 128 % 2 == 0) h->ld += 128;
-        const size_t ld = (size_t)h->ld;
-        MTRY(malloc_t(h, &h->xt, FKI * ld));
-        for (auto& q : h->ht) MTRY(malloc_t(h, &q, FH * ld));
-        for (int l = 0; l < 4; ++l) MTRY(malloc_t(h, &h->gt[l], (l == 3 ? FNO : FH) * ld));
-    }
     FusedTrain G{};
     G.t = t; G.idx = idx; G.w_over = h->w_over; G.y = h->y;
     G.xt = h->xt; G.ld = h->ld;
@@ -792,10 +817,6 @@ int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, i
     for (int l = 0; l < 4; ++l) G.gt[l] = h->gt[l];
     const int ns = dw_splits(rows);
     const int per = ((rows + ns - 1) / ns + 31) & ~31;
-    if (ns > 1 && ns > h->nsplit_cap) {
-        h->nsplit_cap = dw_splits(h->max_batch);
-        MTRY(malloc_t(h, &h->gsplit, (size_t)h->nsplit_cap * (size_t)h->np));
-    }
     launch_fused<true>(h, G, x, rows, h->y, h->stream);
     const unsigned nb = DW_TILES + (unsigned)((3 * FH + h->n_out + 1) / 2) + (unsigned)loss_parts(h, rows);
     float* dst = ns > 1 ? h->gsplit : h->g;
@@ -814,24 +835,12 @@ int fused_grad(cmf_mlp* h, const float* x, const float* t, const int64_t* idx, i
 // PCIe (96 bytes a row): 1,500,120 rows 2.9 ms, 51 GB/s (one pageable copy, kernel and
 // copy back after another 7.1; chunks of 8,192 rows 3.9, of 4,096 6.2: the launches of
 // a chunk cost about 20 us).
-constexpr int FWD_ROWS = 16384, FWD_STREAMS = 4;
 int forward_fused(cmf_mlp* h, const float* x, int64_t n, float* y) {
     const int64_t nc = (n + FWD_ROWS - 1) / FWD_ROWS;
     if (nc > 0x7fffffff) return mfail(CMF_MLP_EINVAL, "too many rows");
     const int slots = (int)std::min<int64_t>(nc, cmf::XFER_SLOTS);
     const size_t nx = (size_t)FWD_ROWS * h->n_in, ny = (size_t)FWD_ROWS * h->n_out;
-    if (slots > h->fwd_slots) {
-        MCHK(h->fwd_pin.grow((size_t)slots * (nx + ny) * sizeof(float)));
-        float* q = nullptr;
-        MTRY(malloc_t(h, &q, (size_t)slots * nx));
-        if (h->fwd_x) {
-            (void)hipFree(h->fwd_x);
-            for (size_t k = 0; k < h->allocs.size(); ++k)
-                if (h->allocs[k] == (void*)h->fwd_x) { h->allocs.erase(h->allocs.begin() + (long)k); break; }
-        }
-        h->fwd_x = q;
-        h->fwd_slots = slots;
-    }
+    MTRY(grow_forward(h, slots));
     float* const pin = reinterpret_cast<float*>(h->fwd_pin.p);
     auto rows_of = [n](int64_t c) { return (int)std::min<int64_t>(FWD_ROWS, n - c * FWD_ROWS); };
     auto start_on = [&](int c, int slot, hipStream_t st) -> hipError_t {
@@ -959,6 +968,7 @@ int cmf_mlp_create(int32_t n_in, int32_t hidden, int32_t n_out, int32_t max_batc
     if (!rc) rc = malloc_t(h, &h->y, B * n_out);
     if (!rc) rc = malloc_t(h, &h->t, B * n_out);
     if (!rc) rc = malloc_t(h, &h->part, (B * n_out + 255) / 256);
+    if (!rc) rc = malloc_t(h, &h->xd, B * n_in);
     if (!rc && !h->fused) {                                         // batch buffers of the layer kernels
         if ((rc = malloc_t(h, &h->xb, B * n_in)) || (rc = malloc_t(h, &h->hb[0], B * H)) ||
             (rc = malloc_t(h, &h->hb[1], B * H)) || (rc = malloc_t(h, &h->hb[2], B * H)) ||
@@ -975,6 +985,7 @@ int cmf_mlp_create(int32_t n_in, int32_t hidden, int32_t n_out, int32_t max_batc
         if (!rc) rc = malloc_t(h, &h->off, 8);
         if (!rc && hipMemcpy(h->off, o, sizeof o, hipMemcpyHostToDevice) != hipSuccess)
             rc = mfail(CMF_MLP_EHIP, "hipMemcpy failed");
+        if (!rc) rc = alloc_fused(h);
     }
     if (rc) {
         std::string keep = m_err;
@@ -1032,7 +1043,6 @@ int cmf_mlp_get_params(cmf_mlp_handle h, float* params, float* grads) {
 int cmf_mlp_forward(cmf_mlp_handle h, const float* x, int64_t n, float* y) {
     if (!h || !x || !y || n < 0) return mfail(CMF_MLP_EINVAL, "bad argument");
     if (h->fused) return n > 0 ? forward_fused(h, x, n, y) : 0;
-    if (!h->xd) MTRY(malloc_t(h, &h->xd, (size_t)h->max_batch * h->n_in));
     for (int64_t r0 = 0; r0 < n; r0 += h->max_batch) {
         const int rows = (int)((n - r0) < h->max_batch ? (n - r0) : h->max_batch);
         MCHK(hipMemcpyAsync(h->xd, x + (size_t)r0 * h->n_in, (size_t)rows * h->n_in * sizeof(float),
@@ -1050,7 +1060,6 @@ int cmf_mlp_forward(cmf_mlp_handle h, const float* x, int64_t n, float* y) {
 
 int cmf_mlp_grad(cmf_mlp_handle h, const float* x, const float* t, int32_t rows, float* loss) {
     if (!h || !x || !t || rows <= 0 || rows > h->max_batch) return mfail(CMF_MLP_EINVAL, "bad argument");
-    if (!h->xd) MTRY(malloc_t(h, &h->xd, (size_t)h->max_batch * h->n_in));
     MCHK(hipMemcpyAsync(h->xd, x, (size_t)rows * h->n_in * sizeof(float), hipMemcpyHostToDevice, h->stream));
     MCHK(hipMemcpyAsync(h->t, t, (size_t)rows * h->n_out * sizeof(float), hipMemcpyHostToDevice, h->stream));
     int rc = 0;
