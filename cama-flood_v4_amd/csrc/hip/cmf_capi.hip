@@ -1109,8 +1109,8 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
         ++nrep;
         return 0;
     };
-    cmf_tune bt = keep;
-    double best_total = 1e300;
+    cmf_tune bt = keep, bf{};                     // best of the phase kernels, and of the persistent one
+    double best_total = 1e300, best_fused = 1e300;
     for (int xcd = 0; xcd < 2; ++xcd) {
         // per-phase block sizes: every phase is its own kernel, so each takes its best
         double bph[3] = {1e300, 1e300, 1e300};
@@ -1128,7 +1128,7 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
             best_total = tot;
             bt = cmf_tune{};
             bt.bs_outflow = bbs[0]; bt.bs_rate = bbs[1]; bt.bs_update = bbs[2];
-            bt.bs_fused = 256; bt.xcd = xcd; bt.fused = 0; bt.graph = keep.graph;
+            bt.bs_fused = 256; bt.xcd = xcd; bt.fused = 0; bt.graph = 0;
         }
         for (int bs : {256, 512}) {
             cmf_tune t{};
@@ -1141,38 +1141,47 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
             if (t.grid_fused <= 0) t.grid_fused = cap;
             double ph[3], totf;
             TRY(trial(t, ph, &totf));
-            if (totf < best_total) { best_total = totf; bt = t; bt.graph = 0; }
+            if (totf < best_fused) { best_fused = totf; bf = t; }
         }
     }
-    // graph replay of the substep launches changes only the launch overhead, which
-    // the kernel events do not see: time the whole capped outer step by wall clock
-    // with and without it (the first call of a configuration captures the graph)
-    if (!bt.fused) {
-        double wall[2] = {0.0, 0.0};
-        for (int g = 0; g < 2; ++g) {
-            cmf_tune t = bt;
-            t.graph = g;
-            h->tune = t;
-            h->timing = false;
-            drop_graphs(h);
-            for (int rep = 0; rep < 2; ++rep) {
-                restore_ptrs(); h->vel_pending = keep_vel; h->fld_pending = keep_fld; h->pth_pending = keep_pth;
-                TRY(snapshot(h, true));
-                const auto c0 = std::chrono::steady_clock::now();
-                TRY(advance_t<R>(h, dt_def, nsub, nullptr, nullptr, nullptr, 0));
-                const auto c1 = std::chrono::steady_clock::now();
-                wall[g] = std::chrono::duration<double, std::milli>(c1 - c0).count();
-            }
-            if (report && nrep < report_cap) {
-                double* r = report + (size_t)nrep * 8;
-                r[0] = 2 + g; r[1] = bt.bs_update; r[2] = bt.xcd; r[3] = 0;
-                r[4] = r[5] = r[6] = 0.0; r[7] = wall[g];
-            }
-            ++nrep;
-        }
-        bt.graph = wall[1] < wall[0] ? 1 : 0;
+    // The kernel events above see neither launches nor block launches (timing runs the
+    // phase kernels). What remains is timed as whole capped outer steps by wall clock,
+    // the second of two calls (the first one captures the graph): the best phase kernels
+    // as they stand, which is block launches where the handle has a partition; their
+    // replay from a graph; and the persistent kernel where it beat them. Without a
+    // partition the kernel times decide on the persistent kernel. An open partition is
+    // timed over eight launches at least.
+    h->timing = false;
+    h->tune = bt;
+    const bool part = use_blocks(h, 2), fused = best_fused < best_total;
+    const int32_t nwall = part ? std::max(nsub, 8 * h->block.kmax) : nsub;
+    double best_wall = 1e300;
+    const cmf_tune phases = bt;
+    for (int g = 0; g < 3; ++g) {
+        if (fused && !part) { bt = bf; break; }
+        if (g == 2 && !fused) break;
+        cmf_tune t = g == 2 ? bf : phases;
+        t.graph = g == 1;
+        h->tune = t;
         drop_graphs(h);
+        double wall = 0.0;
+        for (int rep = 0; rep < 2; ++rep) {
+            restore_ptrs(); h->vel_pending = keep_vel; h->fld_pending = keep_fld; h->pth_pending = keep_pth;
+            TRY(snapshot(h, true));
+            const auto c0 = std::chrono::steady_clock::now();
+            TRY(advance_t<R>(h, dt_def, nwall, nullptr, nullptr, nullptr, 0));
+            const auto c1 = std::chrono::steady_clock::now();
+            wall = std::chrono::duration<double, std::milli>(c1 - c0).count();
+        }
+        if (report && nrep < report_cap) {
+            double* r = report + (size_t)nrep * 8;
+            r[0] = 2 + g; r[1] = g == 2 ? t.bs_fused : t.bs_update; r[2] = t.xcd; r[3] = t.grid_fused;
+            r[4] = r[5] = r[6] = 0.0; r[7] = wall;
+        }
+        ++nrep;
+        if (wall < best_wall) { best_wall = wall; bt = t; }
     }
+    drop_graphs(h);
     // restore the state and the caller's settings; keep the best configuration
     restore_ptrs();
     TRY(snapshot(h, true));

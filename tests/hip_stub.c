@@ -4,6 +4,7 @@
  * first. stub_fail makes single allocations fail. */
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 static long n_dev, n_pin, n_launch, n_live, fail_dev_from, fail_dev_to, fail_pin_from, fail_pin_to;
 
@@ -18,6 +19,9 @@ long stub_device_allocs(void) { return n_dev; }
 long stub_pinned_allocs(void) { return n_pin; }
 long stub_launches(void) { return n_launch; }
 long stub_live(void) { return n_live; }       /* allocations not yet freed */
+/* milliseconds that a cooperative launch and a graph take */
+static unsigned slow_ms;
+void stub_slow(unsigned ms) { slow_ms = ms; }
 
 enum { OK = 0, ENOMEM_HIP = 2 };
 static int take(void **p, size_t n, int fails) {
@@ -39,7 +43,7 @@ int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; memmove(d, s, 
 int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) { (void)st; return hipMemcpy(d, s, n, k); }
 int hipMemsetAsync(void *d, int v, size_t n, void *st) { (void)st; memset(d, v, n); return OK; }
 int hipLaunchKernel(const void *f, ...) { (void)f; ++n_launch; return OK; }
-int hipLaunchCooperativeKernel(const void *f, ...) { (void)f; ++n_launch; return OK; }
+int hipLaunchCooperativeKernel(const void *f, ...) { (void)f; ++n_launch; usleep(1000u * slow_ms); return OK; }
 int hipGetLastError(void) { return OK; }
 const char *hipGetErrorString(int e) { return e == OK ? "success" : "out of memory (stand-in)"; }
 int hipGetDevice(int *d) { *d = 0; return OK; }
@@ -66,3 +70,9 @@ int hipEventDestroy(void *e) { (void)e; return OK; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return OK; }
 int hipEventSynchronize(void *e) { (void)e; return OK; }
 int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 1.0f; return OK; }
+int hipStreamBeginCapture(void *s, int m) { (void)s; (void)m; return OK; }
+int hipStreamEndCapture(void *s, void **g) { (void)s; return handle_of(g); }
+int hipGraphInstantiate(void **x, void *g, void *n, char *log, size_t z) { (void)g; (void)n; (void)log; (void)z; return handle_of(x); }
+int hipGraphLaunch(void *x, void *s) { (void)x; (void)s; ++n_launch; usleep(1000u * slow_ms); return OK; }
+int hipGraphDestroy(void *g) { (void)g; return OK; }
+int hipGraphExecDestroy(void *x) { (void)x; return OK; }
