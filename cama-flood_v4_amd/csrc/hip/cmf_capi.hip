@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <type_traits>
 #include <utility>
@@ -1269,7 +1270,7 @@ struct BlockPaths {
 // partition of the network for block launches, its device copy and the second set
 // of the arrays the launches hand on
 template <class R>
-int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
+int make_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
                  const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
                  const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of, const BlockPaths& pth, const cmf_map* mp) {
     const int n = h->d.nseqall;
@@ -1342,10 +1343,7 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
         const size_t ns = ((size_t)h->M.ns + 63) / 64 * 64, nlev = h->o.llevee ? ns : 0, ndm = h->o.ldamout ? ns : 0;
         const size_t npl = paths ? ((size_t)h->d.npthout * h->d.npthlev + 63) / 64 * 64 : 0, nld = paths ? nlev : 0;
         double* d = nullptr;                              // the doubles, then the fields in R, which is no larger
-        if (dalloc(h, &d, 2 * ns + nlev + ndm + (7 * ns + npl + nld) * sizeof(R) / sizeof(double)) != 0) {
-            (void)hipGetLastError();                      // no memory for it: the three-phase kernels need none
-            return 0;
-        }
+        TRY(dalloc(h, &d, 2 * ns + nlev + ndm + (7 * ns + npl + nld) * sizeof(R) / sizeof(double)));
         auto dbl = [&](double*& p, size_t k) { p = d; d += k; };
         dbl(B.rivsto, ns); dbl(B.fldsto, ns); dbl(B.levsto, nlev); dbl(B.damsto, ndm);
         R* r = reinterpret_cast<R*>(d);
@@ -1358,6 +1356,25 @@ int setup_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::ve
     }
     P.nblk = bp.nblk;
     h->block = P;
+    return 0;
+}
+
+// The three-phase kernels need none of it: a model for which there is no memory left,
+// on the device or the host, keeps them.
+template <class R, class... Net>
+int setup_blocks(cmf_hip_ctx* h, const Net&... net) {
+    const size_t had = h->allocs.size();
+    int rc;
+    try {
+        rc = make_blocks<R>(h, net...);
+    } catch (const std::bad_alloc&) {
+        rc = CMF_ENOMEM;
+    }
+    if (rc != CMF_ENOMEM) return rc;
+    (void)hipGetLastError();
+    for (size_t k = had; k < h->allocs.size(); ++k) (void)hipFree(h->allocs[k]);
+    h->allocs.resize(had);
+    alt_of<R>(h) = BlockState<R>{};
     return 0;
 }
 
