@@ -116,6 +116,7 @@ struct cmf_hip_ctx {
     void* stage = nullptr;            // staging buffer of host <-> device cell-array transfers
     size_t stage_cap = 0;             // bytes
     Pinned xfer, hist;                // slots of device -> host transfers; S.glb_hist
+    double* hist_dev = nullptr;       // S.glb_hist on the device (no pinned memory), else NULL
     // host index of every device slot: cells (ns), path levels (npthlev*nsp), paths (nsp)
     std::vector<int64_t> hx_cell, hx_pthl, hx_pth;
     // several substeps per launch (cmf_block.hip): the device copy of the partition
@@ -174,6 +175,25 @@ int salloc(cmf_hip_ctx* h, T** p, size_t n, bool snap = true) {
     return 0;
 }
 
+// S.glb_hist for `rows` substeps: pinned memory, or where there is none to be had the
+// device's
+template <class R>
+int grow_hist(cmf_hip_ctx* h, DevState<R>& S, int rows) {
+    const size_t n = (size_t)rows * NGLB;
+    double* dev = nullptr;
+    if (h->hist.grow(n * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        TRY(dalloc(h, &dev, n));
+    }
+    if (h->hist_dev) {
+        (void)hipFree(h->hist_dev);
+        for (auto& a : h->allocs) if (a == (void*)h->hist_dev) a = nullptr;
+    }
+    h->hist_dev = dev;
+    S.glb_hist = dev ? dev : reinterpret_cast<double*>(h->hist.p);
+    return 0;
+}
+
 template <class R>
 int alloc_state(cmf_hip_ctx* h, DevState<R>& S) {
     const size_t ns = (size_t)h->d.nseqall * h->nmem;
@@ -206,8 +226,7 @@ int alloc_state(cmf_hip_ctx* h, DevState<R>& S) {
     S.partials = nullptr;
     // what the host reads after a step goes straight to pinned memory: the budget sums,
     // and the CFL minimum of a single model (one store; those of ensembles are atomic)
-    HIPCHK(h->hist.grow((size_t)h->hist_cap * NGLB * sizeof(double)));
-    S.glb_hist = reinterpret_cast<double*>(h->hist.p);
+    TRY(grow_hist(h, S, h->hist_cap));
     if (h->ninst == 1) S.cfl = h->h_cfl;
     else TRY(dalloc(h, &S.cfl, (size_t)h->ninst));
     TRY(dalloc(h, &S.cfl_part, (ns + 255) / 256));                // one value per stage block
@@ -323,21 +342,40 @@ struct Fetch {
         for (size_t k = 0; k < items.size(); ++k) off[k + 1] = off[k] + items[k].n;
         const size_t nc = (off.back() + FETCH_CHUNK - 1) / FETCH_CHUNK;
         if (nc > 0x7fffffff || items.size() > (size_t)FETCH_SEGS) return fail(CMF_EINVAL, "too many arrays in one call");
-        const size_t slots = std::min(nc, (size_t)XFER_SLOTS);
-        HIPCHK(h->xfer.grow((nc == 1 ? off.back() : slots * FETCH_CHUNK) * sizeof(double)));
-        double* const pin = reinterpret_cast<double*>(h->xfer.p);
-        auto start = [&](int c, int slot, hipEvent_t ev) -> hipError_t {
+        auto gather = [&](int c, double* dst) -> hipError_t {
             FetchArgs a;
             a.iperm = h->d_iperm;
             a.lgm = h->lgm;
-            a.dst = pin + (size_t)slot * FETCH_CHUNK;
+            a.dst = dst;
             int ns = 0;
             parts(off, (size_t)c, [&](const Item& it, size_t first, size_t count, size_t at) {
                 a.seg[ns++] = FetchSeg{it.src, (uint32_t)first, (uint32_t)count, (uint32_t)at,
                                        (uint32_t)plane_of(h, it.kind), it.kind == K_CELL, it.f32};
             });
             launch_fetch(a, ns, h->stream);
-            const hipError_t e = hipGetLastError();
+            return hipGetLastError();
+        };
+        const size_t slots = std::min(nc, (size_t)XFER_SLOTS);
+        if (h->xfer.grow((nc == 1 ? off.back() : slots * FETCH_CHUNK) * sizeof(double)) != hipSuccess) {
+            // no pinned memory: gathered on the device, then pageable copies
+            (void)hipGetLastError();
+            TRY(stage_bytes(h, std::min(off.back(), FETCH_CHUNK) * sizeof(double)));
+            double* const stage = static_cast<double*>(h->stage);
+            for (size_t c = 0; c < nc; ++c) {
+                HIPCHK(gather((int)c, stage));
+                hipError_t e = hipSuccess;
+                parts(off, c, [&](const Item& it, size_t first, size_t count, size_t at) {
+                    if (e == hipSuccess)
+                        e = hipMemcpyAsync(it.dst + first, stage + at, count * sizeof(double), hipMemcpyDeviceToHost, h->stream);
+                });
+                HIPCHK(e);
+                HIPCHK(hipStreamSynchronize(h->stream));
+            }
+            return 0;
+        }
+        double* const pin = reinterpret_cast<double*>(h->xfer.p);
+        auto start = [&](int c, int slot, hipEvent_t ev) -> hipError_t {
+            const hipError_t e = gather(c, pin + (size_t)slot * FETCH_CHUNK);
             return e != hipSuccess || !ev ? e : hipEventRecord(ev, h->stream);
         };
         auto finish = [&](int c, int slot) {
@@ -738,8 +776,7 @@ int grow_partials(cmf_hip_ctx* h, DevState<R>& S, int nrun, int ntiles) {
     if (nrun > h->hist_cap) {
         drop_graphs(h);
         const int cap = nrun + nrun / 4;
-        HIPCHK(h->hist.grow((size_t)cap * NGLB * sizeof(double)));
-        S.glb_hist = reinterpret_cast<double*>(h->hist.p);
+        TRY(grow_hist(h, S, cap));
         h->hist_cap = cap;
     }
     return 0;
@@ -931,9 +968,10 @@ int advance_t(cmf_hip_ctx* h, double dt_def, int32_t nt_cap, int32_t* nt_out, do
     h->pth_pending = false;
     if (h->tune.fused)
         HIPCHK(hipMemcpyAsync(h->h_ctl, S.err, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream));
+    const size_t rows = A.budget && glb && glb_cap > 0 ? (size_t)std::min(ntmax, glb_cap) * NGLB * sizeof(double) : 0;
+    if (rows && h->hist_dev) HIPCHK(hipMemcpyAsync(glb, S.glb_hist, rows, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    if (A.budget && glb && glb_cap > 0)
-        std::memcpy(glb, S.glb_hist, (size_t)std::min(ntmax, glb_cap) * NGLB * sizeof(double));
+    if (rows && !h->hist_dev) std::memcpy(glb, S.glb_hist, rows);
     if (h->tune.fused && *reinterpret_cast<int32_t*>(h->h_ctl) != 0) {
         // clear the flag and the barrier counters (arrival count, generation) so
         // that the next fused launch starts from a consistent barrier

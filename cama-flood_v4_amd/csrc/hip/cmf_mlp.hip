@@ -804,7 +804,8 @@ int alloc_fused(cmf_mlp* h) {
     h->ld = (int)ld;
     const int ns = dw_splits(h->max_batch);
     if (ns > 1) MTRY(malloc_t(h, &h->gsplit, (size_t)ns * (size_t)h->np));
-    return grow_forward(h, 1);
+    (void)grow_forward(h, 1);                             // inference can do without
+    return 0;
 }
 
 // forward and backward of a batch by the fused kernels; gradients into h->g, loss
@@ -840,7 +841,20 @@ int forward_fused(cmf_mlp* h, const float* x, int64_t n, float* y) {
     if (nc > 0x7fffffff) return mfail(CMF_MLP_EINVAL, "too many rows");
     const int slots = (int)std::min<int64_t>(nc, cmf::XFER_SLOTS);
     const size_t nx = (size_t)FWD_ROWS * h->n_in, ny = (size_t)FWD_ROWS * h->n_out;
-    MTRY(grow_forward(h, slots));
+    if (grow_forward(h, slots) != 0) {
+        // no pinned memory: pageable copies, one chunk after another
+        (void)hipGetLastError();
+        const int64_t most = std::min(FWD_ROWS, h->max_batch);
+        for (int64_t r0 = 0; r0 < n; r0 += most) {
+            const size_t rows = (size_t)std::min(most, n - r0);
+            MCHK(hipMemcpyAsync(h->xd, x + (size_t)r0 * h->n_in, rows * h->n_in * sizeof(float), hipMemcpyHostToDevice, h->stream));
+            launch_fused<false>(h, FusedTrain{}, h->xd, (int)rows, h->y, h->stream);
+            MCHK(hipGetLastError());
+            MCHK(hipMemcpyAsync(y + (size_t)r0 * h->n_out, h->y, rows * h->n_out * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+            MCHK(hipStreamSynchronize(h->stream));
+        }
+        return 0;
+    }
     float* const pin = reinterpret_cast<float*>(h->fwd_pin.p);
     auto rows_of = [n](int64_t c) { return (int)std::min<int64_t>(FWD_ROWS, n - c * FWD_ROWS); };
     auto start_on = [&](int c, int slot, hipStream_t st) -> hipError_t {

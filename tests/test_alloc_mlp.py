@@ -1,6 +1,7 @@
 """Allocations of the surrogate network (on the CPU, over the stand-in of the HIP
 runtime): cmf_mlp_create makes them all or fails whole, so no later call meets a handle
-with some of its buffers, or pays for buffers in its first pass."""
+with some of its buffers, or pays for buffers in its first pass. Inference can do
+without its pinned slot and the device's side of it."""
 import pytest
 
 import hip_stub
@@ -25,7 +26,10 @@ for k in range(1, ndev + npin + 1):
     else:
         stub.stub_fail(0, 0, k - ndev, k - ndev)
     try:
-        MLP(**kw).close()
+        g = MLP(**kw)
+        g.grad(x, t)
+        g.forward(np.repeat(x, 300, 0))
+        g.close()
         out["refused"].append(False)
     except SurrogateError:
         out["refused"].append(True)
@@ -38,5 +42,6 @@ result(out)
 def test_create_allocates_all(tmp_path, n_in, hidden, n_out):
     got = hip_stub.run(tmp_path, CODE % (n_in, hidden, n_out))
     assert got["first calls"] == [0, 0]
-    assert len(got["refused"]) > 15 and all(got["refused"])
+    assert len(got["refused"]) > 15
+    assert got["refused"].count(False) == (2 if hidden == 256 else 0)
     assert not any(got["left"])

@@ -1,5 +1,6 @@
 """Models for which some memory cannot be had (on the CPU, over the stand-in of the HIP
-runtime): the partition is optional, and nothing is left behind."""
+runtime): the partition is optional, pinned memory beyond that of cmf_hip_create is
+too, and nothing is left behind."""
 import pytest
 
 import hip_stub
@@ -7,7 +8,7 @@ import hip_stub
 CODE = """
 import block_forms
 from cmf.model import CMFError
-out = dict(made=[], left=[])
+out = dict(made=[], left=[], pinned=None)
 make = lambda: block_forms.model(%r, "fp64")
 g, st, ro = make()                                       # (builders use the stand-in once)
 g.close()
@@ -22,6 +23,15 @@ for k in range(1, stub.stub_device_allocs() + 1):
     except CMFError:
         out["made"].append(None)
     out["left"].append(stub.stub_live())
+stub.stub_fail(0, 0, 4, 10**9)                           # only the three of cmf_hip_create
+g = make()[0]
+g.set_state(st)
+g.set_runoff(ro)
+g.get_state()
+g.diag_avemax_output(3600.0)
+g.get_output()
+g.close()
+out["pinned"] = [stub.stub_pinned_allocs() > 4, stub.stub_live()]
 result(out)
 """
 
@@ -34,3 +44,4 @@ def test_partition_is_optional(tmp_path, form):
     assert made == [None] * first + [False] * (len(made) - first)
     assert first > 60 and len(made) - first >= (6 if form == "plain" else 7)
     assert not any(got["left"])
+    assert got["pinned"] == [True, 0]
