@@ -632,7 +632,7 @@ __global__ __launch_bounds__(T, sizeof(R) == 4 && T < 1024 ? 6 : 4) void k_block
         if (b >= args_.P.nblk) return;
     }
     const int nl = block_launches(nt, args_.P.kmax, args_.P.closed);
-    if (MB && args_.j >= nl) return;
+    if (MB && (nt < 1 || args_.j >= nl)) return;                          // done, or no substep to take
     const int it0 = (int)((long long)nt * args_.j / nl), nsub = (int)((long long)nt * (args_.j + 1) / nl) - it0;
     int g, s0;                                                            // cell, state slot
     uint32_t w0, w1;

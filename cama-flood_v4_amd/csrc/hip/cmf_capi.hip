@@ -858,7 +858,7 @@ BlockState<float>& alt_of<float>(cmf_hip_ctx* h) { return h->alt32; }
 // partition would take two launches that move the state for it.
 bool use_blocks(const cmf_hip_ctx* h, int32_t nt) {
     return h->block.nblk > 0 && !h->lkine && !h->lslpmix && (!h->o.ldamout || h->daminf_sparse) && !h->tune.graph &&
-           !h->tune.fused && !h->timing && (h->block.closed || nt >= 2);
+           !h->tune.fused && !h->timing && nt >= (h->block.closed ? 1 : 2);
 }
 
 // NT substeps as block launches. A closed partition takes all of them in one
