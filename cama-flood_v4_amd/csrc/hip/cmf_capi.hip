@@ -851,14 +851,44 @@ BlockState<double>& alt_of<double>(cmf_hip_ctx* h) { return h->alt64; }
 template <>
 BlockState<float>& alt_of<float>(cmf_hip_ctx* h) { return h->alt32; }
 
+// Substeps that a launch has to take on average for block launches to be the faster form.
+// A launch reads and writes the whole state once, which costs as much as 1.5 to 2
+// substeps of the phase kernels from the sizes on where the state leaves the caches,
+// and more with 8 and 16 members, of whose lines of memory a block uses an eighth or a
+// sixteenth at a time. Outer steps of 2, 3, 4 and 8 substeps, in us, phase kernels /
+// blocks (FP64 unless stated):
+//   one member      598,800 cells 259/234 344/267 433/303; 898,905 351/388 470/442 588/503;
+//                   1,499,736 553/661 757/759 961/855; 2,997,135 998/1266 1362/1456 1735/1648
+//   with paths      239,086 163/147 218/174; 578,889 276/286 376/328
+//   2 to 4 members  (slots) 238,140 114/104 148/113; 476,280 172/179 226/195;
+//                   1,905,120 479/631 661/671 844/732, mixed 312/435 408/462 507/505
+//   8               70,560 77/84 96/89; 476,280 170/227 220/238 270/257 475/338;
+//                   1,905,120 450/757 614/789 779/842 1462/1120, mixed 276/493 357/515 441/549 795/716
+//   16              141,120 91/124 114/132 138/137 234/178; 2,857,680 620/1310 848/1323 1088/1398 2049/1785,
+//                   mixed 421/932 562/978 710/1025 1305/1226, and of 12 (3 a launch) 1898/2065
+// A closed partition takes them in one launch: with 4 members and fewer at once as fast
+// (192,992 slots 71/71 for one substep); 8: 96,496 slots 60/67 82/73, 385,984 mixed
+// 76/102 106/111 136/121; 16: 192,992 69/93 96/100 123/111, 771,968 mixed 107/205
+// 153/217 203/234 250/250.
+double least_substeps(const cmf_hip_ctx* h) {
+    const int64_t ns = h->M.ns;
+    const int m = h->nmem;
+    if (h->block.closed) return m < 8 ? 1.0 : (m < 16 ? (ns <= 200000 ? 2.0 : 3.0) : (ns <= 400000 ? 3.0 : 5.0));
+    if (m >= 16) return ns <= 300000 ? 2.5 : (h->o.precision == CMF_PREC_FP64 ? 3.5 : 3.9);
+    if (m >= 8) return ns <= 150000 ? 1.5 : (ns <= 1000000 ? 2.0 : 3.0);
+    if (m > 1 || h->block.npth > 0) return ns <= 300000 ? 1.0 : (ns <= 750000 ? 1.5 : 2.0);
+    return ns <= 750000 ? 1.0 : (ns <= 2000000 ? 1.5 : 2.0);
+}
+
 // Whether an outer step of up to nt substeps runs as block launches: the handle has a
 // partition (setup_blocks), the scheme is the default one,
-// DAMINF is zero outside the dam cells, and no other form of the substep is asked
-// for (graph replay, the persistent kernel, per-phase timing). One substep of an open
-// partition would take two launches that move the state for it.
+// DAMINF is zero outside the dam cells, no other form of the substep is asked
+// for (graph replay, the persistent kernel, per-phase timing), and the launches take
+// enough substeps each.
 bool use_blocks(const cmf_hip_ctx* h, int32_t nt) {
     return h->block.nblk > 0 && !h->lkine && !h->lslpmix && (!h->o.ldamout || h->daminf_sparse) && !h->tune.graph &&
-           !h->tune.fused && !h->timing && nt >= (h->block.closed ? 1 : 2);
+           !h->tune.fused && !h->timing && nt >= (h->block.closed ? 1 : 2) &&
+           nt >= least_substeps(h) * block_launches(nt, h->block.kmax, h->block.closed);
 }
 
 // NT substeps as block launches. A closed partition takes all of them in one
@@ -1192,8 +1222,9 @@ int autotune_t(cmf_hip_ctx* h, double dt_def, int32_t nsub, cmf_tune* best, doub
     // timed over eight launches at least.
     h->timing = false;
     h->tune = bt;
-    const bool part = use_blocks(h, 2), fused = best_fused < best_total;
-    const int32_t nwall = part ? std::max(nsub, 8 * h->block.kmax) : nsub;
+    const int32_t many = std::max(nsub, 8 * h->block.kmax);
+    const bool part = use_blocks(h, many), fused = best_fused < best_total;
+    const int32_t nwall = part ? many : nsub;
     double best_wall = 1e300;
     const cmf_tune phases = bt;
     for (int g = 0; g < 3; ++g) {

@@ -27,8 +27,13 @@ def test_partitions(tmp_path):
             assert got[f"{form}/{prec}"] == (None if want is None else list(want)), (form, prec)
 
 
-def launches(part, nt):
-    if part is None or (nt < 2 and not part[2]):
+# a launch moves the whole state once: least substeps of a step in block launches, where
+# it is not one (closed partitions) or two
+LEAST = {"ens_rounds": 3, "ens_dam_16": 3}
+
+
+def launches(form, part, nt):
+    if part is None or nt < LEAST.get(form, 1 if part[2] else 2):
         return 0
     return 1 if part[2] else 2 * -(-nt // (2 * part[1]))
 
@@ -44,10 +49,10 @@ def test_steps_in_block_launches(form, prec):
     g.set_runoff(ro)
     step = g.ensemble_advance if g.ensemble else g.physics_advance
     assert g.block_info()["launches"] == 0
-    for cap in (1, 2, 13):
+    for cap in (1, 2, 3, 13):
         nt = step(86400.0, nt_cap=cap)
         nt = min(int(np.max(nt[0] if g.ensemble else nt)), cap)
-        assert g.block_info()["launches"] == launches(part, nt), cap
+        assert g.block_info()["launches"] == launches(form, part, nt), cap
     g.close()
 
 
@@ -78,4 +83,29 @@ def test_steps_left_to_the_phase_kernels():
         assert used() == 0
         switch(False)
     assert used() == 2
+    g.close()
+
+
+# the lines of the rule: (cells or domains, members, substeps a launch needs in FP64 and
+# in the mixed form); steps of nt substeps of an open partition take two launches per
+# 2*kmax of them
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("sizes, members, least", [
+    (600000, 1, (1, 1)), (900000, 1, (1.5, 1.5)), ([60000] * 2, 2, (1, 1)), ([60000] * 2, 4, (1.5, 1.5)),
+    ([9000], 8, (1.5, 1.5)), ([60000], 8, (2, 2)), ([9000], 16, (2.5, 2.5)), ([30000], 16, (3.5, 3.9)),
+    ([900] * 10, 8, (2, 2)), ([900] * 10, 16, (3, 3))])
+def test_short_steps_stay_on_the_phase_kernels(sizes, members, least, prec):
+    build = block_forms.regional if members == 1 else block_forms.ensemble
+    g, st, ro = build(sizes, 0.0, 0, prec) if members == 1 else build(sizes, members, 0.0, 0, prec)
+    _, kmax, closed, _ = block_forms.partition(g)
+    g.set_state(st)
+    g.set_runoff(ro)
+    step = g.ensemble_advance if g.ensemble else g.physics_advance
+    for cap in (1, 2, 3, 4, 5, 6, 8, 9, 16):
+        nt = step(86400.0, nt_cap=cap)
+        nt = min(int(np.max(nt[0] if g.ensemble else nt)), cap)
+        nl = 1 if closed else 2 * -(-nt // (2 * kmax))
+        want = nl if nt >= (1 if closed else 2) and nt / nl >= least[prec == "mixed"] else 0
+        assert g.block_info()["launches"] == want, cap
     g.close()
