@@ -241,18 +241,24 @@ __device__ __forceinline__ void outflow_cell(const DevMap& M, const DevState<R>&
         c.storge = storge;
         c.elevtn = f_elevtn; c.rivhgt = f_rivhgt; c.rivwth = f_rivwth; c.rivman = f_rivman;
         c.nxtdst = f_nxtdst; c.rivlen = f_rivlen;
-        c.river = river;
         c.dj = zero; c.dj_pre = zero;
+        Surface<R> sf;
+        // the surface inside the branch, so that its selects are resolved there (FP64:
+        // 1,499,736 cells 52.3 -> 47.3 us, 16 x 4 members of 59,535 128 -> 115)
         if (river) {
             const int sj = sidx<MB>(M, nxt, m);
+            c.river = true;
             c.zdn = rivelv_of(M, nxt);
             c.dj = S.rivdph[sj]; c.dj_pre = S.rivdph_pre[sj];
+            sf = surface_of<R>(c);
         } else {
+            c.river = false;
             c.zdn = M.dwnelv[i];
+            sf = surface_of<R>(c);
         }
-        const Surface<R> sf = surface_of<R>(c);
-        vel = river_vel<R>(c, sf);
+        c.river = river;
         local_inertial<R>(c, sf, A.lfldout, A.pmanfld, A.pdstmth, I.dt, I.gdt, q_r, q_f);
+        vel = river_vel<R>(c, sf);
     }
     // ---- reservoir operation: damout:316-498 (Yamazaki & Funato or Hanazaki-2022 rule)
     if (A.ldamout) {
