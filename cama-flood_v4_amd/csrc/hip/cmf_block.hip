@@ -24,6 +24,28 @@
 
 namespace cmf {
 
+// Whether every basin (total at its mouth), with the basins that paths join to it, is of
+// at most T cells: what a closed plan needs.
+static bool groups_fit(const BlockNet& net, const std::vector<int32_t>& total, int T) {
+    std::vector<int32_t> to((size_t)net.n), size(total);              // a mouth: the mouth it is joined to, or itself
+    for (int p = net.n - 1; p >= 0; --p) to[(size_t)p] = net.next[p] >= 0 ? to[(size_t)net.next[p]] : p;
+    auto mouth = [&](int p) {
+        p = to[(size_t)p];
+        while (to[(size_t)p] != p) p = to[(size_t)p] = to[(size_t)to[(size_t)p]];
+        return p;
+    };
+    for (int q = 0; q < net.npth; ++q) {
+        if (net.pth_up[q] < 0 || net.pth_down[q] < 0) continue;
+        const int a = mouth(net.pth_up[q]), b = mouth(net.pth_down[q]);
+        if (a == b) continue;
+        to[(size_t)b] = a;
+        size[(size_t)a] += size[(size_t)b];
+    }
+    for (int p = 0; p < net.n; ++p)
+        if (to[(size_t)p] == p && size[(size_t)p] > T) return false;
+    return true;
+}
+
 // ---------------------------------------------------------------------------
 // Partition. Cells come in depth-first order (every cell after its upstream
 // subtree). Basins of at most T cells stay whole; larger ones are cut bottom-up
@@ -44,7 +66,7 @@ namespace cmf {
 // 20,000 paths, 702 blocks of 512 load 1.42 times as many for kmax = 3 and compute 1.22
 // times as many outflows (pieces of T/32 cells 780 and 1.58; T/4 710 with more room
 // left; without the small pieces put into the room at the end 714).
-bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
+bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, int64_t max_blocks, BlockPlan& out) {
     const int n = net.n;
     const int32_t *next = net.next, *up_ptr = net.up_ptr, *up_idx = net.up_idx, *domain = net.domain;
     const uint8_t* special = net.special;
@@ -66,6 +88,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
     }
     // basin sizes, then the cuts
     for (int p = n - 1; p >= 0; --p) piece[(size_t)p] = next[p] >= 0 ? piece[(size_t)next[p]] : total[(size_t)p];
+    if (closed_only && !groups_fit(net, total, T)) return false;
     bool closed = true;
     for (int p = 0; p < n; ++p) {
         const int lim = !paths && piece[(size_t)p] <= T ? T : cap;
@@ -124,6 +147,8 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
         for (int k = net.out_ptr[x]; k < net.out_ptr[x + 1]; ++k) f(net.pth_down[net.out_idx[k]], net.out_idx[k]);
         for (int k = net.in_ptr[x]; k < net.in_ptr[x + 1]; ++k) f(net.pth_up[net.in_idx[k]], net.in_idx[k]);
     };
+    // more cells than max_blocks hold
+    auto too_many = [&] { return (int64_t)loc.size() > max_blocks * (int64_t)T; };
     // the surroundings of the owned cells in cur, with their codes
     auto surround = [&] {
         const int id = stamp++;
@@ -264,6 +289,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
                     }
                     share = std::max(0.1, std::min(1.0, (double)grown.size() / T));
                     keep(pc, (int)grown.size());
+                    if (too_many()) return false;
                     break;
                 }
                 if (ok) {                                           // room for more
@@ -310,6 +336,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
             const Piece pc = piece_of(cur, 0, (int)cur.size());
             if (fits(pc)) {
                 keep(pc, nown);
+                if (too_many()) return false;
                 continue;
             }
             if (nown < 2) return false;
@@ -395,6 +422,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out) {
     });
     for (size_t b = 0; b < bins.size(); ++b) out.dom[b] = done[(size_t)bins[b][0]].dom;
     const int nb = (int)bins.size();
+    if ((closed_only && !closed) || nb > max_blocks) return false;
     const size_t np = (size_t)nb * (size_t)T;
     out.T = T; out.kmax = kmax; out.nblk = nb; out.closed = closed;
     out.cell.assign(np, -1);

@@ -41,8 +41,9 @@ struct BlockNet {
     const int32_t *pth_up, *pth_down, *out_ptr, *out_idx, *in_ptr, *in_idx;
 };
 // False when the network cannot be cut into such blocks (a cell with too many
-// upstream cells, or whose surroundings alone overfill a block).
-bool build_block_plan(const BlockNet& net, int T, int kmax, BlockPlan& out);
+// upstream cells, or whose surroundings alone overfill a block), not into max_blocks of
+// them, or, with closed_only, not into blocks of whole basins; as soon as that is known.
+bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, int64_t max_blocks, BlockPlan& out);
 
 // Order of the cells of a block: dam cells from 0, kinematic cells (above a dam)
 // from BLK_KINE_AT, so that the two rare flow rules are computed by different

@@ -1362,8 +1362,7 @@ int make_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vec
     bool ok = false;
     for (const BlockShape& b : paths ? path_shapes(n)
                                      : block_shapes(h->M.ns, h->ninst, sizeof(R) == sizeof(float))) {
-        ok = build_block_plan(net, b.T, b.kmax, bp) &&
-             (bp.closed || !b.closed_only) && (int64_t)bp.nblk * h->nmem <= b.max_blocks;
+        ok = build_block_plan(net, b.T, b.kmax, b.closed_only, b.max_blocks / h->nmem, bp);
         // blocks hold cells of one domain: many small domains would leave them empty
         ok = ok && ((int64_t)bp.nblk * h->nmem <= 256 || (int64_t)bp.nblk * bp.T <= 2 * (int64_t)n);
         if (ok) break;
