@@ -1,6 +1,6 @@
 """Models for which some memory cannot be had (on the CPU, over the stand-in of the HIP
 runtime): the partition is optional, pinned memory beyond that of cmf_hip_create is
-too, and nothing is left behind."""
+too, and nothing is left behind. The slots of a state's transfer come with the map."""
 import pytest
 
 import hip_stub
@@ -11,6 +11,9 @@ from cmf.model import CMFError
 out = dict(made=[], left=[], pinned=None)
 make = lambda: block_forms.model(%r, "fp64")
 g, st, ro = make()                                       # (builders use the stand-in once)
+stub.stub_fail(0, 0, 0, 0)
+g.get_state()
+out["first get"] = [stub.stub_device_allocs(), stub.stub_pinned_allocs()]
 g.close()
 stub.stub_fail(0, 0, 0, 0)
 make()[0].close()
@@ -44,4 +47,5 @@ def test_partition_is_optional(tmp_path, form):
     assert made == [None] * first + [False] * (len(made) - first)
     assert first > 60 and len(made) - first >= (6 if form == "plain" else 7)
     assert not any(got["left"])
+    assert got["first get"] == [0, 0]
     assert got["pinned"] == [True, 0]
