@@ -1813,7 +1813,7 @@ int cmf_hip_instance_storage(cmf_handle h, double* out) {
         if (nch > maxch) nch = maxch;
         if (nch < 1) nch = 1;
         h->ist_nch = nch;
-        TRY(dalloc(h, &h->d_ist_part, (size_t)h->ninst * (size_t)nch));
+        if (!h->d_ist_part) TRY(dalloc(h, &h->d_ist_part, (size_t)h->ninst * (size_t)nch));
         TRY(dalloc(h, &h->d_ist_out, (size_t)h->ninst));
     }
     const double *rs, *fs, *ls;
@@ -1880,10 +1880,8 @@ int cmf_hip_set_runoff_scaled(cmf_handle h, const double* base_in, const double*
     const size_t n = (size_t)h->d.nseqall;
     Widen w(h);
     const double* base = w(base_in, n);
-    if (!h->d_rbase) {
-        TRY(dalloc(h, &h->d_rbase, n));
-        TRY(dalloc(h, &h->d_rfac, (size_t)h->ninst));
-    }
+    if (!h->d_rbase) TRY(dalloc(h, &h->d_rbase, n));
+    if (!h->d_rfac) TRY(dalloc(h, &h->d_rfac, (size_t)h->ninst));
     if (h->d_perm) {                                                     // to device cell order there
         TRY(stage_bytes(h, n * sizeof(double)));
         HIPCHK(hipMemcpyAsync(h->stage, base, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
@@ -1982,12 +1980,13 @@ namespace {
 int npth_slots(const cmf_hip_ctx* h) { return h->o.lpthout ? h->M.nsp * h->d.npthlev : 0; }
 
 int out_alloc(cmf_hip_ctx* h) {
-    if (h->out.rivout) return 0;
+    if (h->out.pthflw) return 0;                            // the last of them
     const size_t ns = (size_t)h->M.ns, np = (size_t)npth_slots(h);
     double** cell[] = {&h->out.rivout, &h->out.fldout, &h->out.outflw, &h->out.rivvel, &h->out.pthout,
                        &h->out.runoff, &h->out.daminf, &h->out.outflw_max, &h->out.rivdph_max,
                        &h->out.storge_max};
-    for (double** p : cell) TRY(dalloc(h, p, ns));          // dalloc clears
+    for (double** p : cell)
+        if (!*p) TRY(dalloc(h, p, ns));                     // dalloc clears
     TRY(dalloc(h, &h->out.pthflw, np));
     h->nadd_out = 0.0;
     return 0;
@@ -2021,7 +2020,7 @@ int cmf_hip_diag_avemax_output(cmf_handle h, double dt) {
 
 int cmf_hip_diag_getave_output(cmf_handle h, double* nadd_out) {
     if (!h) return fail(CMF_EINVAL, "NULL handle");
-    if (!h->out.rivout) return fail(CMF_ESTATE, "no output period: call cmf_hip_diag_avemax_output first");
+    if (!h->out.pthflw) return fail(CMF_ESTATE, "no output period: call cmf_hip_diag_avemax_output first");
     launch_out_getave(h->out, h->M.ns, npth_slots(h), h->nadd_out, h->o.ldamout, h->stream);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -2045,7 +2044,7 @@ int get_output_impl(cmf_hip_ctx* h, const cmf_output* o) {
 
 int cmf_hip_get_output(cmf_handle h, const cmf_output* o) {
     if (!h || !o) return fail(CMF_EINVAL, "NULL argument");
-    if (!h->out.rivout) return fail(CMF_ESTATE, "no output period: call cmf_hip_diag_avemax_output first");
+    if (!h->out.pthflw) return fail(CMF_ESTATE, "no output period: call cmf_hip_diag_avemax_output first");
     Narrow nw(h);
     cmf_output c = *o;
     const size_t ns = (size_t)h->M.ns;
@@ -2232,7 +2231,7 @@ int cmf_hip_output_write(cmf_handle h, const char* var, const char* file, int32_
     if ((v == "damsto" || v == "daminf") && !h->o.ldamout) return 0;
     if ((v == "levsto" || v == "levdph") && !h->o.llevee) return 0;
     if (avg) {
-        if (!h->out.rivout) return fail(CMF_ESTATE, "%s is an output-period value: no output period yet", var);
+        if (!h->out.pthflw) return fail(CMF_ESTATE, "%s is an output-period value: no output period yet", var);
         cmf_output o{};
         vec.resize(v == "pthflw" ? (size_t)h->d.npthout * h->d.npthlev : n);
         double* p = vec.data();

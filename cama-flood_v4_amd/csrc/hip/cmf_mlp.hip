@@ -1103,6 +1103,7 @@ int cmf_mlp_set_data(cmf_mlp_handle h, const float* x, const float* t, int64_t n
     for (void* q : h->allocs) if (q) keep.push_back(q);
     h->allocs = keep;
     h->tx = h->tt = nullptr;
+    h->tn = 0;                                            // no data until both are there
     MTRY(malloc_t(h, &h->tx, (size_t)n * h->n_in));
     MTRY(malloc_t(h, &h->tt, (size_t)n * h->n_out));
     MCHK(hipMemcpyAsync(h->tx, x, (size_t)n * h->n_in * sizeof(float), hipMemcpyHostToDevice, h->stream));
@@ -1116,7 +1117,7 @@ int cmf_mlp_train(cmf_mlp_handle h, const int64_t* order, int64_t n_order, int32
                   float beta2, float eps, int32_t step0, float* loss_out) {
     if (!h || !order || n_order <= 0 || batch <= 0 || batch > h->max_batch)
         return mfail(CMF_MLP_EINVAL, "bad argument");
-    if (!h->tx) return mfail(CMF_MLP_ESTATE, "cmf_mlp_set_data must come first");
+    if (h->tn == 0) return mfail(CMF_MLP_ESTATE, "cmf_mlp_set_data must come first");
     for (int64_t k = 0; k < n_order; ++k)
         if (order[k] < 0 || order[k] >= h->tn) return mfail(CMF_MLP_EINVAL, "order[%lld] outside the data", (long long)k);
     double lsum = 0.0;
