@@ -72,7 +72,7 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
     const uint8_t* special = net.special;
     const bool paths = net.npth > 0;
     out = BlockPlan();
-    if (n <= 0 || T > 1024 || kmax < 1 || 3 * kmax > (paths ? 60 : 200)) return false;
+    if (n <= 0 || T > (paths ? 512 : 1024) || kmax < 1 || 3 * kmax > (paths ? 60 : 200)) return false;
     if (paths && (net.npthlev < 1 || net.npthlev > 64)) return false;
     const int per_wave = paths ? 64 / net.npthlev : 0;             // paths of a wavefront
     const int max_paths = paths ? std::min(blk_paths(T), per_wave * (T / 64)) : 0;
@@ -568,7 +568,8 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
 // Values of the cells of a block between the phases and substeps. With FP64 state
 // the arrays of T cells take 120 bytes a cell and the first NL floodplain heights 20
 // more, which fills the 160 KB of a CU with 1024 cells; the mixed form has room for
-// all heights.
+// all heights. With paths and levees or dams there is room for one, if two blocks of 512
+// cells are to share a CU.
 template <class R, int T, bool LEV, bool DAM, bool PTH>
 struct BlockLds {
     static constexpr bool kOutSum = sizeof(R) == sizeof(float);
@@ -1118,8 +1119,7 @@ hipError_t launch_block(const DevMap& M, const DevState<R>& S, const BlockState<
     if (P.npth > 0) {
         switch (P.T) {
             case 256: return launch_block_t<R, 256, false, true>(a, st);
-            case 512: return launch_block_t<R, 512, false, true>(a, st);
-            default: return launch_block_t<R, 1024, false, true>(a, st);
+            default: return launch_block_t<R, 512, false, true>(a, st);
         }
     }
     if (M.nmem > 1 || M.cell_dom) return launch_block_mb<R, true>(a, st);

@@ -53,7 +53,7 @@ constexpr int BLK_KINE_AT = 64;
 constexpr int blk_dams(int T) { return T / 32; }
 constexpr int blk_kines(int T) { return 3 * T / 32; }
 constexpr int blk_special(int T) { return 3 * T / 8; }
-constexpr int blk_paths(int T) { return T < 1024 ? T / 4 : 255; }
+constexpr int blk_paths(int T) { return T / 4; }            // blocks along paths have 512 cells at most
 
 // The levels of a path are computed by neighbouring lanes, whole paths in a wavefront,
 // from the last one of the block down (the ring's, which has least to do otherwise).
