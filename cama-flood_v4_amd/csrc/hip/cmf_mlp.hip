@@ -273,7 +273,7 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 template <int NJ, int NK>
 __device__ __forceinline__ void tile_product(const uint16_t* __restrict__ A, int lda, const uint16_t* Bs, int ldb,
                                              f32x4 (&acc)[4][NJ]) {
-    constexpr int D = NK == 1 ? 1 : (NJ <= 2 ? 8 : (NJ == 4 ? 2 : 1));
+    constexpr int D = NK == 1 ? 1 : (NJ <= 2 ? 8 : 2);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -747,9 +747,10 @@ FusedNet fused_net(const cmf_mlp* h) {
 }
 
 // Rows per workgroup: small batches need many workgroups more than large tiles
-// (1024 rows fill 64 of them with 16 rows); from 32768 rows on, 128-row tiles keep
-// the matrix cores busy and read the weights once per 128 rows (a gradient stops at
-// 64: its masks and accumulators would spill).
+// (1024 rows fill 64 of them with 16 rows); from 8192 rows on, 64-row tiles keep the
+// matrix cores busy and read the weights once per 64 rows. Larger ones have no use: a
+// chunk of the inference is 16,384 rows, and the masks and accumulators of a gradient
+// would spill.
 template <bool TRAIN>
 void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, float* y, hipStream_t st) {
     const FusedNet N = fused_net(h);
@@ -759,11 +760,8 @@ void launch_fused(cmf_mlp* h, const FusedTrain& G, const float* x, int rows, flo
         hipLaunchKernelGGL((k_mlp_fused<16, TRAIN>), blocks(16), dim3(256), 0, st, N, G, x, rows, y);
     else if (rows <= 8192)
         hipLaunchKernelGGL((k_mlp_fused<32, TRAIN>), blocks(32), dim3(256), 0, st, N, G, x, rows, y);
-    else if (rows <= 32768)
-        hipLaunchKernelGGL((k_mlp_fused<64, TRAIN>), blocks(64), dim3(256), 0, st, N, G, x, rows, y);
     else
-        hipLaunchKernelGGL((k_mlp_fused<TRAIN ? 64 : 128, TRAIN>), blocks(TRAIN ? 64 : 128), dim3(256), 0, st, N, G,
-                           x, rows, y);
+        hipLaunchKernelGGL((k_mlp_fused<64, TRAIN>), blocks(64), dim3(256), 0, st, N, G, x, rows, y);
 }
 
 // slots of the chunked inference: rows of x and y in pinned memory, x on the device
