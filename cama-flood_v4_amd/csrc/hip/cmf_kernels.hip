@@ -655,11 +655,12 @@ __device__ __forceinline__ void update_tile(const DevMap& M, const DevState<R>& 
 }
 
 // The mixed-precision ensemble outflow of the default scheme is held to 64 VGPRs
-// (8 waves per SIMD) and spills nothing; the single-model forms and the
-// kinematic / slope-mixed ensemble form would spill under that bound and keep the
-// compiler's choice.
+// (8 waves per SIMD) and spills nothing; its kinematic / slope-mixed form would spill
+// under that bound and is held to 72 (7 waves; left alone it takes 76: 64 members of
+// 99,473 cells, kinematic, 116 us instead of 106, slope-mixed 136 instead of 127). The
+// single-model forms keep the compiler's choice.
 template <class R, int BS, bool MB, bool KINE>
-__global__ __launch_bounds__(BS, (MB && sizeof(R) == 4 && !KINE) ? 8 : 1) void k_outflow(DevMap M, DevState<R> S, StepArgs A, int ntc, int nt_all) {
+__global__ __launch_bounds__(BS, (MB && sizeof(R) == 4) ? (KINE ? 7 : 8) : 1) void k_outflow(DevMap M, DevState<R> S, StepArgs A, int ntc, int nt_all) {
     const int t = tile_of(blockIdx.x, gridDim.x, nt_all, A.xcd);
     if (t < nt_all) outflow_tile<R, BS, MB, KINE>(M, S, A, t, ntc);
 }
@@ -670,10 +671,10 @@ __global__ __launch_bounds__(BS) void k_rate(DevMap M, DevState<R> S, StepArgs A
     if (t < ntc) rate_tile<R, BS, MB>(M, S, A, t);
 }
 
-// at most 96 VGPRs (5 waves per SIMD): the FP64 single-model update needs 97
-// without the bound and spills nothing to memory with it. The mixed-precision
-// ensemble update fits 80 (6 waves; 82 without the bound), again without spills;
-// the FP64 ensemble update would spill at 6.
+// at most 96 VGPRs (5 waves per SIMD): the FP64 single-model update spills two
+// registers (12 bytes a lane) with the bound, the others none. The mixed-precision
+// ensemble update fits 80 (6 waves), again without spills; the FP64 ensemble update
+// would spill at 6.
 template <class R, int BS, bool MB>
 __global__ __launch_bounds__(BS, (MB && sizeof(R) == 4) ? 6 : 5) void k_update(DevMap M, DevState<R> S, StepArgs A, int ntc, int nt_all) {
     __shared__ double lds[2 * NGLB * (BS / 64)];
