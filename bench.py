@@ -86,7 +86,8 @@ def run_gpu(net, m, rvec, precision, steps, warmup, dt, tune="auto"):
         best, trials = gm.autotune(dt, nsub=12)       # restores the state it times on
         for r in trials:
             if r[0] >= 2:
-                log(f"  trial graph={int(r[0]) - 2}: outer step of 12 substeps {r[7]:.3f} ms wall")
+                form = ("default form", "graph replay", "persistent kernel")[int(r[0]) - 2]
+                log(f"  trial {form}: capped outer step {r[7]:.3f} ms wall")
                 continue
             log(f"  trial fused={int(r[0])} bs={int(r[1])} xcd={int(r[2])} grid={int(r[3])}: "
                 f"outflow {r[4]:.3f} rate {r[5]:.3f} update {r[6]:.3f} total {r[7]:.3f} ms / 12 substeps")
@@ -105,14 +106,18 @@ def run_gpu(net, m, rvec, precision, steps, warmup, dt, tune="auto"):
         gm.synchronize()
         t_total += time.perf_counter() - t0
         sum_nt += nt
+    info = gm.block_info()
+    ran = ("block launches: {launches} of k_block in the last step, {blocks} blocks of {cells} cells, "
+           "up to {substeps} substeps each".format(**info)) if info["launches"] else (
+               "persistent kernel" if tune_used["fused"] else "phase kernels")
     # kernel timing pass (HIP events on the model's stream): times the three phase
-    # kernels one by one; the steps above ran block launches, several substeps each
+    # kernels one by one; the steps above ran what `ran` says
     gm.kernel_times(True)
     gm.set_runoff(rvec[rec % len(rvec)])
     gm.physics_advance(dt)
     kt = gm.kernel_times(False)
     gm.close()
-    return sum_nt, t_total, kt, tune_used
+    return sum_nt, t_total, kt, tune_used, ran
 
 
 def _reference_case(d, net, ro, dt, steps, llevee=True, ldamout=True, inpmat=None):
@@ -854,7 +859,7 @@ def roofline(kt, n_cells, bytes_tab):
     achieved = bytes_tab[dom] * n_cells / (ms * 1e-3) / 1e9
     return dom, per, dict(bound="hbm", achieved=round(achieved, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                           frac=round(achieved / HBM_PEAK_GBS, 4), traffic=None,
-                          kernel=f"k_{dom}", avg_ms=round(ms, 4),
+                          kernel=f"k_{dom}", avg_ms=round(ms, 4), timed_by="events, in a step of its own",
                           bytes_per_cell_substep=bytes_tab[dom])
 
 
@@ -943,7 +948,7 @@ def main():
     n = m.n
     log("FP64 run")
     tune_arg = "auto" if a.tune == "auto" else json.loads(a.tune)
-    sum_nt, t, kt, tune64 = run_gpu(net, m, rvec, "fp64", a.steps, a.warmup, dt, tune=tune_arg)
+    sum_nt, t, kt, tune64, ran = run_gpu(net, m, rvec, "fp64", a.steps, a.warmup, dt, tune=tune_arg)
     value = n * sum_nt / t
     dom, per, roof = roofline(kt, n, BYTES_FP64)
     log(f"FP64: {value:.4g} cell-substeps/s, sum NT {sum_nt}, {t:.3f}s; kernels ms {per}")
@@ -952,7 +957,7 @@ def main():
         from cmf import maps
         os.environ["CMF_HIP_ORDER"] = "nseq"
         m3 = maps.build_map(net, maps.Options(llevee=True, ldamout=True))
-        s3, t3, kt3, _ = run_gpu(net, m3, rvec, "fp64", a.steps, a.warmup, dt, tune=tune64)
+        s3, t3, kt3, *_ = run_gpu(net, m3, rvec, "fp64", a.steps, a.warmup, dt, tune=tune64)
         del os.environ["CMF_HIP_ORDER"]
         order_cmp = dict(value=n * s3 / t3, kernels_ms=roofline(kt3, n, BYTES_FP64)[1])
         log(f"FP64 NSEQ order: {order_cmp['value']:.4g} cell-substeps/s; kernels ms {order_cmp['kernels_ms']}")
@@ -961,10 +966,10 @@ def main():
         net2, m2, _ = net, None, None
         from cmf import maps
         m2 = maps.build_map(net, maps.Options(llevee=True, ldamout=True))
-        sum_nt2, t2, kt2, tune32 = run_gpu(net, m2, rvec, "mixed", a.steps, a.warmup, dt, tune=tune_arg)
+        sum_nt2, t2, kt2, tune32, ran2 = run_gpu(net, m2, rvec, "mixed", a.steps, a.warmup, dt, tune=tune_arg)
         dom2, per2, roof2 = roofline(kt2, n, BYTES_MIXED)
         mixed = dict(value=n * sum_nt2 / t2, unit="cell-substeps/s", sum_nt=sum_nt2,
-                     ms_per_step=1e3 * t2 / a.steps, roofline=roof2, tune=tune32)
+                     ms_per_step=1e3 * t2 / a.steps, timed_steps=ran2, roofline=roof2, tune=tune32)
         log(f"mixed: {mixed['value']:.4g} cell-substeps/s; kernels ms {per2}")
     ens = None
     if not a.no_ensemble:
@@ -1010,7 +1015,7 @@ def main():
     roof["traffic"] = measured_traffic(roof["kernel"]) if a.nx == 3600 and a.ny == 1800 else None
     sub_ms = sum(per.values())
     roof_sub = dict(bound="hbm", kernels="k_outflow + k_rate + k_update", avg_ms=round(sub_ms, 4),
-                    bytes_per_cell_substep=508.0,
+                    timed_by="events, in a step of its own", bytes_per_cell_substep=508.0,
                     achieved=round(508.0 * n / (sub_ms * 1e-3) / 1e9, 1), peak=HBM_PEAK_GBS, unit="GB/s")
     roof_sub["frac"] = round(roof_sub["achieved"] / HBM_PEAK_GBS, 4)
     out = {
@@ -1021,6 +1026,7 @@ def main():
         "config": {"workload": f"glb_06min-shaped synthetic network {a.nx}x{a.ny}, {n} cells, "
                                f"3% levees, 2500 dams, hourly runoff, DT=3600 s adaptive",
                    "cells": n, "sum_nt": sum_nt, "precision": "fp64", "tune": tune64},
+        "timed_steps": ran,
         "roofline": roof,
         "roofline_substep": roof_sub,
         "cpu_baseline": cpu,
