@@ -20,7 +20,10 @@
 #include "cmf_block.hpp"
 
 #include <algorithm>
+#include <atomic>
+#include <new>
 #include <queue>
+#include <thread>
 
 namespace cmf {
 
@@ -44,6 +47,40 @@ static bool groups_fit(const BlockNet& net, const std::vector<int32_t>& total, i
     for (int p = 0; p < net.n; ++p)
         if (to[(size_t)p] == p && size[(size_t)p] > T) return false;
     return true;
+}
+
+// What the surroundings ask of a cell, in one place: downstream cell, upstream list, and
+// the other ends of its paths (those out of it, then those into it)
+struct Node {
+    int32_t next, up, end;
+    uint16_t nend;
+    uint8_t nup;
+    bool damup;
+};
+struct PathEnd { int32_t cell, path; };
+
+// f(0) .. f(nw - 1), on threads of their own where there are any
+constexpr int PLAN_THREADS = 4;
+template <class F>
+static void in_threads(int nw, F f) {
+    std::atomic<bool> nomem{false};
+    std::atomic<int> next{0};
+    auto run = [&] {
+        try {
+            for (int w = next++; w < nw; w = next++) f(w);
+        } catch (const std::bad_alloc&) {
+            nomem = true;
+        }
+    };
+    std::vector<std::thread> th;
+    try {
+        for (int w = 1; w < nw; ++w) th.emplace_back(run);
+    } catch (const std::exception&) {
+        // no more threads: those there are do it all
+    }
+    run();
+    for (std::thread& t : th) t.join();
+    if (nomem) throw std::bad_alloc();
 }
 
 // ---------------------------------------------------------------------------
@@ -79,8 +116,21 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
     const int cap = paths ? std::max(8, T / 8) : std::max(T / 4, T - 48 * kmax);
     std::vector<int32_t> total((size_t)n, 1), resid((size_t)n), piece((size_t)n);
     std::vector<uint8_t> root((size_t)n, 0);
+    std::vector<Node> node((size_t)n);
+    std::vector<PathEnd> ends;
+    if (paths) ends.reserve((size_t)net.out_ptr[n] + (size_t)net.in_ptr[n]);
     for (int p = 0; p < n; ++p) {
+        Node& x = node[(size_t)p];
+        x = Node{next[p], up_ptr[p], (int32_t)ends.size(), 0, 0, special && (special[p] & BLK_DAMUP)};
+        if (paths) {
+            const int no = net.out_ptr[p + 1] - net.out_ptr[p], ni = net.in_ptr[p + 1] - net.in_ptr[p];
+            if (no > 255 || ni > 255) return false;
+            for (int k = net.out_ptr[p]; k < net.out_ptr[p + 1]; ++k) ends.push_back({net.pth_down[net.out_idx[k]], net.out_idx[k]});
+            for (int k = net.in_ptr[p]; k < net.in_ptr[p + 1]; ++k) ends.push_back({net.pth_up[net.in_idx[k]], net.in_idx[k]});
+            x.nend = (uint16_t)(no + ni);
+        }
         if (up_ptr[p + 1] - up_ptr[p] > 250) return false;
+        x.nup = (uint8_t)(up_ptr[p + 1] - up_ptr[p]);
         if (next[p] >= 0) {
             if (next[p] <= p) return false;                        // needs the depth-first order
             total[(size_t)next[p]] += total[(size_t)p];
@@ -144,8 +194,8 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
     int stamp = 0;
     // f(the other end, path) of every path of cell x
     auto each_path = [&](int x, auto f) {
-        for (int k = net.out_ptr[x]; k < net.out_ptr[x + 1]; ++k) f(net.pth_down[net.out_idx[k]], net.out_idx[k]);
-        for (int k = net.in_ptr[x]; k < net.in_ptr[x + 1]; ++k) f(net.pth_up[net.in_idx[k]], net.in_idx[k]);
+        const Node& c = node[(size_t)x];
+        for (int k = c.end; k < c.end + c.nend; ++k) f(ends[(size_t)k].cell, ends[(size_t)k].path);
     };
     // more cells than max_blocks hold
     auto too_many = [&] { return (int64_t)loc.size() > max_blocks * (int64_t)T; };
@@ -154,34 +204,37 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
         const int id = stamp++;
         curc.assign(cur.size(), 0);
         for (int x : cur) mark[(size_t)x] = id;
-        uint8_t c = 0;
         auto add = [&](int x) {
-            if (x >= 0 && mark[(size_t)x] != id) { mark[(size_t)x] = id; cur.push_back(x); curc.push_back(c); }
+            if (x >= 0 && mark[(size_t)x] != id) { mark[(size_t)x] = id; cur.push_back(x); }
         };
-        auto add_up = [&](int x) { for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) add(up_idx[k]); };
-        auto add_ends = [&](int x) { each_path(x, [&](int y, int) { add(y); }); };
-        size_t r0 = 0, q0 = 0;                                      // members whose neighbours are already in
+        auto add_up = [&](const Node& x) { for (int k = x.up; k < x.up + x.nup; ++k) add(up_idx[k]); };
+        auto add_ends = [&](const Node& x) { for (int k = x.end; k < x.end + x.nend; ++k) add(ends[(size_t)k].cell); };
+        size_t eu = 0;                                              // members whose neighbours are all in
         for (int r = 0; r < kmax && (int)cur.size() <= T; ++r) {
-            const size_t eu = cur.size();
-            c = (uint8_t)(3 * r + 1);
-            for (size_t j = r0; j < eu; ++j) { add_up(cur[j]); add(next[cur[j]]); if (paths) add_ends(cur[j]); }
-            const size_t er = cur.size();
-            c = (uint8_t)(3 * r + 2);
-            for (size_t j = r0; j < er; ++j) add_up(cur[j]);
-            const size_t eq = cur.size();
-            c = (uint8_t)(3 * r + 3);
-            for (size_t j = q0; j < eq; ++j) {
-                add(next[cur[j]]);
-                if (special && (special[(size_t)cur[j]] & BLK_DAMUP)) add_up(cur[j]);
+            const size_t r0 = eu;
+            eu = cur.size();
+            for (size_t j = r0; j < eu; ++j) {
+                const Node& x = node[(size_t)cur[j]];
+                add_up(x); add(x.next); add_ends(x);
             }
-            for (size_t j = r0; paths && j < er; ++j) add_ends(cur[j]);
-            r0 = er;
-            q0 = eq;
+            const size_t er = cur.size();
+            curc.resize(er, (uint8_t)(3 * r + 1));
+            for (size_t j = eu; j < er; ++j) add_up(node[(size_t)cur[j]]);
+            const size_t eq = cur.size();
+            curc.resize(eq, (uint8_t)(3 * r + 2));
+            for (size_t j = eu; j < eq; ++j) {
+                const Node& x = node[(size_t)cur[j]];
+                add(x.next);
+                if (x.damup) add_up(x);
+            }
+            for (size_t j = eu; paths && j < er; ++j) add_ends(node[(size_t)cur[j]]);
+            curc.resize(cur.size(), (uint8_t)(3 * r + 3));
+            eu = er;
         }
     };
     // paths whose flows a cell of this code asks for, from its set R_r on (kmax: none)
     auto path_step = [&](int code) { return std::min(kmax, code < 2 ? 0 : (code + 1) / 3); };
-    std::vector<int32_t> pmark(paths ? (size_t)net.npth : 0, -1), pslot(pmark.size());
+    std::vector<int32_t> pmark(paths ? (size_t)net.npth : 0, -1);
     auto count_paths = [&] {
         const int id = stamp++;
         int m = 0;
@@ -211,8 +264,9 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
             for (int e = off[(size_t)i]; e < off[(size_t)i + 1]; ++e) {
                 const int x = own[(size_t)e];
                 auto to = [&](int y) { if (y >= 0 && piece[(size_t)y] != i && !in[(size_t)piece[(size_t)y]]) f(piece[(size_t)y]); };
-                to(next[x]);
-                for (int k = up_ptr[x]; k < up_ptr[x + 1]; ++k) to(up_idx[k]);
+                const Node& c = node[(size_t)x];
+                to(c.next);
+                for (int k = c.up; k < c.up + c.nup; ++k) to(up_idx[k]);
                 each_path(x, [&](int y, int) { to(y); });
             }
         };
@@ -437,127 +491,149 @@ bool build_block_plan(const BlockNet& net, int T, int kmax, bool closed_only, in
         out.ppx_ptr.assign(np, 0);
         out.pends.assign((size_t)nb * npb, 0);
     }
-    std::vector<std::pair<int, int>> plist;                        // code, path
-    // order inside a block: dam, kinematic and levee cells in places of their own
-    // (their wavefronts take the rare paths, the others never do), then the owned
-    // cells, then the ring by code
-    std::vector<int32_t>& pos = resid;                               // local index in the block
-    std::vector<int32_t> place((size_t)T), count((size_t)3 * kmax + 6), spot((size_t)T);
-    std::fill(mark.begin(), mark.end(), -1);
-    std::fill(pmark.begin(), pmark.end(), -1);
-    for (int b = 0; b < nb; ++b) {
-        const std::vector<int32_t>& bin = bins[(size_t)b];
+    // Tables of blocks `from` to `to` - 1; the lists of the cells with more than two upstream
+    // cells or paths go to upx and ppx. Order inside a block: dam, kinematic and levee cells
+    // in places of their own (their wavefronts take the rare paths, the others never do),
+    // then the owned cells, then the ring by code.
+    auto tables = [&](int from, int to, std::vector<uint16_t>& upx, std::vector<uint16_t>& ppx) {
+        std::vector<int32_t> pos((size_t)n), in((size_t)n, -1);        // place in the block, piece it is of
+        std::vector<int32_t> slot(pmark.size()), slot_of(pmark.size(), -1);
+        std::vector<int32_t> place((size_t)T), count((size_t)3 * kmax + 6), spot((size_t)T);
+        std::vector<std::pair<int, int>> plist;                        // code, path
         auto code_of = [&](size_t e) { return closed ? 0 : (int)codes[e]; };
         auto key_of = [&](size_t e) {
             const uint8_t f = special ? special[(size_t)loc[e]] : 0;
             return f & BLK_KINE ? 1 : (f & BLK_DAM ? 0 : (f & BLK_LEV ? 2 : 3 + code_of(e)));
         };
-        std::fill(count.begin(), count.end(), 0);
-        for (int32_t k : bin)
-            for (int j = 0; j < done[(size_t)k].size; ++j) count[(size_t)key_of((size_t)done[(size_t)k].beg + j) + 1] += 1;
-        const int na = count[1], nk = count[2];
-        out.ndam[(size_t)b] = na | (nk << 16);
-        for (size_t i = 0; i + 1 < count.size(); ++i) count[i + 1] += count[i];
-        // spot[rank in that order] = place
-        for (int i = 0; i < na; ++i) spot[(size_t)i] = i;
-        for (int i = 0; i < nk; ++i) spot[(size_t)(na + i)] = BLK_KINE_AT + i;
-        for (int i = na + nk, l = na; i < T; ++i, ++l) {
-            if (nk > 0 && l == BLK_KINE_AT) l += nk;
-            spot[(size_t)i] = l;
-        }
-        int q = 0;
-        for (int32_t k : bin)
-            for (int j = 0; j < done[(size_t)k].size; ++j, ++q)
-                place[(size_t)q] = spot[(size_t)count[(size_t)key_of((size_t)done[(size_t)k].beg + j)]++];
-        q = 0;
-        int slots = 0;
-        for (int32_t k : bin) {
-            const Piece& pc = done[(size_t)k];
-            // a piece's neighbours are looked up inside the piece: two pieces of one
-            // block may both hold a cell
-            for (int j = 0; j < pc.size; ++j) {
-                const int x = loc[(size_t)pc.beg + j];
-                mark[(size_t)x] = k;
-                pos[(size_t)x] = place[(size_t)(q + j)];
+        for (int b = from; b < to; ++b) {
+            const std::vector<int32_t>& bin = bins[(size_t)b];
+            std::fill(count.begin(), count.end(), 0);
+            for (int32_t k : bin)
+                for (int j = 0; j < done[(size_t)k].size; ++j) count[(size_t)key_of((size_t)done[(size_t)k].beg + j) + 1] += 1;
+            const int na = count[1], nk = count[2];
+            out.ndam[(size_t)b] = na | (nk << 16);
+            for (size_t i = 0; i + 1 < count.size(); ++i) count[i + 1] += count[i];
+            // spot[rank in that order] = place
+            for (int i = 0; i < na; ++i) spot[(size_t)i] = i;
+            for (int i = 0; i < nk; ++i) spot[(size_t)(na + i)] = BLK_KINE_AT + i;
+            for (int i = na + nk, l = na; i < T; ++i, ++l) {
+                if (nk > 0 && l == BLK_KINE_AT) l += nk;
+                spot[(size_t)i] = l;
             }
-            if (paths) {
-                // slots of the paths, the owner's (of the upstream end) first; two
-                // pieces of one block may both have a path
-                plist.clear();
+            int q = 0;
+            for (int32_t k : bin)
+                for (int j = 0; j < done[(size_t)k].size; ++j, ++q)
+                    place[(size_t)q] = spot[(size_t)count[(size_t)key_of((size_t)done[(size_t)k].beg + j)]++];
+            q = 0;
+            int slots = 0;
+            for (int32_t k : bin) {
+                const Piece& pc = done[(size_t)k];
+                // a piece's neighbours are looked up inside the piece: two pieces of one
+                // block may both hold a cell
                 for (int j = 0; j < pc.size; ++j) {
-                    const int x = loc[(size_t)pc.beg + j], step = path_step(code_of((size_t)pc.beg + j));
-                    const bool mine = codes[(size_t)pc.beg + j] == 0;
-                    if (step < kmax)
-                        each_path(x, [&](int, int w) {
-                            const int code = mine && net.pth_up[w] == x ? 0 : 3 * step + 2;
-                            if (pmark[(size_t)w] != k) {
-                                pmark[(size_t)w] = k;
-                                pslot[(size_t)w] = (int)plist.size();
-                                plist.push_back({code, w});
-                            } else {
-                                int& c = plist[(size_t)pslot[(size_t)w]].first;
-                                c = std::min(c, code);
-                            }
+                    const int x = loc[(size_t)pc.beg + j];
+                    in[(size_t)x] = k;
+                    pos[(size_t)x] = place[(size_t)(q + j)];
+                }
+                if (paths) {
+                    // slots of the paths, the owner's (of the upstream end) first; two
+                    // pieces of one block may both have a path
+                    plist.clear();
+                    for (int j = 0; j < pc.size; ++j) {
+                        const int x = loc[(size_t)pc.beg + j], step = path_step(code_of((size_t)pc.beg + j));
+                        const bool mine = codes[(size_t)pc.beg + j] == 0;
+                        if (step < kmax)
+                            each_path(x, [&](int, int w) {
+                                const int code = mine && net.pth_up[w] == x ? 0 : 3 * step + 2;
+                                if (slot_of[(size_t)w] != k) {
+                                    slot_of[(size_t)w] = k;
+                                    slot[(size_t)w] = (int)plist.size();
+                                    plist.push_back({code, w});
+                                } else {
+                                    int& c = plist[(size_t)slot[(size_t)w]].first;
+                                    c = std::min(c, code);
+                                }
+                            });
+                    }
+                    std::stable_sort(plist.begin(), plist.end(),
+                                     [](const std::pair<int, int>& x, const std::pair<int, int>& y) { return x.first < y.first; });
+                    for (const auto& cw : plist) {
+                        const int w = cw.second, sl = slots++;
+                        slot[(size_t)w] = sl;
+                        out.pends[(size_t)b * npb + sl] = (uint32_t)pos[(size_t)net.pth_up[w]] | ((uint32_t)pos[(size_t)net.pth_down[w]] << 10);
+                        for (int v = 0; v < net.npthlev; ++v) {
+                            const size_t e = (size_t)b * T + (size_t)(T - 64 * (1 + sl / per_wave) + sl % per_wave * net.npthlev + v);
+                            out.path[e] = w;
+                            out.pword[e] = (uint32_t)v | ((uint32_t)sl << PATH_SLOT) | ((uint32_t)(closed ? 0 : cw.first) << PATH_CODE);
+                        }
+                    }
+                }
+                for (int j = 0; j < pc.size; ++j, ++q) {
+                    const int x = loc[(size_t)pc.beg + j];
+                    const int code = code_of((size_t)pc.beg + j);
+                    const size_t e0 = (size_t)b * T + place[(size_t)q];
+                    uint32_t nx = TOPO_MOUTH;
+                    if (next[x] >= 0) {
+                        const bool inside = in[(size_t)next[x]] == k;
+                        if (!inside && code <= 3 * (kmax - 1) + 2) return false;   // cannot be
+                        nx = inside ? (uint32_t)pos[(size_t)next[x]] : (uint32_t)place[(size_t)q];
+                    }
+                    int nup = up_ptr[x + 1] - up_ptr[x];
+                    for (int e = up_ptr[x]; e < up_ptr[x + 1]; ++e)
+                        if (in[(size_t)up_idx[e]] != k) {
+                            if (code <= 3 * (kmax - 1) + 1) return false;          // cannot be
+                            nup = 0;                                      // never asked for
+                            break;
+                        }
+                    const uint32_t u0 = nup > 0 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x]]] : 0u;
+                    const uint32_t u1 = nup > 1 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x] + 1]] : u0;
+                    const uint32_t fl = special ? special[(size_t)x] & (BLK_DAM | BLK_LEV) : 0u;
+                    out.cell[e0] = x;
+                    out.topo[e0] = nx | (u0 << TOPO_UP0) | (fl << TOPO_FLAGS);
+                    out.topo[np + e0] = u1 | ((uint32_t)nup << TOPO_NUP) | ((uint32_t)code << TOPO_CODE);
+                    if (paths && path_step(code) < kmax) {
+                        const int no = net.out_ptr[x + 1] - net.out_ptr[x], ni = net.in_ptr[x + 1] - net.in_ptr[x];
+                        uint32_t w = ((uint32_t)no << 16) | ((uint32_t)ni << 24);
+                        int at = 0;
+                        if (no + ni > 2) out.ppx_ptr[e0] = (int32_t)ppx.size();
+                        each_path(x, [&](int, int p) {
+                            if (at < 2) w |= (uint32_t)slot[(size_t)p] << (8 * at);
+                            else ppx.push_back((uint16_t)slot[(size_t)p]);
+                            ++at;
                         });
-                }
-                std::stable_sort(plist.begin(), plist.end(),
-                                 [](const std::pair<int, int>& x, const std::pair<int, int>& y) { return x.first < y.first; });
-                for (const auto& cw : plist) {
-                    const int w = cw.second, sl = slots++;
-                    pslot[(size_t)w] = sl;
-                    out.pends[(size_t)b * npb + sl] = (uint32_t)pos[(size_t)net.pth_up[w]] | ((uint32_t)pos[(size_t)net.pth_down[w]] << 10);
-                    for (int v = 0; v < net.npthlev; ++v) {
-                        const size_t e = (size_t)b * T + (size_t)(T - 64 * (1 + sl / per_wave) + sl % per_wave * net.npthlev + v);
-                        out.path[e] = w;
-                        out.pword[e] = (uint32_t)v | ((uint32_t)sl << PATH_SLOT) | ((uint32_t)(closed ? 0 : cw.first) << PATH_CODE);
+                        out.pcell[e0] = w;
+                    }
+                    if (nup > 2) {
+                        out.upx_ptr[e0] = (int32_t)upx.size();
+                        for (int e = up_ptr[x] + 2; e < up_ptr[x + 1]; ++e)
+                            upx.push_back((uint16_t)pos[(size_t)up_idx[e]]);
                     }
                 }
             }
-            for (int j = 0; j < pc.size; ++j, ++q) {
-                const int x = loc[(size_t)pc.beg + j];
-                const int code = code_of((size_t)pc.beg + j);
-                const size_t e0 = (size_t)b * T + place[(size_t)q];
-                uint32_t nx = TOPO_MOUTH;
-                if (next[x] >= 0) {
-                    const bool in = mark[(size_t)next[x]] == k;
-                    if (!in && code <= 3 * (kmax - 1) + 2) return false;   // cannot be
-                    nx = in ? (uint32_t)pos[(size_t)next[x]] : (uint32_t)place[(size_t)q];
-                }
-                int nup = up_ptr[x + 1] - up_ptr[x];
-                for (int e = up_ptr[x]; e < up_ptr[x + 1]; ++e)
-                    if (mark[(size_t)up_idx[e]] != k) {
-                        if (code <= 3 * (kmax - 1) + 1) return false;      // cannot be
-                        nup = 0;                                      // never asked for
-                        break;
-                    }
-                const uint32_t u0 = nup > 0 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x]]] : 0u;
-                const uint32_t u1 = nup > 1 ? (uint32_t)pos[(size_t)up_idx[up_ptr[x] + 1]] : u0;
-                const uint32_t fl = special ? special[(size_t)x] & (BLK_DAM | BLK_LEV) : 0u;
-                out.cell[e0] = x;
-                out.topo[e0] = nx | (u0 << TOPO_UP0) | (fl << TOPO_FLAGS);
-                out.topo[np + e0] = u1 | ((uint32_t)nup << TOPO_NUP) | ((uint32_t)code << TOPO_CODE);
-                if (paths && path_step(code) < kmax) {
-                    const int no = net.out_ptr[x + 1] - net.out_ptr[x], ni = net.in_ptr[x + 1] - net.in_ptr[x];
-                    if (no > 255 || ni > 255) return false;
-                    uint32_t w = ((uint32_t)no << 16) | ((uint32_t)ni << 24);
-                    int at = 0;
-                    out.ppx_ptr[e0] = (int32_t)out.ppx.size();
-                    each_path(x, [&](int, int p) {
-                        if (at < 2) w |= (uint32_t)pslot[(size_t)p] << (8 * at);
-                        else out.ppx.push_back((uint16_t)pslot[(size_t)p]);
-                        ++at;
-                    });
-                    out.pcell[e0] = w;
-                }
-                if (nup > 2) {
-                    out.upx_ptr[e0] = (int32_t)out.upx.size();
-                    for (int e = up_ptr[x] + 2; e < up_ptr[x + 1]; ++e)
-                        out.upx.push_back((uint16_t)pos[(size_t)up_idx[e]]);
-                }
-            }
+            for (int l = 0; l < T; ++l)
+                if (out.cell[(size_t)b * T + l] < 0) out.topo[np + (size_t)b * T + l] = 255u << TOPO_CODE;   // idle
         }
-        for (int l = 0; l < T; ++l)
-            if (out.cell[(size_t)b * T + l] < 0) out.topo[np + (size_t)b * T + l] = 255u << TOPO_CODE;   // idle
+        return true;
+    };
+    // in a few ranges of blocks, then their lists one after another
+    const int nr = nb < 64 ? 1 : PLAN_THREADS;
+    std::vector<std::vector<uint16_t>> upx((size_t)nr), ppx((size_t)nr);
+    std::atomic<bool> ok{true};
+    auto range = [&](int r) { return (int)((int64_t)nb * r / nr); };
+    in_threads(nr, [&](int r) {
+        if (!tables(range(r), range(r + 1), upx[(size_t)r], ppx[(size_t)r])) ok = false;
+    });
+    if (!ok) return false;
+    out.upx.swap(upx[0]);
+    out.ppx.swap(ppx[0]);
+    for (int r = 1; r < nr; ++r) {
+        const int32_t du = (int32_t)out.upx.size(), dp = (int32_t)out.ppx.size();
+        for (size_t e = (size_t)range(r) * (size_t)T; e < (size_t)range(r + 1) * (size_t)T; ++e) {
+            if (((out.topo[np + e] >> TOPO_NUP) & 0xff) > 2) out.upx_ptr[e] += du;
+            if (paths && ((out.pcell[e] >> 16) & 0xff) + (out.pcell[e] >> 24) > 2) out.ppx_ptr[e] += dp;
+        }
+        out.upx.insert(out.upx.end(), upx[(size_t)r].begin(), upx[(size_t)r].end());
+        out.ppx.insert(out.ppx.end(), ppx[(size_t)r].begin(), ppx[(size_t)r].end());
     }
     if (out.upx.empty()) out.upx.push_back(0);
     if (out.ppx.empty()) out.ppx.push_back(0);
