@@ -16,6 +16,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -1340,38 +1341,75 @@ struct BlockPaths {
     int live = 0;
 };
 
-// partition of the network for block launches, its device copy and the second set
-// of the arrays the launches hand on
-template <class R>
-int make_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
-                 const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
-                 const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of, const BlockPaths& pth, const cmf_map* mp) {
-    const int n = h->d.nseqall;
+// The partition of a network for block launches, computed by a thread of its own while the
+// map goes to the device: creating a model of 239,086 cells with paths takes 49 ms, 57 with
+// one after the other; of 1,500,120 cells 157 and 207; of 59,535 8.2 and 9.3. Below 8,192
+// cells it is sooner done than a thread is there.
+struct PlanJob {
+    const cmf_hip_ctx* h = nullptr;
+    BlockNet net{};
     std::vector<uint8_t> special;
-    if (h->o.ldamout || h->o.llevee) special.assign((size_t)n, 0);
-    for (int p = 0; p < n && h->o.ldamout; ++p)
-        special[(size_t)p] |= (uint8_t)((i1d[(size_t)p] > 0 ? BLK_DAM | BLK_DAMUP : 0) | (dam_of[(size_t)p] != -1 ? BLK_DAM : 0) |
-                                        (i1d[(size_t)p] == 10 ? BLK_KINE : 0));
-    for (int p = 0; p < n && h->o.llevee; ++p)
-        if (lev_of[(size_t)p] >= 0) special[(size_t)p] |= BLK_LEV;
-    BlockNet net{n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(), dom_of.data()};
+    BlockPlan plan;
+    bool ok = false, nomem = false;
+    std::thread th;
+    void work() {
+        const bool paths = net.npth > 0;
+        try {
+            for (const BlockShape& b : paths ? path_shapes(net.n)
+                                             : block_shapes(h->M.ns, h->ninst, h->o.precision != CMF_PREC_FP64)) {
+                ok = build_block_plan(net, b.T, b.kmax, b.closed_only, b.max_blocks / h->nmem, plan);
+                // blocks hold cells of one domain: many small domains would leave them empty
+                ok = ok && ((int64_t)plan.nblk * h->nmem <= 256 || (int64_t)plan.nblk * plan.T <= 2 * (int64_t)net.n);
+                if (ok) break;
+            }
+        } catch (const std::bad_alloc&) {
+            nomem = true;
+        }
+    }
+    // the vectors are read until finish() is back
+    void start(const cmf_hip_ctx* ctx, const std::vector<int32_t>& next, const std::vector<int32_t>& up_ptr,
+               const std::vector<int32_t>& up_idx, const std::vector<int32_t>& i1d, const std::vector<int32_t>& dam_of,
+               const std::vector<int32_t>& lev_of, const std::vector<int32_t>& dom_of, const BlockPaths& pth) {
+        const int n = ctx->d.nseqall;
+        try {
+            if (ctx->o.ldamout || ctx->o.llevee) special.assign((size_t)n, 0);
+        } catch (const std::bad_alloc&) {
+            return;                                       // no memory: no partition
+        }
+        h = ctx;
+        for (int p = 0; p < n && h->o.ldamout; ++p)
+            special[(size_t)p] |= (uint8_t)((i1d[(size_t)p] > 0 ? BLK_DAM | BLK_DAMUP : 0) | (dam_of[(size_t)p] != -1 ? BLK_DAM : 0) |
+                                            (i1d[(size_t)p] == 10 ? BLK_KINE : 0));
+        for (int p = 0; p < n && h->o.llevee; ++p)
+            if (lev_of[(size_t)p] >= 0) special[(size_t)p] |= BLK_LEV;
+        net = BlockNet{n, next.data(), up_ptr.data(), up_idx.data(), special.empty() ? nullptr : special.data(), dom_of.data()};
+        if (pth.live > 0) {
+            net.npth = h->d.npthout; net.npthlev = h->d.npthlev;
+            net.pth_up = pth.up.data(); net.pth_down = pth.down.data();
+            net.out_ptr = pth.out_ptr.data(); net.out_idx = pth.out_idx.data();
+            net.in_ptr = pth.in_ptr.data(); net.in_idx = pth.in_idx.data();
+        }
+        if (n < 8192) return;
+        try {
+            th = std::thread([this] { work(); });
+        } catch (const std::exception&) {
+            // no more threads: finish() does it
+        }
+    }
+    bool finish() {
+        if (th.joinable()) th.join();
+        else if (h) work();
+        return ok && !nomem;
+    }
+    ~PlanJob() {
+        if (th.joinable()) th.join();
+    }
+};
+
+// device copy of the partition and the second set of the arrays its launches hand on
+template <class R>
+int put_blocks(cmf_hip_ctx* h, const BlockPlan& bp, const BlockPaths& pth, const cmf_map* mp) {
     const bool paths = pth.live > 0;
-    if (paths) {
-        net.npth = h->d.npthout; net.npthlev = h->d.npthlev;
-        net.pth_up = pth.up.data(); net.pth_down = pth.down.data();
-        net.out_ptr = pth.out_ptr.data(); net.out_idx = pth.out_idx.data();
-        net.in_ptr = pth.in_ptr.data(); net.in_idx = pth.in_idx.data();
-    }
-    BlockPlan bp;
-    bool ok = false;
-    for (const BlockShape& b : paths ? path_shapes(n)
-                                     : block_shapes(h->M.ns, h->ninst, sizeof(R) == sizeof(float))) {
-        ok = build_block_plan(net, b.T, b.kmax, b.closed_only, b.max_blocks / h->nmem, bp);
-        // blocks hold cells of one domain: many small domains would leave them empty
-        ok = ok && ((int64_t)bp.nblk * h->nmem <= 256 || (int64_t)bp.nblk * bp.T <= 2 * (int64_t)n);
-        if (ok) break;
-    }
-    if (!ok) return 0;                                    // the three-phase kernels serve every network
     BlockTab P{};
     P.T = bp.T; P.kmax = bp.kmax; P.closed = bp.closed;
     int32_t* p32 = nullptr;
@@ -1431,14 +1469,15 @@ int make_blocks(cmf_hip_ctx* h, const std::vector<int32_t>& next, const std::vec
     return 0;
 }
 
-// The three-phase kernels need none of it: a model for which there is no memory left,
-// on the device or the host, keeps them.
-template <class R, class... Net>
-int setup_blocks(cmf_hip_ctx* h, const Net&... net) {
+// The three-phase kernels serve every network and need none of it: a model without a
+// partition, or for which there is no memory left, on the device or the host, keeps them.
+template <class R>
+int setup_blocks(cmf_hip_ctx* h, PlanJob& job, const BlockPaths& pth, const cmf_map* mp) {
+    if (!job.finish()) return 0;
     const size_t had = h->allocs.size();
     int rc;
     try {
-        rc = make_blocks<R>(h, net...);
+        rc = put_blocks<R>(h, job.plan, pth, mp);
     } catch (const std::bad_alloc&) {
         rc = CMF_ENOMEM;
     }
@@ -1668,22 +1707,7 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
         }
     }
     TRY(validate_tables(h, mp));
-    TRY(put_f32(h, &M.grarea, mp->grarea, n, "GRAREA"));
-    TRY(put_f32(h, &M.elevtn, mp->elevtn, n, "ELEVTN"));
-    TRY(put_f32(h, &M.nxtdst, mp->nxtdst, n, "NXTDST"));
-    TRY(put_f32(h, &M.rivlen, mp->rivlen, n, "RIVLEN"));
-    TRY(put_f32(h, &M.rivwth, mp->rivwth, n, "RIVWTH"));
-    TRY(put_f32(h, &M.rivhgt, mp->rivhgt, n, "RIVHGT"));
-    TRY(put_f32(h, &M.rivman, mp->rivman, n, "RIVMAN"));
-    TRY(put_f32(h, &M.fldhgt, mp->fldhgt, (size_t)n, "FLDHGT", (size_t)nl));
     double* pd = nullptr;
-    {
-        std::vector<double> v = to_dev(h, mp->dwnelv, (size_t)n);
-        TRY(put_raw(h, &pd, v.data(), (size_t)n)); M.dwnelv = pd;
-        h->dwnelv_dev = pd;
-        std::vector<int32_t> m2 = to_dev(h, mp->i2mask, (size_t)n);
-        TRY(put_raw(h, &p32, m2.data(), (size_t)n)); M.i2mask = p32;
-    }
     // bifurcation paths (maps:531-639)
     BlockPaths bpth;
     M.pth_dom = nullptr;
@@ -1792,13 +1816,29 @@ int cmf_hip_set_map(cmf_handle h, const cmf_map* mp_in) {
             if (ddom[(size_t)p] < ddom[(size_t)p - 1]) return fail(CMF_EMAP, "domains are not contiguous in device order");
         TRY(put_raw(h, &h->d_dom_off, doff.data(), doff.size()));
     }
-    // the slots of a whole state (16 MB at most), touched while the partition is made: the
-    // first cmf_hip_get_state of 59,535 cells 2.7 -> 0.5 ms (pageable copies 1.5)
+    PlanJob job;
+    if (h->permuted && h->nmem <= BLOCK_MEMBERS && (!h->o.lpthout || h->ninst == 1))
+        job.start(h, dnext, dptr, didx, i1d, doc, lidx, ddom, bpth);
+    // the slots of a whole state (16 MB at most), touched meanwhile: the first
+    // cmf_hip_get_state of 59,535 cells 2.7 -> 0.5 ms (pageable copies 1.5)
     if (h->xfer.grow(xfer_bytes((size_t)30 * M.ns)) != hipSuccess) (void)hipGetLastError();
     Prefault touch(h->xfer.p, h->xfer.cap);
-    if (h->permuted && h->nmem <= BLOCK_MEMBERS && (!h->o.lpthout || h->ninst == 1))
-        TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, dnext, dptr, didx, i1d, doc, lidx, ddom, bpth, mp)
-                                            : setup_blocks<float>(h, dnext, dptr, didx, i1d, doc, lidx, ddom, bpth, mp));
+    TRY(put_f32(h, &M.grarea, mp->grarea, n, "GRAREA"));
+    TRY(put_f32(h, &M.elevtn, mp->elevtn, n, "ELEVTN"));
+    TRY(put_f32(h, &M.nxtdst, mp->nxtdst, n, "NXTDST"));
+    TRY(put_f32(h, &M.rivlen, mp->rivlen, n, "RIVLEN"));
+    TRY(put_f32(h, &M.rivwth, mp->rivwth, n, "RIVWTH"));
+    TRY(put_f32(h, &M.rivhgt, mp->rivhgt, n, "RIVHGT"));
+    TRY(put_f32(h, &M.rivman, mp->rivman, n, "RIVMAN"));
+    TRY(put_f32(h, &M.fldhgt, mp->fldhgt, (size_t)n, "FLDHGT", (size_t)nl));
+    {
+        std::vector<double> v = to_dev(h, mp->dwnelv, (size_t)n);
+        TRY(put_raw(h, &pd, v.data(), (size_t)n)); M.dwnelv = pd;
+        h->dwnelv_dev = pd;
+        std::vector<int32_t> m2 = to_dev(h, mp->i2mask, (size_t)n);
+        TRY(put_raw(h, &p32, m2.data(), (size_t)n)); M.i2mask = p32;
+    }
+    if (job.h) TRY(h->o.precision == CMF_PREC_FP64 ? setup_blocks<double>(h, job, bpth, mp) : setup_blocks<float>(h, job, bpth, mp));
     h->map_set = true;
     return 0;
 }
