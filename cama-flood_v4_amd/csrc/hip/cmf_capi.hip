@@ -1357,9 +1357,13 @@ struct PlanJob {
         try {
             for (const BlockShape& b : paths ? path_shapes(net.n)
                                              : block_shapes(h->M.ns, h->ninst, h->o.precision != CMF_PREC_FP64)) {
-                ok = build_block_plan(net, b.T, b.kmax, b.closed_only, b.max_blocks / h->nmem, plan);
                 // blocks hold cells of one domain: many small domains would leave them empty
-                ok = ok && ((int64_t)plan.nblk * h->nmem <= 256 || (int64_t)plan.nblk * plan.T <= 2 * (int64_t)net.n);
+                auto filled = [&](int64_t nblk) { return nblk * h->nmem <= 256 || nblk * b.T <= 2 * (int64_t)net.n; };
+                int64_t least = 0;
+                for (int d = 0; d < h->ndom; ++d)
+                    least += (h->dom_off[(size_t)d + 1] - h->dom_off[(size_t)d] + b.T - 1) / b.T;
+                ok = filled(least) && build_block_plan(net, b.T, b.kmax, b.closed_only, b.max_blocks / h->nmem, plan) &&
+                     filled(plan.nblk);
                 if (ok) break;
             }
         } catch (const std::bad_alloc&) {
