@@ -675,6 +675,7 @@ struct BlockHgt {
     __device__ __forceinline__ float operator()(int l) const {
         return l <= NL ? s[(l - 1) * T] : h[(size_t)(l - 1) * n];
     }
+    __device__ __forceinline__ const BlockHgt& row() const { return *this; }
 };
 
 template <class R>

@@ -671,10 +671,10 @@ __global__ __launch_bounds__(BS) void k_rate(DevMap M, DevState<R> S, StepArgs A
     if (t < ntc) rate_tile<R, BS, MB>(M, S, A, t);
 }
 
-// at most 96 VGPRs (5 waves per SIMD): the FP64 single-model update spills two
-// registers (12 bytes a lane) with the bound, the others none. The mixed-precision
-// ensemble update fits 80 (6 waves), again without spills; the FP64 ensemble update
-// would spill at 6.
+// at most 96 VGPRs (5 waves per SIMD): the FP64 single-model update needs 97
+// without the bound and spills nothing to memory with it. The mixed-precision
+// ensemble update fits 80 (6 waves; 82 without the bound), again without spills;
+// the FP64 ensemble update would spill at 6.
 template <class R, int BS, bool MB>
 __global__ __launch_bounds__(BS, (MB && sizeof(R) == 4) ? 6 : 5) void k_update(DevMap M, DevState<R> S, StepArgs A, int ntc, int nt_all) {
     __shared__ double lds[2 * NGLB * (BS / 64)];
