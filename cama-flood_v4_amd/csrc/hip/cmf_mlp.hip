@@ -320,8 +320,8 @@ __device__ __forceinline__ void sync_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Measured (24-256-256-256-2): inference of 262144 rows 224 us, 321 TFLOP/s, bound by the
-// products and their LDS operands (layer kernels: 1.8 ms); a gradient's pass over 1024
+// Measured (24-256-256-256-2): a chunk of the inference, 16,384 rows, 27 us, 169 TFLOP/s,
+// one tile of 64 rows per CU (layer kernels: 112 us); a gradient's pass over 1024
 // rows 29 us and over 4099 rows 38 us, bound by the chain of seven layers on one
 // wavefront per SIMD (layer kernels, forward and backward with k_mlp_dw's part: 860 us
 // and 2.4 ms).
