@@ -1030,7 +1030,7 @@ int advance_t(cmf_hip_ctx* h, double dt_def, int32_t nt_cap, int32_t* nt_out, do
         h->t_ms[4] += ntmax;
         h->inst_ms.assign((size_t)ni, 0.0);
         for (int k = 0; k < ni; ++k) {
-            const size_t e1 = 1 + (size_t)per * h->h_inst[k].nt;
+            const size_t e1 = 1 + (size_t)per * std::max(h->h_inst[k].nt, 0);   // no bound, no substep
             HIPCHK(hipEventElapsedTime(&ms, h->ev[0], h->ev[e1]));
             h->inst_ms[(size_t)k] = ms;
         }
